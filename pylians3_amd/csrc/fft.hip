@@ -15,10 +15,24 @@
 // host in double and rounded to float.  Other sizes use a rocFFT 3D plan.
 #include "pyl_internal.h"
 
+#include <algorithm>
+
 namespace pyl {
 namespace {
 
 constexpr int kFftBlock = 256;
+
+// Input of the row pass: cube (field f, realisation r) at in[f] + r*N^3; with apply,
+// x/scale - shift of scales[f*sfield + r*sreal] (or the one scale).  The pass also
+// clears nzero words at zero (the maxima a later pass of the same stream fills).
+constexpr int kRowFields = 8;
+struct RowSrc {
+    const float *in[kRowFields];
+    const float *scales, *shifts;
+    unsigned *zero;
+    float scale, shift;
+    int nreal, apply, sfield, sreal, nzero;
+};
 
 __device__ __forceinline__ float2 cmul(float2 a, float2 b) {
     return make_float2(a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x);
@@ -266,9 +280,16 @@ absmax_kernel(const float2 *__restrict__ dk, long long nrows, int zlen, long lon
 // X[k] = E[k] + e^{-2 pi i k/N} O[k] with E[k] = (Z[k] + conj(Z[N/2-k]))/2 and
 // O[k] = -i (Z[k] - conj(Z[N/2-k]))/2, k = 0..N/2 (indices mod N/2).  Output
 // rows of N/2+1 complex.
+//
+// The rows are read where the caller keeps them (RowSrc: one array per field) and the
+// prologue x/scale - shift is applied to them as they are read, so no copy of the
+// field is made before the transform: the pass is HBM-bound, and the copy (512^3:
+// 0.21 ms beside this kernel's 0.25) and, for a batch with scales, the prologue's own
+// pass over it (32 x 2 x 128^3: 0.34 + 0.25 ms) were pure extra traffic.  Pk of a 512^3
+// field on the GPU: 1.41 -> 1.18 ms, the batch of 32: 5.66 -> 5.20 ms.
 template <int N, int R>
 __global__ void __launch_bounds__(kFftBlock)
-fft_r2c_rows_kernel(const float *__restrict__ in, float2 *__restrict__ out, long long nrows,
+fft_r2c_rows_kernel(RowSrc rs, float2 *__restrict__ out, long long nrows,
                     const float2 *__restrict__ tw_half, const float2 *__restrict__ tw_full,
                     long long zs) {
     constexpr int H = N / 2;
@@ -278,14 +299,28 @@ fft_r2c_rows_kernel(const float *__restrict__ in, float2 *__restrict__ out, long
     __shared__ float2 buf[H * RP];
     const long long row0 = (long long)blockIdx.x * R;
     const int rw = (int)min((long long)R, nrows - row0);
+    static_assert((N * N) % R == 0, "the rows of a workgroup lie in one cube");
+    const int cube = (int)(row0 / (N * N));               // field * nreal + realisation
+    const int field = cube / rs.nreal, real = cube - field * rs.nreal;
+    for (int i = blockIdx.x * kFftBlock + threadIdx.x; i < rs.nzero; i += gridDim.x * kFftBlock) rs.zero[i] = 0u;
     // R consecutive rows are N*R contiguous floats: read them as float2 pairs
-    const float2 *src = (const float2 *)(in + row0 * N);
+    const float2 *src = (const float2 *)(rs.in[field] + ((long long)real * (N * N) + row0 % (N * N)) * N);
     float2 v[PER];
 #pragma unroll
     for (int p = 0; p < PER; ++p) {
         const int t = threadIdx.x + p * kFftBlock;        // pair index within the block
         const int r = min(t / H, rw - 1);
         v[p] = src[(long long)r * H + t % H];
+    }
+    if (rs.apply) {                                       // uniform: (x / scale) - shift in float32
+        const int si = field * rs.sfield + real * rs.sreal;
+        const float scale = rs.scales ? rs.scales[si] : rs.scale;
+        const float shift = rs.shifts ? rs.shifts[si] : rs.shift;
+#pragma unroll
+        for (int p = 0; p < PER; ++p) {
+            v[p].x = v[p].x / scale - shift;
+            v[p].y = v[p].y / scale - shift;
+        }
     }
 #pragma unroll
     for (int p = 0; p < PER; ++p) {
@@ -339,7 +374,7 @@ int cols(Ctx *c, int n, float2 *data, long long nstride, long long ostride, long
 }
 
 template <int N>
-int launch_rows(Ctx *c, const float *in, float2 *out, long long nrows, const float2 *twh,
+int launch_rows(Ctx *c, const RowSrc &in, float2 *out, long long nrows, const float2 *twh,
                 const float2 *twf, long long zs) {
     constexpr int R = (N >= 512) ? 8 : 32;
     const long long nb = (nrows + R - 1) / R;
@@ -348,7 +383,7 @@ int launch_rows(Ctx *c, const float *in, float2 *out, long long nrows, const flo
     return PYL_OK;
 }
 
-int rows(Ctx *c, int n, const float *in, float2 *out, long long nrows, const float2 *twh,
+int rows(Ctx *c, int n, const RowSrc &in, float2 *out, long long nrows, const float2 *twh,
          const float2 *twf, long long zs) {
     switch (n) {
         case 16: return launch_rows<16>(c, in, out, nrows, twh, twf, zs);
@@ -415,10 +450,47 @@ int complex_absmax(Ctx *c, const float2 *dk, int dims, long long zs, int ncube, 
     return PYL_OK;
 }
 
-// out = r2c FFT of `batch` contiguous (N,N,N) float cubes, rows of N/2+1 modes zs
-// apart (zs = 0: dense, N/2+1), N*N*zs per cube.  `in` may be overwritten.  amax
-// (optional, 64 zeroed words per cube): the largest |Re| or |Im| of each cube's
+// out = own r2c FFT passes of the cubes of nfields fields (RowSrc: nreal contiguous
+// (N,N,N) float cubes per field, prologue applied as they are read), cube (f, r) at
+// index f*nreal + r; rows of N/2+1 modes zs apart, N*N*zs per cube.  amax (optional, 64
+// words per cube, zeroed here by the row pass): the largest |Re| or |Im| of each cube's
 // transform, float bits (see fft_col_kernel).
+int fft_r2c_fields(Ctx *c, const FieldSrc &fs, float2 *out, int dims, long long zs, unsigned *amax) {
+    PYL_CHECK(fft_own_size(dims), PYL_EINVAL, "no own FFT passes for side %d", dims);
+    if (zs <= 0) zs = dims / 2 + 1;
+    const long long N = dims, Z = dims / 2 + 1;
+    const long long batch = (long long)fs.nfields * fs.nreal;
+    const float2 *tw = nullptr, *twh = nullptr;
+    PYL_TRY(get_twiddles(c, dims, &tw));
+    PYL_TRY(get_twiddles(c, dims / 2, &twh));
+    // z: real rows -> half-complex rows (zs apart); kRowFields fields per launch
+    for (int f0 = 0; f0 < fs.nfields; f0 += kRowFields) {
+        RowSrc rs{};
+        const int nf = std::min(kRowFields, fs.nfields - f0);
+        for (int f = 0; f < nf; ++f) rs.in[f] = fs.in[f0 + f];
+        rs.nreal = fs.nreal;
+        rs.apply = fs.apply;
+        rs.scale = fs.scale;
+        rs.shift = fs.shift;
+        rs.scales = fs.scales ? fs.scales + (long long)f0 * fs.sfield : nullptr;
+        rs.shifts = fs.shifts ? fs.shifts + (long long)f0 * fs.sfield : nullptr;
+        rs.sfield = fs.sfield;
+        rs.sreal = fs.sreal;
+        rs.zero = amax;
+        rs.nzero = (amax && f0 == 0) ? (int)(64 * batch) : 0;
+        PYL_TRY(rows(c, dims, rs, out + (long long)f0 * fs.nreal * N * N * zs, N * N * fs.nreal * nf, twh, tw, zs));
+    }
+    // y: n = y (stride zs), other = x (stride N*zs); Z columns of each row
+    PYL_TRY(cols(c, dims, out, zs, N * zs, N * N * zs, (int)Z, dims, (int)batch, tw));
+    // x: n = x (stride N*zs), other = y (stride zs)
+    PYL_TRY(cols(c, dims, out, N * zs, zs, N * N * zs, (int)Z, dims, (int)batch, tw, amax));
+    return PYL_OK;
+}
+
+// out = r2c FFT of `batch` contiguous (N,N,N) float cubes, rows of N/2+1 modes zs
+// apart (zs = 0: dense, N/2+1), N*N*zs per cube: the own passes where there are any
+// (`in` is only read), a rocFFT plan otherwise (`in` may be overwritten).  amax
+// (optional, 64 zeroed words per cube): as fft_r2c_fields.
 int fft_r2c_3d(Ctx *c, float *in, float2 *out, int dims, int batch, long long zs, unsigned *amax) {
     if (zs <= 0) zs = dims / 2 + 1;
     if (!fft_own_size(dims)) {
@@ -432,17 +504,11 @@ int fft_r2c_3d(Ctx *c, float *in, float2 *out, int dims, int batch, long long zs
             PYL_TRY(complex_absmax(c, out, dims, zs, batch, (long long)dims * dims * zs, amax));
         return PYL_OK;
     }
-    const long long N = dims, Z = dims / 2 + 1;
-    const float2 *tw = nullptr, *twh = nullptr;
-    PYL_TRY(get_twiddles(c, dims, &tw));
-    PYL_TRY(get_twiddles(c, dims / 2, &twh));
-    // z: real rows -> half-complex rows (zs apart)
-    PYL_TRY(rows(c, dims, in, out, N * N * batch, twh, tw, zs));
-    // y: n = y (stride zs), other = x (stride N*zs); Z columns of each row
-    PYL_TRY(cols(c, dims, out, zs, N * zs, N * N * zs, (int)Z, dims, batch, tw));
-    // x: n = x (stride N*zs), other = y (stride zs)
-    PYL_TRY(cols(c, dims, out, N * zs, zs, N * N * zs, (int)Z, dims, batch, tw, amax));
-    return PYL_OK;
+    const float *ptr = in;
+    FieldSrc fs;
+    fs.in = &ptr;
+    fs.nreal = batch;
+    return fft_r2c_fields(c, fs, out, dims, zs, amax);
 }
 
 }  // namespace pyl

@@ -995,14 +995,17 @@ __global__ void zero_u32_kernel(unsigned *__restrict__ p, int n) {
     if (i < n) p[i] = 0u;
 }
 
-// 64 zeroed words per cube for the transforms' largest |Re|, |Im| (a fill kernel,
-// not a memset node, so that a captured call clears them on every replay).
-int pk_amax_words(Ctx *c, int ncube, unsigned **out) {
+// 64 words per cube for the transforms' largest |Re|, |Im|, zeroed (a fill kernel, not
+// a memset node, so that a captured call clears them on every replay) unless the own
+// row pass clears them (own: one launch less).
+int pk_amax_words(Ctx *c, int ncube, bool own, unsigned **out) {
     const int n = 64 * ncube;
     PYL_TRY(ensure(c, BUF_PK_AMAX, sizeof(unsigned) * (size_t)n));
     unsigned *a = (unsigned *)c->bufs[BUF_PK_AMAX].ptr;
-    zero_u32_kernel<<<ceil_div(n, 256), 256, 0, c->stream>>>(a, n);
-    PYL_HIP(hipGetLastError());
+    if (!own) {
+        zero_u32_kernel<<<ceil_div(n, 256), 256, 0, c->stream>>>(a, n);
+        PYL_HIP(hipGetLastError());
+    }
     *out = a;
     return PYL_OK;
 }
@@ -1011,6 +1014,35 @@ int fft_device(Ctx *c, float *in, float2 *out, int dims, int batch, long long zs
                unsigned *amax = nullptr) {
     PYL_TRY(stage_begin(c, PYL_STAGE_PK_FFT));
     PYL_TRY(fft_r2c_3d(c, in, out, dims, batch, zs, amax));
+    PYL_TRY(stage_end(c, PYL_STAGE_PK_FFT));
+    return PYL_OK;
+}
+
+// Own FFT passes of nfields fields of nreal cubes each (n floats per cube).  Device
+// arrays are read in place; host arrays, and device arrays that are not 8-byte aligned
+// (the row pass reads pairs), are brought into BUF_FFT_IN first.
+int fft_fields_device(Ctx *c, const float *const *deltas, FieldSrc fs, bool dev, float2 *out, int dims,
+                      long long zs, unsigned *amax) {
+    const size_t cube = (size_t)dims * dims * dims * fs.nreal;
+    std::vector<const float *> src(fs.nfields);
+    int ncopy = 0;
+    for (int f = 0; f < fs.nfields; ++f)
+        if (!dev || ((uintptr_t)deltas[f] & 7)) ++ncopy;
+    if (ncopy) PYL_TRY(ensure(c, BUF_FFT_IN, cube * ncopy * sizeof(float)));
+    float *dst = (float *)c->bufs[BUF_FFT_IN].ptr;
+    PYL_TRY(stage_begin(c, PYL_STAGE_PK_PREP));
+    for (int f = 0; f < fs.nfields; ++f) {
+        src[f] = deltas[f];
+        if (dev && ((uintptr_t)deltas[f] & 7) == 0) continue;
+        PYL_HIP(hipMemcpyAsync(dst, deltas[f], cube * sizeof(float),
+                               dev ? hipMemcpyDeviceToDevice : hipMemcpyHostToDevice, c->stream));
+        src[f] = dst;
+        dst += cube;
+    }
+    PYL_TRY(stage_end(c, PYL_STAGE_PK_PREP));
+    fs.in = src.data();
+    PYL_TRY(stage_begin(c, PYL_STAGE_PK_FFT));
+    PYL_TRY(fft_r2c_fields(c, fs, out, dims, zs, amax));
     PYL_TRY(stage_end(c, PYL_STAGE_PK_FFT));
     return PYL_OK;
 }
@@ -1171,6 +1203,14 @@ int pyl_fft_r2c(pyl_ctx *ctx, const float *delta, float *delta_k, int dims, int 
     reset_stages(c);
     const long long n = (long long)dims * dims * dims;
     const long long nk = (long long)dims * dims * (dims / 2 + 1);
+    // the own passes read a device input in place, unless it overlaps the output
+    const bool apart = (const char *)(delta + n) <= (const char *)delta_k ||
+                       (const char *)((const float2 *)delta_k + nk) <= (const char *)delta;
+    if ((flags & PYL_PTR_DEVICE) && fft_own_size(dims) && apart) {
+        FieldSrc fs;
+        PYL_TRY(fft_fields_device(c, &delta, fs, true, (float2 *)delta_k, dims, 0, nullptr));
+        return finish(c, flags);
+    }
     PYL_TRY(ensure(c, BUF_FFT_IN, (size_t)n * sizeof(float)));
     float *in = (float *)c->bufs[BUF_FFT_IN].ptr;
     float2 *outp;
@@ -1213,14 +1253,23 @@ int pyl_pk(pyl_ctx *ctx, const float *const *deltas, int nfields, const int *mas
     const bool destroy = dev && (flags & PYL_PK_DESTROY_INPUT);
     PYL_TRY(ensure(c, BUF_FFT_OUT, (size_t)nk * nfields * sizeof(float2)));
     float2 *dk = (float2 *)c->bufs[BUF_FFT_OUT].ptr;
+    const bool own = fft_own_size(dims);
     unsigned *amax = nullptr;
-    PYL_TRY(pk_amax_words(c, nfields, &amax));
+    PYL_TRY(pk_amax_words(c, nfields, own, &amax));
     std::vector<const unsigned *> amf(nfields);
     for (int f = 0; f < nfields; ++f) amf[f] = amax + 64 * f;
     std::vector<const float2 *> dks(nfields);
     const int pb = 256;
     const int nb = (int)std::min<long long>((n + pb - 1) / pb, 8192);
-    if (destroy) {
+    if (own) {
+        FieldSrc fs;
+        fs.nfields = nfields;
+        fs.apply = apply;
+        fs.scale = scale;
+        fs.shift = shift;
+        PYL_TRY(fft_fields_device(c, deltas, fs, dev, dk, dims, zs, amax));
+        for (int f = 0; f < nfields; ++f) dks[f] = dk + (size_t)f * nk;
+    } else if (destroy) {
         for (int f = 0; f < nfields; ++f) {
             float *x = (float *)deltas[f];
             if (apply) {
@@ -1290,11 +1339,12 @@ int pyl_pk_batch(pyl_ctx *ctx, const float *const *deltas, int nreal, int nfield
     PYL_TRY(ensure(c, BUF_FFT_OUT, (size_t)nk * ncube * sizeof(float2)));
     float2 *dk = (float2 *)c->bufs[BUF_FFT_OUT].ptr;
     unsigned *amax = nullptr;                          // cube (f, r) at (f*nreal + r)*64
-    PYL_TRY(pk_amax_words(c, ncube, &amax));
+    const bool own = fft_own_size(dims);
+    PYL_TRY(pk_amax_words(c, ncube, own, &amax));
     std::vector<const unsigned *> amf(nfields);
     for (int f = 0; f < nfields; ++f) amf[f] = amax + (size_t)64 * nreal * f;
     float *in = nullptr;
-    if (!destroy) {
+    if (!destroy && !own) {
         PYL_TRY(ensure(c, BUF_FFT_IN, (size_t)n * ncube * sizeof(float)));
         in = (float *)c->bufs[BUF_FFT_IN].ptr;
     }
@@ -1326,27 +1376,39 @@ int pyl_pk_batch(pyl_ctx *ctx, const float *const *deltas, int nreal, int nfield
         dsc = d;
         dsh = d + ncube;
     }
-    const int nbx = (int)std::max<long long>(1, std::min<long long>((n + 255) / 256, 2048));
-    PYL_TRY(stage_begin(c, PYL_STAGE_PK_PREP));
-    for (int f = 0; f < nfields; ++f) {
-        float *dst = destroy ? (float *)deltas[f] : in + (size_t)f * nreal * n;
-        if (!destroy)
-            PYL_HIP(hipMemcpyAsync(dst, deltas[f], (size_t)n * nreal * sizeof(float),
-                                   dev ? hipMemcpyDeviceToDevice : hipMemcpyHostToDevice, c->stream));
-        if (apply) {
-            const size_t off = sdev ? (size_t)f : (size_t)f * nreal;
-            prologue_kernel<<<dim3(nbx, nreal), 256, 0, c->stream>>>(
-                dst, dst, n, dsc + off, dsh + off, 1.0f, 0.0f, 1, sstride);
-            PYL_HIP(hipGetLastError());
-        }
-    }
-    PYL_TRY(stage_end(c, PYL_STAGE_PK_PREP));
-    if (destroy) {
-        for (int f = 0; f < nfields; ++f)
-            PYL_TRY(fft_device(c, (float *)deltas[f], dk + (size_t)f * nreal * nk, dims, nreal, zs,
-                               amax + (size_t)64 * nreal * f));
+    if (own) {
+        FieldSrc fs;
+        fs.nfields = nfields;
+        fs.nreal = nreal;
+        fs.apply = apply;
+        fs.scales = dsc;
+        fs.shifts = dsh;
+        fs.sfield = sdev ? 1 : nreal;
+        fs.sreal = sdev ? nfields : 1;
+        PYL_TRY(fft_fields_device(c, deltas, fs, dev, dk, dims, zs, amax));
     } else {
-        PYL_TRY(fft_device(c, in, dk, dims, ncube, zs, amax));
+        const int nbx = (int)std::max<long long>(1, std::min<long long>((n + 255) / 256, 2048));
+        PYL_TRY(stage_begin(c, PYL_STAGE_PK_PREP));
+        for (int f = 0; f < nfields; ++f) {
+            float *dst = destroy ? (float *)deltas[f] : in + (size_t)f * nreal * n;
+            if (!destroy)
+                PYL_HIP(hipMemcpyAsync(dst, deltas[f], (size_t)n * nreal * sizeof(float),
+                                       dev ? hipMemcpyDeviceToDevice : hipMemcpyHostToDevice, c->stream));
+            if (apply) {
+                const size_t off = sdev ? (size_t)f : (size_t)f * nreal;
+                prologue_kernel<<<dim3(nbx, nreal), 256, 0, c->stream>>>(
+                    dst, dst, n, dsc + off, dsh + off, 1.0f, 0.0f, 1, sstride);
+                PYL_HIP(hipGetLastError());
+            }
+        }
+        PYL_TRY(stage_end(c, PYL_STAGE_PK_PREP));
+        if (destroy) {
+            for (int f = 0; f < nfields; ++f)
+                PYL_TRY(fft_device(c, (float *)deltas[f], dk + (size_t)f * nreal * nk, dims, nreal, zs,
+                                   amax + (size_t)64 * nreal * f));
+        } else {
+            PYL_TRY(fft_device(c, in, dk, dims, ncube, zs, amax));
+        }
     }
     std::vector<const float2 *> dks(nfields);
     for (int f = 0; f < nfields; ++f) dks[f] = dk + (size_t)f * nreal * nk;
@@ -1378,7 +1440,7 @@ int pyl_pk_from_fourier(pyl_ctx *ctx, const float *const *delta_k, int nfields, 
         }
     }
     unsigned *amax = nullptr;
-    PYL_TRY(pk_amax_words(c, nfields, &amax));
+    PYL_TRY(pk_amax_words(c, nfields, false, &amax));
     std::vector<const unsigned *> amf(nfields);
     for (int f = 0; f < nfields; ++f) {
         PYL_TRY(complex_absmax(c, dks[f], dims, 0, 1, nk, amax + 64 * f));

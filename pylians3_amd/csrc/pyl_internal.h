@@ -233,6 +233,18 @@ int check_total(Ctx *c);                 // reports a tile sort that lost partic
 // Transform kinds of the resident rocFFT plans (all single precision, out of place).
 enum FFTKind { FFT_R2C_3D = 0, FFT_C2R_3D = 1, FFT_R2C_2D = 2, FFT_R2C_1D = 3 };
 int get_fft_plan(Ctx *c, int dims, int batch, FFTPlan **out, int kind = FFT_R2C_3D);
+// Fields to transform: nreal contiguous cubes each, read in place (8-byte aligned
+// arrays); apply: x/scale - shift in float32 as they are read, scales[f*sfield +
+// r*sreal] (device arrays) or one scale for all.
+struct FieldSrc {
+    const float *const *in = nullptr;
+    int nfields = 1, nreal = 1;
+    int apply = 0;
+    float scale = 1.0f, shift = 0.0f;
+    const float *scales = nullptr, *shifts = nullptr;
+    int sfield = 0, sreal = 0;
+};
+int fft_r2c_fields(Ctx *c, const FieldSrc &fs, float2 *out, int dims, long long zs, unsigned *amax);
 // Forward r2c of `batch` contiguous cubes (own passes for power-of-two sizes).
 // Rows of N/2+1 modes zs apart (zs = 0: dense); fft_zstride(dims): the padded
 // stride of the library's own half-complex buffers.
