@@ -309,7 +309,8 @@ int pyl_graph_launch(pyl_graph *graph);     /* replay, wait, run the host steps 
 int pyl_graph_destroy(pyl_graph *graph);
 
 /* Launch parameters for a tuner (value 0 / -1: the built-in choice). */
-#define PYL_TUNE_BIN_ROWS      1   /* binning rows per work item, 1..256 */
+#define PYL_TUNE_BIN_ROWS      1   /* binning rows per work item, 1..256 (taken in the groups of
+                                      up to four symmetric rows that are binned together) */
 #define PYL_TUNE_DEPOSIT_ORDER 2   /* MA deposit in largest-tile-first order: 1 on, 0 off */
 #define PYL_TUNE_SORT_WINDOW   3   /* tiled MA sort: 0 the one-pass sort with the grid's
                                       default window; 1 the wide window (every tile in LDS;

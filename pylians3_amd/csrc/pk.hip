@@ -9,15 +9,17 @@
 // |delta_k|^2 in double (:355-357), mu-Legendre weights for l = 0, 2, 4 and the
 // phase (:358), and the 1D / 2D / 3D accumulations (:361-378).
 //
-// Work decomposition.  Rows (kxx, kyy) of the half-complex cube are grouped by
-// a key that fixes the 2D bins a row can reach: |kx| (axis 0), |ky| (axis 1)
-// or k_per = isqrt(kx^2+ky^2) (axis 2).  A work item is up to R rows with one
-// key; one workgroup per item accumulates into LDS: the 3D bins, one "line" of
-// 2D bins (all k_per at fixed k_par for axes 0/1, all k_par at fixed k_per for
-// axis 2) and the 1D bins.  Each lane handles runs of 4 consecutive kz and
-// merges equal bins in registers before its LDS atomics.  Items write their
-// LDS partials with plain stores; a reduce kernel sums them in item order, so
-// the result is deterministic and no global atomics are used.
+// Work decomposition.  The up to four rows (+-kx, +-ky) of one (|kx|, |ky|) form a
+// row group: at every kz they share |k|, the bins, mu and the MAS factor, and differ
+// only in their values.  Groups are ordered by a key that fixes the 2D bins they can
+// reach: |kx| (axis 0), |ky| (axis 1) or k_per = isqrt(kx^2+ky^2) (axis 2).  A work
+// item is some groups with one key; one workgroup per item accumulates into LDS: the 3D
+// bins, one "line" of 2D bins (all k_per at fixed k_par for axes 0/1, all k_par at
+// fixed k_per for axis 2) and the 1D bins.  Each lane handles runs of 4 consecutive kz
+// of a group, adds up the group's |delta|^2 at each kz and merges equal bins along the
+// run in registers before its LDS atomics.  Items write their LDS partials with plain
+// stores; a reduce kernel sums them, so the result is deterministic and no global
+// atomics are used.
 //
 // Mode counts and k sums do not depend on the data: they are computed exactly
 // on the host once per (dims, axis) from Hermitian-pair counting and cached.
@@ -168,13 +170,11 @@ PkDims pk_dims(int dims) {
     return p;
 }
 
-int row_key(int kxx, int kyy, int dims, int axis) {
-    const int m = dims / 2;
-    int kx = kxx > m ? kxx - dims : kxx;
-    int ky = kyy > m ? kyy - dims : kyy;
-    if (axis == 0) return std::abs(kx);
-    if (axis == 1) return std::abs(ky);
-    long long v = (long long)kx * kx + (long long)ky * ky;
+// Key of the row group (a, b) = (|kx|, |ky|).
+int group_key(int a, int b, int axis) {
+    if (axis == 0) return a;
+    if (axis == 1) return b;
+    const long long v = (long long)a * a + (long long)b * b;
     long long s = (long long)std::sqrt((double)v);
     while (s * s > v) --s;
     while ((s + 1) * (s + 1) <= v) ++s;
@@ -182,19 +182,25 @@ int row_key(int kxx, int kyy, int dims, int axis) {
 }
 
 int get_bin_plan(Ctx *c, int dims, int axis, int nreal, BinPlan **out) {
-    // rows per item: ~2048 items for one large grid; for a batch, ~16K items in total
-    // so that the partials stay small
-    const long long nrows_total = (long long)dims * dims;
+    // Groups per item.  Large grids: ~2048 items (for a batch ~16K items in total, so
+    // that the partials stay small).  Small grids: at least one run per lane of the
+    // workgroup, since an item's fixed cost (clearing, writing and reducing its P bins)
+    // does not shrink with it: 64^3 took 513 items of four rows, 36 of 512 lanes at
+    // work, and their reduction (18 us) took longer than the binning (13 us).
+    const PkDims p = pk_dims(dims);
+    const long long ngroups_total = (long long)(p.m + 1) * (p.m + 1);
+    const int runs_per_group = p.zpad / kRun;
     const long long target = nreal > 1 ? std::max(1LL, 16384LL / nreal) : 2048LL;
-    int R = c->tune_bin_rows > 0 ? std::min(256, c->tune_bin_rows)
-                                 : (int)std::max(4LL, std::min(256LL, nrows_total / target));
+    int G = c->tune_bin_rows > 0
+                ? std::max(1, std::min(256, c->tune_bin_rows) / 4)
+                : (int)std::max<long long>(ceil_div(kBinBlock, runs_per_group),
+                                           std::min<long long>(64, ngroups_total / target));
     // an exact bin sum's low word takes at most kFixMaxAdds additions: one per run of
-    // kRun modes of the item's rows
-    const int runs_per_row = (pk_dims(dims).zpad) / kRun;
-    R = std::max(1, std::min(R, kFixMaxAdds / runs_per_row));
+    // kRun modes of the item's groups
+    G = std::max(1, std::min(G, kFixMaxAdds / runs_per_group));
     SharedTables &st = shared_tables();
     std::lock_guard<std::mutex> lk(st.mu);
-    const auto key = std::make_tuple(c->device, dims, axis, R);
+    const auto key = std::make_tuple(c->device, dims, axis, G);
     auto it = st.bin.find(key);
     if (it != st.bin.end()) {
         *out = &it->second;
@@ -202,44 +208,45 @@ int get_bin_plan(Ctx *c, int dims, int axis, int nreal, BinPlan **out) {
     }
     PYL_CHECK(!c->capturing, PYL_EINVAL, "binning plan created while a graph is captured: run the "
               "same work once on the context before capturing it");
-    PkDims p = pk_dims(dims);
+    PYL_CHECK(p.m < 32768, PYL_EINVAL, "grid too large for the binning plan");
     const int nkeys = (axis == 2) ? p.kmax_per + 1 : p.m + 1;
     std::vector<std::vector<int>> by_key(nkeys);
-    for (int kxx = 0; kxx < dims; ++kxx)
-        for (int kyy = 0; kyy < dims; ++kyy)
-            by_key[row_key(kxx, kyy, dims, axis)].push_back(kxx * dims + kyy);
-    std::vector<int> rows;
-    rows.reserve(nrows_total);
+    for (int a = 0; a <= p.m; ++a)
+        for (int b = 0; b <= p.m; ++b) by_key[group_key(a, b, axis)].push_back(a << 16 | b);
+    std::vector<int> groups;
+    groups.reserve(ngroups_total);
     std::vector<int4> items;
     std::vector<int> key_items(nkeys + 1, 0);
     for (int k = 0; k < nkeys; ++k) {
         key_items[k] = (int)items.size();
         const auto &v = by_key[k];
-        for (size_t s = 0; s < v.size(); s += R) {
-            int n = (int)std::min<size_t>(R, v.size() - s);
-            items.push_back(make_int4((int)rows.size() + (int)s, n, k, 0));
+        // equal shares of the key's groups
+        const int n = (int)v.size(), ni = ceil_div(n, G);
+        for (int i = 0; i < ni; ++i) {
+            const int s = (int)((long long)n * i / ni), e = (int)((long long)n * (i + 1) / ni);
+            items.push_back(make_int4((int)groups.size() + s, e - s, k, 0));
         }
-        rows.insert(rows.end(), v.begin(), v.end());
+        groups.insert(groups.end(), v.begin(), v.end());
     }
     key_items[nkeys] = (int)items.size();
     BinPlan bp;
     bp.dims = dims;
     bp.axis = axis;
-    bp.R = R;
+    bp.G = G;
     bp.nitems = (int)items.size();
     bp.nkeys = nkeys;
     auto fail = [&](hipError_t e) {
-        (void)hipFree(bp.d_rows);
+        (void)hipFree(bp.d_groups);
         (void)hipFree(bp.d_items);
         (void)hipFree(bp.d_key_items);
         set_error("binning plan upload failed: %s", hipGetErrorString(e));
         return e == hipErrorOutOfMemory ? PYL_ENOMEM : PYL_EHIP;
     };
     hipError_t e;
-    if ((e = hipMalloc(&bp.d_rows, rows.size() * sizeof(int))) != hipSuccess) return fail(e);
+    if ((e = hipMalloc(&bp.d_groups, groups.size() * sizeof(int))) != hipSuccess) return fail(e);
     if ((e = hipMalloc(&bp.d_items, items.size() * sizeof(int4))) != hipSuccess) return fail(e);
     if ((e = hipMalloc(&bp.d_key_items, key_items.size() * sizeof(int))) != hipSuccess) return fail(e);
-    if ((e = hipMemcpy(bp.d_rows, rows.data(), rows.size() * sizeof(int), hipMemcpyHostToDevice)) !=
+    if ((e = hipMemcpy(bp.d_groups, groups.data(), groups.size() * sizeof(int), hipMemcpyHostToDevice)) !=
         hipSuccess)
         return fail(e);
     if ((e = hipMemcpy(bp.d_items, items.data(), items.size() * sizeof(int4),
@@ -263,7 +270,7 @@ struct BinArgs {
     const unsigned *amax[2]; // per field [realisation][64]: largest |Re|, |Im| (float bits)
     int *escale;             // [realisation][2]: E of the power and the phase sums
     int nreal;
-    const int *rows;
+    const int *groups;       // |kx| << 16 | |ky| per row group
     const int4 *items;
     unsigned long long *plo; // [nreal][nitems][P] low words of the item sums
     int *phi;                // [nreal][nitems][P] high words
@@ -272,7 +279,8 @@ struct BinArgs {
     int nitems;
     int dims, m, zlen, zpad, even, kmax, L2, L1;
     int P, off2, off1;       // partial layout: acc3 at 0, line2 at off2, line1 at off1
-    int rmax;                // max rows per item (LDS row table size)
+    int gmax;                // max groups per item (LDS group table size)
+    int wide;                // rows are 16-byte aligned and padded to zpad: 16-byte loads
 };
 
 // floor(sqrt(v)) for 0 <= v < 2^24: the hardware square root (within 1 ulp)
@@ -305,6 +313,26 @@ __device__ __forceinline__ float atan_halfplane(float a, float b) {
     return t * p;
 }
 
+// The phase^2 of Pk_library.pyx:358, atan2(Re, |delta|)^2, from the float components
+// scaled by a power of two near 1/max(|Re|, |Im|) (exact): |delta|^2 formed in float
+// would overflow or underflow for |delta| beyond ~1e19 or below ~1e-19.
+__device__ __forceinline__ float phase_sq(float xr, float xi) {
+    float ph = 0.0f;
+    const float mx = fmaxf(fabsf(xr), fabsf(xi));
+    if (mx > 0.0f) {
+        const int e = __builtin_amdgcn_frexp_expf(mx);
+        const float xs = __builtin_ldexpf(xr, -e), ys = __builtin_ldexpf(xi, -e);
+        ph = atan_halfplane(xs, __builtin_amdgcn_sqrtf(xs * xs + ys * ys));
+    }
+    return ph * ph;
+}
+
+// VALU-bound: about 170 instructions per mode when every row was binned by itself
+// (0.305 ms at 512^3, axis 0, against 0.1 ms for its 0.54 GB).  The symmetric rows of a
+// group share everything but their values, so the geometry, the MAS factor, the
+// multipole products and the flush into LDS are done once for up to four modes:
+// 0.171 ms at 512^3 (3.2 TB/s of modes read), 0.092 -> 0.049 ms for two fields at 256^3
+// (axis 2), 0.573 -> 0.223 ms for 32 realisations of two 128^3 fields.
 template <int AXIS, int NFL, bool PHASE>
 __global__ void __launch_bounds__(kBinBlock) pk_bin_kernel(BinArgs a) {
     constexpr int S = Spec<NFL>::S;
@@ -318,12 +346,12 @@ __global__ void __launch_bounds__(kBinBlock) pk_bin_kernel(BinArgs a) {
     int *ahi = (int *)(alo + a.P);
     const int K1 = a.kmax + 1;
     double *corrz = (double *)(ahi + ((a.P + 1) & ~1));  // [zlen*NFL]
-    double *rowc = corrz + a.zlen * NFL;              // [rmax*NFL]
-    int *rowi = (int *)(rowc + a.rmax * NFL);         // [rmax*3]: kx, ky, linear row
+    double *rowc = corrz + a.zlen * NFL;              // [gmax*NFL]
+    int *grp = (int *)(rowc + a.gmax * NFL);          // [gmax]
     __shared__ int sE[2];
 
     const int4 item = a.items[blockIdx.x];
-    const int nrows = item.y;
+    const int ngrp = item.y;
     const int key = item.z;
     const int tid = threadIdx.x;
     const int n3 = (a.kmax + 1) * NA3;
@@ -331,37 +359,39 @@ __global__ void __launch_bounds__(kBinBlock) pk_bin_kernel(BinArgs a) {
         alo[i] = 0ull;
         ahi[i] = 0;
     }
-    if (tid == 0) {
+    if (tid < 64) {
         // the realisation's scale: the same in every work item
+        float mw[NFL];
+#pragma unroll
+        for (int f = 0; f < NFL; ++f) mw[f] = __uint_as_float(a.amax[f][(long long)blockIdx.y * 64 + tid]);
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1)
+#pragma unroll
+            for (int f = 0; f < NFL; ++f) mw[f] = fmaxf(mw[f], __shfl_xor(mw[f], o));
         const double nm = (double)a.dims * a.dims * a.zlen;
         double bound = 0.0;
+#pragma unroll
         for (int f = 0; f < NFL; ++f) {
-            const unsigned *w = a.amax[f] + (long long)blockIdx.y * 64;
-            float m = 0.0f;
-            for (int j = 0; j < 64; ++j) m = fmaxf(m, __uint_as_float(w[j]));
-            const double am = (double)m * (double)a.cmax[f];
+            const double am = (double)fmaxf(0.0f, mw[f]) * (double)a.cmax[f];
             bound = fmax(bound, 2.0 * nm * am * am);
         }
-        sE[0] = fix_exponent(bound * 1.01);
-        sE[1] = fix_exponent(nm);
-        if (blockIdx.x == 0) {
-            a.escale[2 * blockIdx.y] = sE[0];
-            a.escale[2 * blockIdx.y + 1] = sE[1];
+        if (tid == 0) {
+            sE[0] = fix_exponent(bound * 1.01);
+            sE[1] = fix_exponent(nm);
+            if (blockIdx.x == 0) {
+                a.escale[2 * blockIdx.y] = sE[0];
+                a.escale[2 * blockIdx.y + 1] = sE[1];
+            }
         }
     }
     for (int i = tid; i < a.zlen * NFL; i += blockDim.x) {
         int f = i / a.zlen, kz = i - f * a.zlen;
         corrz[i] = a.corr[f][kz];
     }
-    for (int r = tid; r < nrows; r += blockDim.x) {
-        int lin = a.rows[item.x + r];
-        int kxx = lin / a.dims, kyy = lin - kxx * a.dims;
-        int kx = kxx > a.m ? kxx - a.dims : kxx;
-        int ky = kyy > a.m ? kyy - a.dims : kyy;
-        rowi[3 * r + 0] = kx;
-        rowi[3 * r + 1] = ky;
-        rowi[3 * r + 2] = lin;
-        for (int f = 0; f < NFL; ++f) rowc[r * NFL + f] = a.corr[f][kxx] * a.corr[f][kyy];
+    for (int r = tid; r < ngrp; r += blockDim.x) {
+        const int g = a.groups[item.x + r];
+        grp[r] = g;
+        for (int f = 0; f < NFL; ++f) rowc[r * NFL + f] = a.corr[f][g >> 16] * a.corr[f][g & 0xffff];
     }
     __syncthreads();
     const int Ep = sE[0], Eph = sE[1];
@@ -369,7 +399,7 @@ __global__ void __launch_bounds__(kBinBlock) pk_bin_kernel(BinArgs a) {
     const int mm = a.m * a.m;
     // 1D accumulator (axes 0/1: k_par = key): each run's sum in fixed point, added
     // up per lane in integers, so the result does not depend on which lane took which
-    // run (nor on how the rows were cut into work items)
+    // run (nor on how the groups were cut into work items)
     unsigned long long p1lo[S];
     long long p1hi[S];
 #pragma unroll
@@ -379,33 +409,57 @@ __global__ void __launch_bounds__(kBinBlock) pk_bin_kernel(BinArgs a) {
     }
 
     // Lane runs start at flat index tid*kRun and advance by blockDim*kRun over the
-    // item's rows x zpad (zpad is a multiple of kRun, so a run never crosses a row).
+    // item's groups x zpad (zpad is a multiple of kRun, so a run never crosses a group).
     const int step = blockDim.x * kRun;
     const int dr = step / a.zpad, dc = step - dr * a.zpad;
     int r = (tid * kRun) / a.zpad;
     int kz0 = tid * kRun - r * a.zpad;
-    for (; r < nrows; r += dr, kz0 += dc) {
+    for (; r < ngrp; r += dr, kz0 += dc) {
         if (kz0 >= a.zpad) {
             kz0 -= a.zpad;
             ++r;
-            if (r >= nrows) break;
+            if (r >= ngrp) break;
         }
-        const int kx = rowi[3 * r + 0], ky = rowi[3 * r + 1];
-        const long long rowoff = (long long)blockIdx.y * a.fstride + (long long)rowi[3 * r + 2] * a.zs;
-        const int kxy2 = kx * kx + ky * ky;
-        const bool kx_neg = kx < 0;
-        const bool kx_edge = (kx == 0) || (a.even && kx == a.m);
-        const bool ky_neg = ky < 0;
+        const int ka = grp[r] >> 16, kb = grp[r] & 0xffff;    // |kx|, |ky|
+        const int kxy2 = ka * ka + kb * kb;
+        // rows of the group: (ka, kb), (ka, -kb), (-ka, kb), (-ka, -kb); -ka (-kb) is a
+        // row of its own unless it is 0 or the Nyquist index
+        const bool hasx = ka != 0 && !(a.even && ka == a.m);
+        const bool hasy = kb != 0 && !(a.even && kb == a.m);
+        const unsigned rows = 1u | (hasy ? 2u : 0u) | (hasx ? 4u : 0u) | (hasx && hasy ? 8u : 0u);
+        // of them, the independent ones in the kz = 0 and kz = m (even) planes
+        // (Pk_library.pyx:324-327: kx < 0, and ky < 0 at the kx edges, are skipped)
+        const unsigned prows = 1u | (hasy && hasx ? 2u : 0u);
+        const int xn = hasx ? a.dims - ka : ka, yn = hasy ? a.dims - kb : kb;
+        const long long fo = (long long)blockIdx.y * a.fstride + kz0;
+        const long long ro[4] = {fo + (long long)(ka * a.dims + kb) * a.zs, fo + (long long)(ka * a.dims + yn) * a.zs,
+                                 fo + (long long)(xn * a.dims + kb) * a.zs, fo + (long long)(xn * a.dims + yn) * a.zs};
         double c01[NFL];
 #pragma unroll
         for (int f = 0; f < NFL; ++f) c01[f] = rowc[r * NFL + f];
 
-        float2 v[NFL][kRun];
+        float2 v[NFL][4][kRun];
+        if (a.wide) {
 #pragma unroll
-        for (int f = 0; f < NFL; ++f)
+            for (int f = 0; f < NFL; ++f)
 #pragma unroll
-            for (int s = 0; s < kRun; ++s)
-                v[f][s] = (kz0 + s < a.zlen) ? a.dk[f][rowoff + kz0 + s] : make_float2(0.f, 0.f);
+                for (int q = 0; q < 4; ++q) {
+                    const float4 *src = (const float4 *)(a.dk[f] + ro[q]);
+                    const float4 x = src[0], y = src[1];
+                    v[f][q][0] = make_float2(x.x, x.y);
+                    v[f][q][1] = make_float2(x.z, x.w);
+                    v[f][q][2] = make_float2(y.x, y.y);
+                    v[f][q][3] = make_float2(y.z, y.w);
+                }
+        } else {
+#pragma unroll
+            for (int f = 0; f < NFL; ++f)
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
+#pragma unroll
+                    for (int s = 0; s < kRun; ++s)
+                        v[f][q][s] = (kz0 + s < a.zlen) ? a.dk[f][ro[q] + s] : make_float2(0.f, 0.f);
+        }
 
         int cur3 = -1, cur2 = -1;
         double r3[NA3], r2[S], p1[S];
@@ -422,7 +476,7 @@ __global__ void __launch_bounds__(kBinBlock) pk_bin_kernel(BinArgs a) {
         // most one: one test per mode instead of a square root
         int k2 = kxy2 + kz0 * kz0;
         int kidx = isqrt_i(k2);
-        int p2 = (AXIS == 0 ? ky * ky : kx * kx) + kz0 * kz0;
+        int p2 = (AXIS == 0 ? kb * kb : ka * ka) + kz0 * kz0;
         int kpr = (AXIS == 2) ? key : isqrt_i(p2);
 #pragma unroll
         for (int s = 0; s < kRun; ++s) {
@@ -435,36 +489,45 @@ __global__ void __launch_bounds__(kBinBlock) pk_bin_kernel(BinArgs a) {
                     kpr += ((kpr + 1) * (kpr + 1) <= p2) ? 1 : 0;
                 }
             }
-            bool ok = kz < a.zlen;
-            if (kz == 0 || (a.even && kz == a.m)) {     // Pk_library.pyx:324-327
-                if (kx_neg) ok = false;
-                else if (kx_edge && ky_neg) ok = false;
-            }
-            if (!ok) continue;
-            int kpar;
+            if (kz >= a.zlen) continue;
+            const unsigned mask = (kz == 0 || (a.even && kz == a.m)) ? prows : rows;
             const int kper = kpr;
-            if (AXIS == 0) kpar = kx < 0 ? -kx : kx;
-            else if (AXIS == 1) kpar = ky < 0 ? -ky : ky;
-            else kpar = kz;
+            const int kpar = AXIS == 0 ? ka : AXIS == 1 ? kb : kz;
             // mu^2 = k_par^2 / k^2 in float (hardware reciprocal, within 2 ulp)
             const float mu2 = (k2 == 0) ? 0.0f : (float)(kpar * kpar) * __builtin_amdgcn_rcpf((float)k2);
             const float L2 = 1.5f * mu2 - 0.5f;
             const float L4 = (35.0f * mu2 * mu2 - 30.0f * mu2 + 3.0f) * 0.125f;
 
-            double re[NFL], im[NFL];
+            float mf[NFL];
 #pragma unroll
-            for (int f = 0; f < NFL; ++f) {
-                const float mf = (float)(c01[f] * corrz[f * a.zlen + kz]);
-                const float xr = v[f][s].x * mf, xi = v[f][s].y * mf;   // complex64 * float
-                re[f] = (double)xr;
-                im[f] = (double)xi;
-            }
-            double d2[S];
-            // the products of floats are exact in double: one rounding, as re*re + im*im
-            d2[0] = fma(re[0], re[0], im[0] * im[0]);
-            if (NFL == 2) {
-                d2[1] = fma(re[1], re[1], im[1] * im[1]);
-                d2[2] = fma(re[0], re[1], im[0] * im[1]);
+            for (int f = 0; f < NFL; ++f) mf[f] = (float)(c01[f] * corrz[f * a.zlen + kz]);
+            double d2[S], ph2 = 0.0;
+#pragma unroll
+            for (int sp = 0; sp < S; ++sp) d2[sp] = 0.0;
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                // rows that are not there, or not independent, count with factor 0
+                const bool on = (mask >> q) & 1u;
+                double re[NFL], im[NFL];
+                float xr0 = 0.0f, xi0 = 0.0f;
+#pragma unroll
+                for (int f = 0; f < NFL; ++f) {
+                    const float mq = on ? mf[f] : 0.0f;
+                    const float xr = v[f][q][s].x * mq, xi = v[f][q][s].y * mq;   // complex64 * float
+                    re[f] = (double)xr;
+                    im[f] = (double)xi;
+                    if (f == 0) {
+                        xr0 = xr;
+                        xi0 = xi;
+                    }
+                }
+                // the products of floats are exact in double
+                d2[0] = fma(re[0], re[0], fma(im[0], im[0], d2[0]));
+                if (NFL == 2) {
+                    d2[1] = fma(re[1], re[1], fma(im[1], im[1], d2[1]));
+                    d2[2] = fma(re[0], re[1], fma(im[0], im[1], d2[2]));
+                }
+                if (PHASE) ph2 += (double)phase_sq(xr0, xi0);
             }
             // 3D: merge equal bins in registers, flush on change
             if (kidx != cur3) {
@@ -480,23 +543,10 @@ __global__ void __launch_bounds__(kBinBlock) pk_bin_kernel(BinArgs a) {
 #pragma unroll
             for (int sp = 0; sp < S; ++sp) {
                 r3[3 * sp + 0] += d2[sp];
-                r3[3 * sp + 1] += d2[sp] * (double)L2;
-                r3[3 * sp + 2] += d2[sp] * (double)L4;
+                r3[3 * sp + 1] = fma(d2[sp], (double)L2, r3[3 * sp + 1]);
+                r3[3 * sp + 2] = fma(d2[sp], (double)L4, r3[3 * sp + 2]);
             }
-            if (PHASE) {
-                // atan2(Re, |delta|) from the float components scaled by a power of two
-                // near 1/max(|Re|, |Im|) (exact): |delta|^2 formed in float would
-                // overflow or underflow for |delta| beyond ~1e19 or below ~1e-19
-                float ph = 0.0f;
-                const float xr = (float)re[0], xi = (float)im[0];
-                const float mx = fmaxf(fabsf(xr), fabsf(xi));
-                if (mx > 0.0f) {
-                    const int e = __builtin_amdgcn_frexp_expf(mx);
-                    const float xs = __builtin_ldexpf(xr, -e), ys = __builtin_ldexpf(xi, -e);
-                    ph = atan_halfplane(xs, __builtin_amdgcn_sqrtf(xs * xs + ys * ys));
-                }
-                r3[NA3 - 1] += (double)(ph * ph);
-            }
+            if (PHASE) r3[NA3 - 1] += ph2;
             // 2D line: axes 0/1 index k_per (slowly varying), axis 2 index kz
             const int li = (AXIS == 2) ? kz : kper;
             if (AXIS == 2) {
@@ -798,12 +848,12 @@ int launch_bin(Ctx *c, const BinPlan *bp, const PkDims &p, const float2 *const *
     const int n3 = (p.kmax + 1) * NA3;
     const int P = n3 + (L2 + L1) * S;
     const int off2 = n3, off1 = n3 + L2 * S;
-    const int rmax = bp->R;
+    const int gmax = bp->G;
     // LDS: P low words (8 B) and P high words (4 B, padded to an even count), the
-    // kz corrections, the row corrections and the row table
+    // kz corrections, the group corrections and the group table
     size_t lds = sizeof(unsigned long long) * (size_t)P + sizeof(int) * (size_t)((P + 1) & ~1) +
-                 sizeof(double) * ((size_t)p.zlen * NFL + (size_t)rmax * NFL) +
-                 sizeof(int) * 3 * (size_t)rmax;
+                 sizeof(double) * ((size_t)p.zlen * NFL + (size_t)gmax * NFL) +
+                 sizeof(int) * (size_t)gmax;
     PYL_CHECK(lds <= 160 * 1024, PYL_EINVAL, "grid too large for the binning kernel (%zu B LDS)", lds);
     // scratch: partials (low words | high words), reduced outputs, chunk sums, scales
     const size_t part_elems = (size_t)bp->nitems * P * nreal;
@@ -833,7 +883,7 @@ int launch_bin(Ctx *c, const BinPlan *bp, const PkDims &p, const float2 *const *
     }
     a.escale = escale;
     a.nreal = nreal;
-    a.rows = bp->d_rows;
+    a.groups = bp->d_groups;
     a.items = bp->d_items;
     a.plo = plo;
     a.phi = phi;
@@ -841,7 +891,11 @@ int launch_bin(Ctx *c, const BinPlan *bp, const PkDims &p, const float2 *const *
     a.zs = zs;
     a.nitems = bp->nitems;
     a.dims = p.dims; a.m = p.m; a.zlen = p.zlen; a.zpad = p.zpad; a.even = p.even;
-    a.kmax = p.kmax; a.L2 = L2; a.L1 = L1; a.P = P; a.off2 = off2; a.off1 = off1; a.rmax = rmax;
+    a.kmax = p.kmax; a.L2 = L2; a.L1 = L1; a.P = P; a.off2 = off2; a.off1 = off1; a.gmax = gmax;
+    // 16-byte loads of a run's four modes: rows padded to zpad (the padding is read and
+    // not used) and 16-byte aligned, as the own passes' buffer has them
+    a.wide = zs >= p.zpad && zs % 2 == 0 && fstride % 2 == 0;
+    for (int f = 0; f < NFL; ++f) a.wide = a.wide && ((uintptr_t)dk[f] & 15) == 0;
     auto kern = pk_bin_kernel<AXIS, NFL, PHASE>;
     PYL_TRY(set_lds(kern, lds));
     PYL_TRY(stage_begin(c, PYL_STAGE_PK_BIN));

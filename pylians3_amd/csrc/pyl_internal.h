@@ -91,13 +91,13 @@ struct ModePlan {
     std::vector<double> N1D, N2D, N3D, k1D, k3D;
 };
 
-// Rows of the half-complex cube grouped by binning key and cut into work items
-// (device-resident).
+// Row groups (|kx|, |ky|) of the half-complex cube ordered by binning key and cut into
+// work items of up to G groups (device-resident).
 struct BinPlan {
-    int dims = 0, axis = 0, R = 0;
+    int dims = 0, axis = 0, G = 0;
     int nitems = 0, nkeys = 0;
-    int *d_rows = nullptr;       // kxx*dims + kyy, grouped by key
-    int4 *d_items = nullptr;     // (first row, nrows, key, 0)
+    int *d_groups = nullptr;     // |kx| << 16 | |ky|, ordered by key
+    int4 *d_items = nullptr;     // (first group, ngroups, key, 0)
     int *d_key_items = nullptr;  // [nkeys+1] item range of each key
 };
 
@@ -203,7 +203,7 @@ struct Ctx {
 // Tables that depend only on the grid, built once per process and shared by every
 // context (the device tables once per device), so that the slots of a server or the
 // threads of a pipeline do not each rebuild them: mode counts per (dims, axis),
-// binning plans per (device, dims, axis, rows per item), MAS corrections per (device,
+// binning plans per (device, dims, axis, groups per item), MAS corrections per (device,
 // dims, p) and FFT twiddles exp(-2 pi i k/N) per (device, N).  Built under `mu` and
 // never changed or freed afterwards (they live until the process ends).
 struct SharedTables {
