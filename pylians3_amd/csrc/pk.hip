@@ -626,117 +626,124 @@ __global__ void __launch_bounds__(kBinBlock) pk_bin_kernel(BinArgs a) {
 }
 
 // Sum the item partials (exact integer sums, so the order does not matter) and
-// convert each bin to double with its realisation's scale.  blockIdx.y =
-// realisation.  Output layout per realisation: out3[(kmax+1)*NA3], out2[nb2*S]
-// (reference 2D index), out1[(m+1)*S].
+// convert each bin to double with its realisation's scale.  Output layout per
+// realisation: out3[(kmax+1)*NA3], out2[nb2*S] (reference 2D index), out1[(m+1)*S].
 struct ReduceArgs {
     const unsigned long long *plo;
     const int *phi;
     const int *key_items;
     const int *escale;
     double *out3, *out2, *out1;
-    int nitems, nkeys, n3, L2, L1, S, P, off2, off1, axis, kmax_par, nreal;
+    int nitems, nkeys, n3, na3, L2, L1, S, P, off2, off1, axis, kmax_par, nreal;
     long long nb2, n1;       // out2 / out1 elements per realisation (nb2*S, (m+1)*S)
 };
 
-// Columns summed over every item (3D bins; the 1D line for axis 2) are reduced
-// in two stages: chunks of kRedChunk items, then the chunk sums.
-constexpr int kRedChunk = 64;
+// All reductions of a binning launch in one launch of kRedBlock threads, by block range:
+//  * g3 blocks: columns every item contributes to (the 3D bins; the 1D line for axis
+//    2), 16 columns x 64 slices of the items per block, one realisation per xb blocks;
+//  * g2 blocks: the 2D line, each bin the sum of its key's items (blocks of 1024 bins
+//    for axis 2, whose output order is the partials' order; tiles of 32 keys x about 32
+//    line entries for axes 0 and 1, turned round in LDS, since k_par = key runs fastest
+//    in the output);
+//  * g1 blocks: axes 0/1, the 1D bins (k_par = key).
+// The outputs go straight into the pinned host buffer the caller reads after the
+// stream, in runs of whole cache lines.  Latency-bound: the chunk sums, their sum, the
+// 1D line's own pair of launches (axis 2) and the download used to take 36 us at 64^3
+// and 46 us at 512^3 for microseconds of data movement; now 4 and 28 us, and Pk of a 64^3
+// field went from 98 to 70 us, of a 512^3 field from 1084 to 1057 us.
+constexpr int kRedBlock = 1024;
+constexpr int kRedCols = 16;                       // columns per block (128 B of low words)
+constexpr int kRedSlices = kRedBlock / kRedCols;
 
-// (tlo, thi)[r][ch][c] = sum over items of chunk ch (of nch) of the partials' column
-// col0 + c, realisation r
-__device__ __forceinline__ void reduce_chunk_col(const unsigned long long *__restrict__ plo,
-                                                 const int *__restrict__ phi, int nitems, int P, int col0,
-                                                 int ncol, unsigned long long *__restrict__ tlo,
-                                                 long long *__restrict__ thi, int c, int ch, int nch, int r) {
-    const long long base = (long long)r * nitems * P + col0 + c;
-    const int i0 = ch * kRedChunk, i1 = min(nitems, i0 + kRedChunk);
-    unsigned long long slo = 0;
-    long long shi = 0;
-#pragma unroll 8
-    for (int it = i0; it < i1; ++it) fix_acc(slo, shi, plo[base + (long long)it * P], phi[base + (long long)it * P]);
-    const long long o = ((long long)r * nch + ch) * ncol + c;
-    tlo[o] = slo;
-    thi[o] = shi;
-}
+// Line columns per tile of the 2D transpose: whole line entries of S spectra.
+__host__ __device__ __forceinline__ int red_tile_cols(int S) { return 32 / S * S; }
 
-__global__ void pk_reduce_chunks_kernel(const unsigned long long *__restrict__ plo,
-                                        const int *__restrict__ phi, int nitems, int P,
-                                        int col0, int ncol, unsigned long long *__restrict__ tlo,
-                                        long long *__restrict__ thi) {
-    const int c = blockIdx.x * blockDim.x + threadIdx.x;
-    if (c >= ncol) return;
-    reduce_chunk_col(plo, phi, nitems, P, col0, ncol, tlo, thi, c, blockIdx.y, gridDim.y, blockIdx.z);
-}
-
-// out[r*ostride + c] = sum over chunks of (tlo, thi)[r][ch][c], as a double; with
-// na3 > 0, column c of the 3D block is a phase sum when c % na3 == na3 - 1
-__global__ void pk_reduce_final_kernel(const unsigned long long *__restrict__ tlo,
-                                       const long long *__restrict__ thi, int nch, int ncol,
-                                       double *__restrict__ out, long long ostride,
-                                       const int *__restrict__ escale, int na3) {
-    const int c = blockIdx.x * blockDim.x + threadIdx.x;
-    if (c >= ncol) return;
-    const long long t0 = (long long)blockIdx.y * nch * ncol + c;
-    unsigned long long slo = 0;
-    long long shi = 0;
-    for (int ch = 0; ch < nch; ++ch) fix_acc(slo, shi, tlo[t0 + (long long)ch * ncol], thi[t0 + (long long)ch * ncol]);
-    const int E = escale[2 * blockIdx.y + ((na3 > 0 && c % na3 == na3 - 1) ? 1 : 0)];
-    out[(long long)blockIdx.y * ostride + c] = fix_value(slo, shi, E);
-}
-
-// 2D line element i = (key, line index, spectrum) of realisation r: sums the key's items.
-__device__ __forceinline__ void reduce2_elem(const ReduceArgs &a, long long i, int r) {
-    const long long base = (long long)r * a.nitems * a.P;
-    int sp = (int)(i % a.S);
-    int li = (int)((i / a.S) % a.L2);
-    int key = (int)(i / ((long long)a.S * a.L2));
-    unsigned long long slo = 0;
-    long long shi = 0;
-    for (int it = a.key_items[key]; it < a.key_items[key + 1]; ++it) {
-        const long long j = base + (long long)it * a.P + a.off2 + li * a.S + sp;
+__device__ __forceinline__ void reduce_key_items(const ReduceArgs &a, int key, int col, long long base,
+                                                 unsigned long long &slo, long long &shi) {
+    slo = 0;
+    shi = 0;
+    const int i1 = a.key_items[key + 1];
+#pragma unroll 4
+    for (int it = a.key_items[key]; it < i1; ++it) {
+        const long long j = base + (long long)it * a.P + col;
         fix_acc(slo, shi, a.plo[j], a.phi[j]);
     }
-    // reference 2D index: (kmax_par+1)*k_per + k_par
-    long long idx2 = (a.axis == 2) ? (long long)(a.kmax_par + 1) * key + li
-                                   : (long long)(a.kmax_par + 1) * li + key;
-    a.out2[(long long)r * a.nb2 + idx2 * a.S + sp] = fix_value(slo, shi, a.escale[2 * r]);
 }
 
-// Axes 0/1: 1D bin = key = k_par; element i = (key, spectrum) sums the key's items.
-// (Axis 2 keeps one 1D line per item and goes through the chunked reduction.)
-__device__ __forceinline__ void reduce1_elem(const ReduceArgs &a, int i, int r) {
-    const long long base = (long long)r * a.nitems * a.P;
-    double *out1 = a.out1 + (long long)r * a.n1;
-    int key = i / a.S, sp = i % a.S;
-    unsigned long long slo = 0;
-    long long shi = 0;
-    for (int it = a.key_items[key]; it < a.key_items[key + 1]; ++it) {
-        const long long j = base + (long long)it * a.P + a.off1 + sp;
-        fix_acc(slo, shi, a.plo[j], a.phi[j]);
-    }
-    out1[key * a.S + sp] = fix_value(slo, shi, a.escale[2 * r]);
-}
-
-// The independent first reductions in one launch of 256-thread blocks, by block
-// range: the 3D columns' chunk sums (g3 = ceil(n3/256) * nch * nreal blocks), then
-// the 2D line (g2 blocks), then for axes 0/1 the 1D line (g1 blocks).
-__global__ void __launch_bounds__(256)
-pk_reduce_first_kernel(ReduceArgs a, unsigned long long *__restrict__ tlo, long long *__restrict__ thi,
-                       int nch, int g3, int g2) {
+__global__ void __launch_bounds__(kRedBlock)
+pk_reduce_kernel(ReduceArgs a, int g3, int g2) {
+    __shared__ unsigned long long slo_s[kRedBlock / 64][kRedCols];
+    __shared__ long long shi_s[kRedBlock / 64][kRedCols];
+    __shared__ double tile[32][33];
     const int b = blockIdx.x, t = threadIdx.x;
     if (b < g3) {
-        const int xb = (a.n3 + 255) / 256;
-        const int c = (b % xb) * 256 + t, rest = b / xb;
-        if (c < a.n3) reduce_chunk_col(a.plo, a.phi, a.nitems, a.P, 0, a.n3, tlo, thi, c, rest % nch, nch, rest / nch);
+        const int xb = g3 / a.nreal, r = b / xb;
+        const int ncol = a.n3 + (a.axis == 2 ? a.L1 * a.S : 0);
+        const int c = (b - r * xb) * kRedCols + (t & (kRedCols - 1));
+        unsigned long long lo = 0;
+        long long hi = 0;
+        if (c < ncol) {
+            const long long base = (long long)r * a.nitems * a.P + (c < a.n3 ? c : a.off1 + c - a.n3);
+#pragma unroll 4
+            for (int it = t / kRedCols; it < a.nitems; it += kRedSlices) {
+                const long long j = base + (long long)it * a.P;
+                fix_acc(lo, hi, a.plo[j], a.phi[j]);
+            }
+        }
+#pragma unroll
+        for (int o = kRedCols; o < 64; o <<= 1) {
+            const unsigned long long olo = (unsigned long long)__shfl_xor((long long)lo, o);
+            const long long ohi = __shfl_xor(hi, o);
+            fix_acc(lo, hi, olo, ohi);
+        }
+        if ((t & 63) < kRedCols) {
+            slo_s[t >> 6][t & 63] = lo;
+            shi_s[t >> 6][t & 63] = hi;
+        }
+        __syncthreads();
+        if (t >= kRedCols || c >= ncol) return;
+        for (int w = 1; w < kRedBlock / 64; ++w) fix_acc(lo, hi, slo_s[w][t], shi_s[w][t]);
+        const int E = a.escale[2 * r + ((c < a.n3 && a.na3 > 0 && c % a.na3 == a.na3 - 1) ? 1 : 0)];
+        const double v = fix_value(lo, hi, E);
+        if (c < a.n3) a.out3[(long long)r * a.n3 + c] = v;
+        else a.out1[(long long)r * a.n1 + (c - a.n3)] = v;
     } else if (b < g3 + g2) {
-        const int xb = g2 / a.nreal, bb = b - g3;
-        const long long i = (long long)(bb % xb) * 256 + t;
-        if (i < (long long)a.nkeys * a.L2 * a.S) reduce2_elem(a, i, bb / xb);
+        const int xb = g2 / a.nreal, bb = b - g3, r = bb / xb, x = bb - r * xb;
+        const long long base = (long long)r * a.nitems * a.P;
+        const int E = a.escale[2 * r];
+        double *out2 = a.out2 + (long long)r * a.nb2;
+        const int ncol = a.L2 * a.S;
+        unsigned long long lo;
+        long long hi;
+        if (a.axis == 2) {
+            const long long i = (long long)x * kRedBlock + t;     // (key, line entry, spectrum)
+            if (i >= (long long)a.nkeys * ncol) return;
+            reduce_key_items(a, (int)(i / ncol), a.off2 + (int)(i % ncol), base, lo, hi);
+            out2[i] = fix_value(lo, hi, E);                       // (kmax_par+1) == L2
+            return;
+        }
+        const int tc = red_tile_cols(a.S), nct = (ncol + tc - 1) / tc;
+        const int c0 = x % nct * tc, k0 = x / nct * 32;
+        const int key = k0 + (t >> 5), c = c0 + (t & 31);
+        if (key < a.nkeys && (t & 31) < tc && c < ncol) {
+            reduce_key_items(a, key, a.off2 + c, base, lo, hi);
+            tile[t >> 5][t & 31] = fix_value(lo, hi, E);
+        }
+        __syncthreads();
+        // line entry l, keys k0.. and spectra: consecutive in the output
+        if (t >= 32 * tc) return;
+        const int l = t / (32 * a.S), rest = t - l * 32 * a.S, kl = rest / a.S, sp = rest - kl * a.S;
+        const int cl = l * a.S + sp;
+        if (k0 + kl < a.nkeys && c0 + cl < ncol)
+            out2[((long long)(a.kmax_par + 1) * (c0 / a.S + l) + k0 + kl) * a.S + sp] = tile[kl][cl];
     } else {
-        const int bb = b - g3 - g2, xb = (a.nkeys * a.S + 255) / 256;
-        const int i = (bb % xb) * 256 + t;
-        if (i < a.nkeys * a.S) reduce1_elem(a, i, bb / xb);
+        const int bb = b - g3 - g2, xb = (a.nkeys * a.S + kRedBlock - 1) / kRedBlock, r = bb / xb;
+        const int i = (bb - r * xb) * kRedBlock + t;
+        if (i >= a.nkeys * a.S) return;
+        unsigned long long lo;
+        long long hi;
+        reduce_key_items(a, i / a.S, a.off1 + i % a.S, (long long)r * a.nitems * a.P, lo, hi);
+        a.out1[(long long)r * a.n1 + i] = fix_value(lo, hi, a.escale[2 * r]);
     }
 }
 
@@ -855,24 +862,26 @@ int launch_bin(Ctx *c, const BinPlan *bp, const PkDims &p, const float2 *const *
                  sizeof(double) * ((size_t)p.zlen * NFL + (size_t)gmax * NFL) +
                  sizeof(int) * (size_t)gmax;
     PYL_CHECK(lds <= 160 * 1024, PYL_EINVAL, "grid too large for the binning kernel (%zu B LDS)", lds);
-    // scratch: partials (low words | high words), reduced outputs, chunk sums, scales
+    // scratch: partials (low words | high words), scales
     const size_t part_elems = (size_t)bp->nitems * P * nreal;
     const size_t out3 = (size_t)n3, out2 = (size_t)p.nb2 * S, out1 = (size_t)(p.m + 1) * S;
-    const int nch = ceil_div(bp->nitems, kRedChunk);
-    const int ncol_all = (AXIS == 2) ? std::max(n3, L1 * S) : n3;
-    const size_t tmp_elems = (size_t)nch * ncol_all * nreal;
     const size_t phi_bytes = (sizeof(int) * part_elems + 7) & ~(size_t)7;
     PYL_TRY(ensure(c, BUF_BINS, sizeof(unsigned long long) * part_elems + phi_bytes +
-                                    sizeof(double) * (out3 + out2 + out1) * nreal +
-                                    2 * sizeof(long long) * tmp_elems + sizeof(int) * 2 * (size_t)nreal));
+                                    sizeof(int) * 2 * (size_t)nreal));
     unsigned long long *plo = (unsigned long long *)c->bufs[BUF_BINS].ptr;
     int *phi = (int *)(plo + part_elems);
-    double *d3 = (double *)((char *)phi + phi_bytes);
-    double *d2 = d3 + out3 * nreal;
-    double *d1 = d2 + out2 * nreal;
-    unsigned long long *tlo = (unsigned long long *)(d1 + out1 * nreal);
-    long long *thi = (long long *)(tlo + tmp_elems);
-    int *escale = (int *)(thi + tmp_elems);
+    int *escale = (int *)((char *)phi + phi_bytes);
+    // the reduced outputs (3D | 2D | 1D) are written into pinned memory by the reduction
+    const size_t nout = (out3 + out2 + out1) * nreal;
+    void *hp = nullptr;
+    if (c->capturing) {
+        // a pinned buffer of the graph's own; the host part runs after each replay
+        PYL_HIP(hipHostMalloc(&hp, sizeof(double) * nout, hipHostMallocDefault));
+        c->cap_host.push_back(hp);
+    } else {
+        PYL_TRY(pinned(c, c->pin_down, sizeof(double) * nout, &hp));
+    }
+    double *h3 = (double *)hp, *h2 = h3 + out3 * nreal, *h1 = h2 + out2 * nreal;
 
     BinArgs a{};
     for (int f = 0; f < NFL; ++f) {
@@ -903,40 +912,20 @@ int launch_bin(Ctx *c, const BinPlan *bp, const PkDims &p, const float2 *const *
     PYL_HIP(hipGetLastError());
     ReduceArgs r{};
     r.plo = plo; r.phi = phi; r.escale = escale;
-    r.key_items = bp->d_key_items; r.out3 = d3; r.out2 = d2; r.out1 = d1;
-    r.nitems = bp->nitems; r.nkeys = bp->nkeys; r.n3 = n3; r.L2 = L2; r.L1 = L1; r.S = S;
-    r.P = P; r.off2 = off2; r.off1 = off1; r.axis = AXIS; r.kmax_par = p.kmax_par;
-    r.nb2 = (long long)out2; r.n1 = (long long)out1; r.nreal = nreal;
-    // 3D bins (every item contributes: chunk sums, then their sum), the 2D line and,
-    // for axes 0/1, the 1D line (each bin from its key's items): the first stages in
-    // one launch
-    const long long n2 = (long long)bp->nkeys * L2 * S;
-    const long long g3 = (long long)ceil_div(n3, 256) * nch * nreal;
-    const long long g2 = (n2 + 255) / 256 * nreal;
-    const long long g1 = AXIS == 2 ? 0 : (long long)ceil_div(bp->nkeys * S, 256) * nreal;
+    r.key_items = bp->d_key_items; r.out3 = h3; r.out2 = h2; r.out1 = h1;
+    r.nitems = bp->nitems; r.nkeys = bp->nkeys; r.n3 = n3; r.na3 = PHASE ? NA3 : 0;
+    r.L2 = L2; r.L1 = L1; r.S = S; r.P = P; r.off2 = off2; r.off1 = off1; r.axis = AXIS;
+    r.kmax_par = p.kmax_par; r.nb2 = (long long)out2; r.n1 = (long long)out1; r.nreal = nreal;
+    const long long g3 = (long long)ceil_div(n3 + (AXIS == 2 ? L1 * S : 0), kRedCols) * nreal;
+    const long long ncol2 = (long long)L2 * S;
+    const long long g2 = (AXIS == 2 ? (bp->nkeys * ncol2 + kRedBlock - 1) / kRedBlock
+                                    : (long long)ceil_div((int)ncol2, red_tile_cols(S)) * ceil_div(bp->nkeys, 32)) *
+                         nreal;
+    const long long g1 = AXIS == 2 ? 0 : (long long)ceil_div(bp->nkeys * S, kRedBlock) * nreal;
     PYL_CHECK(g3 + g2 + g1 < (1ll << 31), PYL_EINVAL, "binning reduction too large");
-    pk_reduce_first_kernel<<<(unsigned)(g3 + g2 + g1), 256, 0, c->stream>>>(r, tlo, thi, nch, (int)g3, (int)g2);
-    pk_reduce_final_kernel<<<dim3(ceil_div(n3, 256), nreal), 256, 0, c->stream>>>(
-        tlo, thi, nch, n3, d3, (long long)out3, escale, PHASE ? NA3 : 0);
-    if (AXIS == 2) {   // 1D bins are k_par = kz: every item contributes
-        pk_reduce_chunks_kernel<<<dim3(ceil_div(L1 * S, 256), nch, nreal), 256, 0, c->stream>>>(
-            plo, phi, bp->nitems, P, off1, L1 * S, tlo, thi);
-        pk_reduce_final_kernel<<<dim3(ceil_div(L1 * S, 256), nreal), 256, 0, c->stream>>>(
-            tlo, thi, nch, L1 * S, d1, (long long)out1, escale, 0);
-    }
+    pk_reduce_kernel<<<(unsigned)(g3 + g2 + g1), kRedBlock, 0, c->stream>>>(r, (int)g3, (int)g2);
     PYL_HIP(hipGetLastError());
     PYL_TRY(stage_end(c, PYL_STAGE_PK_BIN));
-    // d3 | d2 | d1 are contiguous: one DMA into pinned memory
-    const size_t nout = (out3 + out2 + out1) * nreal;
-    void *hp = nullptr;
-    if (c->capturing) {
-        // a pinned buffer of the graph's own; the host part runs after each replay
-        PYL_HIP(hipHostMalloc(&hp, sizeof(double) * nout, hipHostMallocDefault));
-        c->cap_host.push_back(hp);
-    } else {
-        PYL_TRY(pinned(c, c->pin_down, sizeof(double) * nout, &hp));
-    }
-    PYL_HIP(hipMemcpyAsync(hp, d3, sizeof(double) * nout, hipMemcpyDeviceToHost, c->stream));
     if (c->capturing) {
         std::array<int, Spec<NFL>::S> so;
         for (int sp = 0; sp < Spec<NFL>::S; ++sp) so[sp] = spec_out[sp];
