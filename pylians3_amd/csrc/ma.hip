@@ -118,21 +118,18 @@ __host__ __device__ __forceinline__ void foot_weights(float dist, int raw, float
         C[0] = 0.5f * q0;
         C[2] = 0.5f * q2;
     } else {
-        // PCS, MAS_library.pyx:485-492 (double polynomials, rounded to float).
-        // With raw = floor(dist) - 1, d0 and d3 lie in [1, 2] and d1, d2 in
-        // [0, 1] (after float rounding too); at d = 1 and d = 2 both branches
-        // of the reference give the same double.
-        float d[4];
-#pragma unroll
-        for (int j = 0; j < 4; ++j) d[j] = fabsf(((float)raw + (float)j) - dist);
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const double dd = (double)d[j];
-            if (j == 1 || j == 2)
-                C[j] = (float)((4.0 - 6.0 * dd * dd + 3.0 * dd * dd * dd) / 6.0);
-            else
-                C[j] = (float)((2.0 - dd) * (2.0 - dd) * (2.0 - dd) / 6.0);
-        }
+        // PCS, MAS_library.pyx:485-492 (double polynomials, rounded to float) at the
+        // distances 1+f, f, 1-f, 2-f of the four nodes, f = dist - floor(dist) exact.
+        // (2-d)^3/6 and 2/3 - d^2 + d^3/2 = (4 - 6 d^2 + 3 d^3)/6 are formed with
+        // constant factors and fused multiply-adds: the twelve double divisions by 6 of
+        // a record took as long as its 64 atomics.
+        const double u = (double)(dist - (float)(raw + 1)), v = 1.0 - u;
+        const double u2 = u * u, v2 = v * v;
+        constexpr double sixth = 1.0 / 6.0, two3 = 2.0 / 3.0;
+        C[0] = (float)(v2 * (v * sixth));
+        C[1] = (float)fma(u2, fma(0.5, u, -1.0), two3);
+        C[2] = (float)fma(v2, fma(0.5, v, -1.0), two3);
+        C[3] = (float)(u2 * (u * sixth));
     }
 }
 
@@ -1443,8 +1440,51 @@ __device__ __forceinline__ float4 load_set_record(const float *__restrict__ set,
     return make_float4(p[0], p[1], p[2], 1.0f);
 }
 
-// Box offset of a record's first footprint node (records of this tile satisfy
-// 0 <= l < e on every axis; the clamp only guards the LDS box).
+// ---- LDS box layout ------------------------------------------------------------
+// A wave's ds_add_u64 is served in passes of 16 lanes; an 8-byte word at offset e is in
+// bank pair e mod 16, and lanes of a pass that agree mod 16 wait for each other.
+//  * CIC and PCS (two and four nodes per axis): the low bits of a node's offset are the
+//    low bits of its coordinates (PCS 3D: z mod 4 + 4 (y mod 4); 2D: y mod 4 + 4 (x mod
+//    4); CIC 3D: z mod 2 + 2 (y mod 2) + 4 (x mod 2); 2D: y mod 2 + 2 (x mod 2)).  A
+//    footprint then has exactly one node of every residue per axis, so the lanes can
+//    go through their nodes in an order of their own in which the 16 lanes of a pass
+//    always have different residues (deposit_rot): no bank conflict whatever the
+//    positions (PCS), or only those of the remaining bits (CIC).
+//  * NGP and TSC: plain rows.
+template <int MAS>
+constexpr bool box_rot() { return MAS == PYL_CIC || MAS == PYL_PCS; }
+
+// Nodes per axis of a box, and blocks of MAS nodes that hold them (swizzled layouts).
+template <int MAS, int AXES>
+struct BoxDim {
+    static constexpr int B = (AXES == 3 ? kT3 : kT2) + MAS - 1;
+    static constexpr int NBLK = (B + MAS - 1) / MAS;
+    static constexpr int words =
+        !box_rot<MAS>() ? (AXES == 3 ? B * B * B : B * B)
+        : AXES == 2     ? MAS * MAS * NBLK * NBLK
+        : MAS == PYL_PCS ? MAS * MAS * NBLK * NBLK * B
+                         : MAS * MAS * MAS * NBLK * NBLK * NBLK;
+    // word strides of a block step along x (PCS 3D: a node step), y, z
+    static constexpr int sz = AXES == 2 ? 0 : MAS == PYL_PCS ? 16 : 8;
+    static constexpr int sy = AXES == 2 ? MAS * MAS : sz * NBLK;
+    static constexpr int sx = sy * NBLK;
+};
+
+// Offset of node (x, y, z) of a box.
+template <int MAS, int AXES>
+__host__ __device__ __forceinline__ int box_off(int x, int y, int z) {
+    using D = BoxDim<MAS, AXES>;
+    if constexpr (!box_rot<MAS>()) return AXES == 3 ? (x * D::B + y) * D::B + z : x * D::B + y;
+    else if constexpr (AXES == 2)
+        return (x / MAS) * D::sx + (y / MAS) * D::sy + (x % MAS) * MAS + y % MAS;
+    else if constexpr (MAS == PYL_PCS)
+        return x * D::sx + (y / MAS) * D::sy + (z / MAS) * D::sz + (y % MAS) * MAS + z % MAS;
+    else
+        return (x / MAS) * D::sx + (y / MAS) * D::sy + (z / MAS) * D::sz + (x % MAS) * 4 + (y % MAS) * 2 + z % MAS;
+}
+
+// Box offset of a record's first footprint node in the plain layout (records of this
+// tile satisfy 0 <= l < e on every axis; the clamp only guards the LDS box).
 template <int MAS, int AXES>
 __host__ __device__ __forceinline__ int box_base(const float4 &rec, const TileGeom &g, const TileBox &tb) {
     constexpr int F = MAS;
@@ -1469,6 +1509,23 @@ __host__ __device__ __forceinline__ int box_base_uni(const float4 &rec) {
     const int ly = first_node<MAS>(rec.y) & (kT3 - 1);
     const int lz = first_node<MAS>(rec.z) & (kT3 - 1);
     return (lx * B + ly) * B + lz;
+}
+
+// Box coordinates of a record's first node (as box_base, box_base_uni).
+template <int MAS, int AXES, bool UNI>
+__host__ __device__ __forceinline__ int3 box_coords(const float4 &rec, const TileGeom &g, const TileBox &tb) {
+    int3 l = make_int3(first_node<MAS>(rec.x), first_node<MAS>(rec.y), AXES == 3 ? first_node<MAS>(rec.z) : 0);
+    if constexpr (UNI) {
+        constexpr int T = AXES == 3 ? kT3 : kT2;
+        l.x &= T - 1;
+        l.y &= T - 1;
+        l.z &= T - 1;
+    } else {
+        l.x = min(max(wrap_node(l.x, g.dims) - tb.ox, 0), tb.ex - 1);
+        l.y = min(max(wrap_node(l.y, g.dims) - tb.oy, 0), tb.ey - 1);
+        if (AXES == 3) l.z = min(max(wrap_node(l.z, g.dims) - tb.oz, 0), tb.ez - 1);
+    }
+    return l;
 }
 
 // Bank class of a record for dealing it to an atomic round: its box offset mod
@@ -1580,10 +1637,112 @@ __device__ __forceinline__ void deposit_record(unsigned long long *a, const floa
     }
 }
 
-// Records each wave stages per round set in the bank-balanced deposit: KR per
-// lane (fewer for the PCS 3D box, so that two workgroups still fit one CU).
-template <int MAS, int AXES>
-constexpr int dep_kr() { return (MAS == 4 && AXES == 3) ? 2 : 4; }
+// One axis of a lane's own node order: in step s the lane takes the node whose
+// coordinate is r = (res + s) mod F (res: the lane's residue on this axis), i.e. node
+// (r - l) mod F of the footprint that starts at l.  w[s]: its weight, off[s]: its byte
+// offset past the block of l (stride: bytes per block step, unit: per node).
+template <int F>
+__host__ __device__ __forceinline__ void rot_axis(const float *C, int l, int res, int unit, int stride, float *w, int *off) {
+    const int lr = l & (F - 1);
+    if constexpr (F == 2) {
+        const bool swap = ((res ^ l) & 1) != 0;
+        w[0] = swap ? C[1] : C[0];
+        w[1] = swap ? C[0] : C[1];
+    } else {
+        const bool r1 = ((res - l) & 1) != 0, r2 = ((res - l) & 2) != 0;
+        const float a0 = r1 ? C[1] : C[0], a1 = r1 ? C[2] : C[1], a2 = r1 ? C[3] : C[2], a3 = r1 ? C[0] : C[3];
+        w[0] = r2 ? a2 : a0;
+        w[1] = r2 ? a3 : a1;
+        w[2] = r2 ? a0 : a2;
+        w[3] = r2 ? a1 : a3;
+    }
+#pragma unroll
+    for (int s = 0; s < F; ++s) {
+        const int r = (res + s) & (F - 1);
+        off[s] = r * unit + (r < lr ? stride : 0);
+    }
+}
+
+// One atomic of a record: the weight product p (in the reference's order) as quanta.
+template <bool WT, bool FX>
+__device__ __forceinline__ void add_quanta(char *box, int off, float p, float w) {
+    unsigned long long *a = (unsigned long long *)(box + off);
+    if constexpr (WT) {
+        const float c = p * w;
+        atomicAdd(a, FX ? fix64(c) : (unsigned long long)(long long)(int)c);
+    } else {
+        atomicAdd(a, (unsigned long long)(unsigned)p);
+    }
+}
+
+// Deposit of one record with first node l (box coordinates) for the swizzled boxes: the
+// same contributions as deposit_record, each lane taking its nodes in the order that
+// gives the 16 lanes of a pass different banks.  PCS (3D) is bound by its 64 LDS
+// atomics (6.1 clk each at best: 10.7 ms for 1.07 G particles) and about 290 VALU
+// instructions per record; with no conflicts and no sorting of the records (a wave used to
+// deal them to rounds by residue, about 110 VALU instructions and 6 LDS operations per
+// record) the deposit of 1024^3 particles on 1024^3 takes 14.4 ms instead of 22.4.  CIC
+// (8 atomics): 3D 0.37 ms for 32 x 128^3 both ways, MA of 4 M particles on a 1024^2 map
+// 129 -> 120 us (PCS 160 -> 134 us).
+template <int MAS, int AXES, bool WT, bool FX>
+__device__ __forceinline__ void deposit_rot(char *box, const float4 &rec, const int3 &l, int lane, float to_q,
+                                            float weight_factor) {
+    constexpr int F = MAS;
+    using D = BoxDim<MAS, AXES>;
+    float C[4], wx[4], wy[4], wz[4];
+    int ox[4], oy[4], oz[4];
+    const float w = WT ? (rec.w * weight_factor) * to_q : 1.0f;
+    if constexpr (AXES == 3) {
+        foot_weights<MAS>(rec.z, first_node<MAS>(rec.z), C);
+        if (!WT)
+#pragma unroll
+            for (int k = 0; k < F; ++k) C[k] *= to_q;     // exact (a power of two)
+        rot_axis<F>(C, l.z, lane & (F - 1), 8, 8 * D::sz, wz, oz);
+        foot_weights<MAS>(rec.y, first_node<MAS>(rec.y), C);
+        rot_axis<F>(C, l.y, (lane / F) & (F - 1), 8 * F, 8 * D::sy, wy, oy);
+        foot_weights<MAS>(rec.x, first_node<MAS>(rec.x), C);
+        if constexpr (MAS == PYL_PCS) {
+            char *b = box + 8 * (l.x * D::sx + (l.y / F) * D::sy + (l.z / F) * D::sz);
+#pragma unroll
+            for (int m = 0; m < F; ++m)
+#pragma unroll
+                for (int k = 0; k < F; ++k) {
+                    char *bb = b + oy[m] + oz[k];
+#pragma unroll
+                    for (int i = 0; i < F; ++i)
+                        add_quanta<WT, FX>(bb, 8 * i * D::sx, (C[i] * wy[m]) * wz[k], w);
+                }
+        } else {
+            rot_axis<F>(C, l.x, (lane / (F * F)) & (F - 1), 8 * F * F, 8 * D::sx, wx, ox);
+            char *b = box + 8 * ((l.x / F) * D::sx + (l.y / F) * D::sy + (l.z / F) * D::sz);
+#pragma unroll
+            for (int i = 0; i < F; ++i)
+#pragma unroll
+                for (int m = 0; m < F; ++m) {
+                    char *bb = b + ox[i] + oy[m];
+                    const float cxy = wx[i] * wy[m];
+#pragma unroll
+                    for (int k = 0; k < F; ++k) add_quanta<WT, FX>(bb, oz[k], cxy * wz[k], w);
+                }
+        }
+    } else {
+        foot_weights<MAS>(rec.y, first_node<MAS>(rec.y), C);
+        if (!WT)
+#pragma unroll
+            for (int k = 0; k < F; ++k) C[k] *= to_q;
+        rot_axis<F>(C, l.y, lane & (F - 1), 8, 8 * D::sy, wy, oy);
+        foot_weights<MAS>(rec.x, first_node<MAS>(rec.x), C);
+        rot_axis<F>(C, l.x, (lane / F) & (F - 1), 8 * F, 8 * D::sx, wx, ox);
+        char *b = box + 8 * ((l.x / F) * D::sx + (l.y / F) * D::sy);
+#pragma unroll
+        for (int i = 0; i < F; ++i)
+#pragma unroll
+            for (int m = 0; m < F; ++m) add_quanta<WT, FX>(b + ox[i], oy[m], wx[i] * wy[m], w);
+    }
+}
+
+// Records per lane of a wave's round set in the bank-balanced deposit.
+constexpr int kDepKR = 4;
 
 // ---- bank-balanced dealing of a wave's records to atomic rounds -------------
 // A wave instruction ds_add_u64 is served as four 16-lane passes (lanes 0-15,
@@ -1671,7 +1830,6 @@ __device__ __forceinline__ void flush_box(const unsigned long long *acc, int key
     constexpr int BY = T + F - 1;
     constexpr int BZ = (AXES == 3) ? T + F - 1 : 1;
     constexpr int BX = T + F - 1;
-    constexpr int NB = BX * BY * BZ;
     float *part = partials + (long long)key * g.pslot;
     if constexpr (UNI && AXES == 3) {
         // Uniform tile: the interior nodes go to the grid, the halo to the
@@ -1685,33 +1843,33 @@ __device__ __forceinline__ void flush_box(const unsigned long long *acc, int key
         const unsigned dd = (unsigned)g.dims * (unsigned)g.dims;
         for (int i = threadIdx.x; i < I * I * I; i += blockDim.x) {
             const int x = F - 1 + i / (I * I), y = F - 1 + (i / I) % I, z = F - 1 + i % I;
-            const float v = (float)((double)(long long)acc[(x * B + y) * B + z] * from_q);
+            const float v = (float)((double)(long long)acc[box_off<MAS, AXES>(x, y, z)] * from_q);
             store_node(grid, (long long)(node0 + (unsigned)x * dd + (unsigned)(y * g.dims + z)), v, om);
         }
         for (int i = threadIdx.x; i < H * B * B; i += blockDim.x) {
             const int xi = i / (B * B), yz = i - xi * (B * B);
             const int x = xi < F - 1 ? xi : xi + I;
-            part[i] = (float)((double)(long long)acc[x * B * B + yz] * from_q);
+            part[i] = (float)((double)(long long)acc[box_off<MAS, AXES>(x, yz / B, yz % B)] * from_q);
         }
         constexpr int SA = H * B * B;
         for (int i = threadIdx.x; i < I * H * B; i += blockDim.x) {
             const int x = F - 1 + i / (H * B), r = i % (H * B), yi = r / B, z = r - yi * B;
             const int y = yi < F - 1 ? yi : yi + I;
-            part[SA + i] = (float)((double)(long long)acc[(x * B + y) * B + z] * from_q);
+            part[SA + i] = (float)((double)(long long)acc[box_off<MAS, AXES>(x, y, z)] * from_q);
         }
         constexpr int SB = SA + I * H * B;
         for (int i = threadIdx.x; i < I * I * H; i += blockDim.x) {
             const int x = F - 1 + i / (I * H), r = i % (I * H), y = F - 1 + r / H, zi = r % H;
             const int z = zi < F - 1 ? zi : zi + I;
-            part[SB + i] = (float)((double)(long long)acc[(x * B + y) * B + z] * from_q);
+            part[SB + i] = (float)((double)(long long)acc[box_off<MAS, AXES>(x, y, z)] * from_q);
         }
         return;
     }
-    for (int c = threadIdx.x; c < NB; c += blockDim.x) {
+    for (int c = threadIdx.x; c < BX * BY * BZ; c += blockDim.x) {
         const int bz = c % BZ, by = (c / BZ) % BY, bx = c / (BZ * BY);
         if (!UNI && (bx >= ex + F - 1 || by >= ey + F - 1 || (AXES == 3 && bz >= ez + F - 1)))
             continue;
-        const float v = (float)((double)(long long)acc[c] * from_q);
+        const float v = (float)((double)(long long)acc[box_off<MAS, AXES>(bx, by, bz)] * from_q);
         const bool inner = bx >= F - 1 && bx < ex && by >= F - 1 && by < ey &&
                            (AXES == 2 || (bz >= F - 1 && bz < ez));
         if (inner) {
@@ -1725,13 +1883,64 @@ __device__ __forceinline__ void flush_box(const unsigned long long *acc, int key
     }
 }
 
+// Records each thread takes per round in the swizzled boxes' deposit (the next round's
+// records are loaded while this one's are deposited).
+template <int MAS>
+constexpr int rot_kr() { return MAS == PYL_PCS ? 2 : 4; }
+
+// This thread's records of a round: rot_kr blocks of up to kDepBlock records at set,
+// `left` of them in all; bit k of the result: dst[k] was loaded.  A block of fewer than
+// kDepBlock records (a sparse tile, or a tile's last) is spread over the waves, which
+// would otherwise leave it to the first of them.
+template <int MAS, bool RW>
+__device__ __forceinline__ unsigned rot_load(const float *set, unsigned long long left, int wv, int ln, float4 *dst) {
+    constexpr int RS = RW ? 4 : 3;
+    unsigned on = 0;
+#pragma unroll
+    for (int k = 0; k < rot_kr<MAS>(); ++k) {
+        const unsigned long long past = (unsigned long long)k * kDepBlock;
+        const unsigned n = left > past ? (unsigned)min(left - past, (unsigned long long)kDepBlock) : 0u;
+        const unsigned i = n == kDepBlock ? threadIdx.x : (unsigned)(ln * (kDepBlock / 64) + wv);
+        if (i < n) {
+            dst[k] = load_set_record<RW>(set + RS * past, i);
+            on |= 1u << k;
+        }
+    }
+    return on;
+}
+
+// Deposits the `left` records at set; rec, on: the first round, loaded by rot_load.
+template <int MAS, int AXES, bool WT, bool RW, bool UNI>
+__device__ __forceinline__ void rot_run(char *box, const float *set, unsigned long long left, float4 *rec, unsigned on,
+                                        int wv, int ln, const TileGeom &g, const TileBox &tb, float to_q,
+                                        float weight_factor) {
+    constexpr int RS = RW ? 4 : 3, KR = rot_kr<MAS>();
+    constexpr unsigned long long round = (unsigned long long)KR * kDepBlock;
+    while (left > 0) {
+        float4 cur[KR];
+        const unsigned con = on;
+#pragma unroll
+        for (int k = 0; k < KR; ++k) cur[k] = rec[k];
+        left -= min(left, round);
+        set += RS * round;
+        on = rot_load<MAS, RW>(set, left, wv, ln, rec);
+#pragma unroll
+        for (int k = 0; k < KR; ++k)
+            if ((con >> k) & 1u)
+                deposit_rot<MAS, AXES, WT, RW>(box, cur[k], box_coords<MAS, AXES, UNI>(cur[k], g, tb), ln, to_q,
+                                               weight_factor);
+    }
+}
+
 // One workgroup per tile.  LDS box of BX*BY*BZ 64-bit integers (the tile plus
 // the upper halo) holding multiples of 2^q; every record adds its whole
 // footprint at fixed offsets from its first node.  WT = false: unit weights
 // and weight_factor 1, so every contribution is >= 0 and the power-of-two
 // scale can be folded into the last axis' weights.
 //
-// Bank balancing (F >= 2): a footprint's F^AXES atomics all share the lanes'
+// CIC and PCS: one record per lane, deposit_rot's order in the swizzled box.
+//
+// Bank balancing (TSC): a footprint's atomics all share the lanes'
 // box offsets up to a constant, so their LDS bank conflicts are fixed by the
 // offsets mod 16.  Each wave takes KR*64 consecutive records, ranks them by
 // class (LDS counters), deals them to rounds as described at deal_slot, stages
@@ -1749,12 +1958,10 @@ tile_deposit_kernel(const float *__restrict__ records, unsigned long long rcap,
                     unsigned long long *__restrict__ gbox, CapRecs cr) {
     constexpr int F = MAS;
     constexpr int T = (AXES == 3) ? kT3 : kT2;
-    constexpr int BY = T + F - 1;
-    constexpr int BZ = (AXES == 3) ? T + F - 1 : 1;
-    constexpr int BX = T + F - 1;
-    constexpr int NB = BX * BY * BZ;
-    constexpr bool BAL = F >= 2;
-    constexpr int KR = BAL ? dep_kr<MAS, AXES>() : 1;
+    constexpr int NB = BoxDim<MAS, AXES>::words;
+    constexpr bool ROT = box_rot<MAS>();
+    constexpr bool BAL = F >= 2 && !ROT;
+    constexpr int KR = BAL ? kDepKR : 1;
     constexpr int NW = kDepBlock / 64;                 // waves
     constexpr int WB = KR * 64;                        // records per wave round set
     __shared__ unsigned long long acc[NB];
@@ -1829,7 +2036,18 @@ tile_deposit_kernel(const float *__restrict__ records, unsigned long long rcap,
     box_quantum<WT>(wmax_bits, real, weight_factor, nrec, to_q, from_q);
     __syncthreads();
 
-    if constexpr (!BAL) {
+    if constexpr (ROT) {
+        for (int seg = 0;; ++seg) {
+            const float *set = recs + (unsigned long long)RS * s0;
+            float4 first[rot_kr<MAS>()];
+            const unsigned on = rot_load<MAS, RW>(set, s1 - s0, wv, ln, first);
+            rot_run<MAS, AXES, WT, RW, UNI>((char *)acc, set, s1 - s0, first, on, wv, ln, g, tb, to_q, weight_factor);
+            if (seg > 0 || !two_seg) break;
+            recs = records;
+            s0 = r0;
+            s1 = r1;
+        }
+    } else if constexpr (!BAL) {
         for (int seg = 0;; ++seg) {
             // the next record is loaded while the current one is deposited
             unsigned long long r = s0 + threadIdx.x;
@@ -1972,7 +2190,7 @@ tile_box_flush_kernel(const unsigned long long *__restrict__ gbox, TileGeom g, f
                       const unsigned long long *__restrict__ offsets, float *__restrict__ grid,
                       float *__restrict__ partials, OutMode om) {
     constexpr int T = (AXES == 3) ? kT3 : kT2;
-    constexpr int NB = (T + MAS - 1) * (T + MAS - 1) * ((AXES == 3) ? T + MAS - 1 : 1);
+    constexpr int NB = BoxDim<MAS, AXES>::words;
     const int key = (int)blockIdx.x;
     const int real = key / (int)g.ntiles;
     const TileBox tb = tile_box<AXES>(key - real * (int)g.ntiles, g);
@@ -2721,8 +2939,7 @@ int run_tiled(Ctx *c, const float *pos, const RSD &rsd, long long n, const long 
     const size_t ch2_bytes = two ? ((size_t)nchunk2 * sizeof(Chunk) + 255) & ~(size_t)255 : 0;
     const size_t chs_bytes = capm ? ((size_t)kSpillChunks * sizeof(Chunk) + 255) & ~(size_t)255 : 0;
     const size_t bdump_bytes = two ? ((size_t)std::max(nchunk, 1) * nbk * sizeof(unsigned) + 255) & ~(size_t)255 : 0;
-    const int T = axes == 3 ? kT3 : kT2;
-    const size_t nbox = (size_t)(T + MAS - 1) * (T + MAS - 1) * (axes == 3 ? T + MAS - 1 : 1);
+    const size_t nbox = axes == 3 ? BoxDim<MAS, 3>::words : BoxDim<MAS, 2>::words;
     // all scratch of the call is taken before the first launch
     void *tbv = nullptr, *pv = nullptr, *rv = nullptr, *bv = nullptr, *kv = nullptr;
     PYL_TRY(take(c, BUF_TILE_CNT, cnt_bytes + off_bytes + bs_bytes + ch_bytes + org_bytes +
