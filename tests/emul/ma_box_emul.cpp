@@ -5,6 +5,7 @@
 //   - the 16 lanes of a pass are in 16 different bank pairs at every step (PCS), or in
 //     the 8 (2D: 4) residues of the coordinates' parities two (four) lanes each (CIC),
 //     whatever the lanes' first nodes;
+//   - the tile of a node, taken by a multiplication, is the exact quotient;
 //   - the PCS weights match the cubic B-spline in long double to float rounding.
 // Built and run by tests/test_ma_box_emul.py (host compile only, no GPU calls).
 #include "../../pylians3_amd/csrc/ma.hip"
@@ -118,10 +119,27 @@ static int check_pcs_weights() {
     return bad;
 }
 
+// node_tile is floor(node * nt / dims) for every node of every grid size.
+static int check_node_tile() {
+    int bad = 0;
+    auto one = [&](int dims, int axes, int step) {
+        const TileGeom g = make_geom(dims, axes, PYL_TSC);
+        if (g.nt == 1) return;                             // (home_tile shifts instead)
+        for (int n = 0; n < dims; n += step)
+            if (node_tile(n, g) != (int)((long long)n * g.nt / dims)) ++bad;
+        if (node_tile(dims - 1, g) != g.nt - 1) ++bad;
+    };
+    for (int d = 17; d <= 2600; ++d) one(d, 3, 1);
+    for (int d = 65; d <= 9000; d += 7) one(d, 2, 1);
+    for (int d : {65521, 65535, 65536, 65537, 131071}) one(d, 2, 1);
+    printf("node tile: %s\n", bad ? "FAIL" : "ok");
+    return bad;
+}
+
 int main() {
     int bad = check_steps<PYL_CIC, 3>() + check_steps<PYL_CIC, 2>() + check_steps<PYL_PCS, 3>() + check_steps<PYL_PCS, 2>();
     bad += check_box<PYL_NGP, 3>() + check_box<PYL_NGP, 2>() + check_box<PYL_TSC, 3>() + check_box<PYL_TSC, 2>();
-    bad += check_pcs_weights();
+    bad += check_pcs_weights() + check_node_tile();
     printf(bad ? "FAILURES: %d\n" : "all ok\n", bad);
     return bad != 0;
 }
