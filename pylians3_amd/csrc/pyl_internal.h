@@ -155,6 +155,7 @@ struct Ctx {
                                                         // were out of order (two-level sort next)
     long long cap_spill_n = -1;      // particles of the capacity call whose spill h_total[3] will hold
     std::pair<int, int> cap_key{0, 0};                // its (dims, MAS)
+    bool cap_two = false;                             // it was the two-level sort's second pass
     std::map<std::pair<int, int>, int> cap_bad;       // per (dims, MAS): calls left without the
                                                       // capacity form after one spilled too much
     int last_window = -1;            // sort window of the latest tiled MA (PYL_WINDOW_*)
