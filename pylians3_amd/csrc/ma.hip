@@ -1829,6 +1829,130 @@ __device__ __forceinline__ void box_quantum(const unsigned *__restrict__ wmax_bi
     from_q = ldexp(1.0, q);
 }
 
+// Records a wave takes per round set of a run of n records: kDepKR per lane, fewer when
+// the run is shorter than a full round of every wave (a sparse tile, whose records the
+// first wave or two would otherwise keep to themselves).
+__device__ __forceinline__ unsigned deal_set(unsigned long long n) {
+    constexpr unsigned NW = kDepBlock / 64, WB = kDepKR * 64;
+    if (n >= (unsigned long long)NW * WB) return WB;
+    return max(64u, (((unsigned)n + NW - 1) / NW + 63u) & ~63u);
+}
+
+// Records b .. b+255 of a run that ends at s1, clamped to its last record, through a
+// wave-uniform pointer and 32-bit lane offsets.
+template <bool RW>
+__device__ __forceinline__ void deal_load(const float *recs, unsigned long long s1, unsigned long long b, int ln,
+                                          float4 *dst) {
+    const unsigned long long sb = min(b, s1 - 1);
+    const float *set = recs + (unsigned long long)(RW ? 4 : 3) * sb;
+    const unsigned lim = (unsigned)min(s1 - 1 - sb, (unsigned long long)(kDepKR * 64));
+#pragma unroll
+    for (int k = 0; k < kDepKR; ++k) dst[k] = load_set_record<RW>(set, min((unsigned)(ln + 64 * k), lim));
+}
+
+// Deposits the records s0 .. s1 (not empty) of recs with the dealing described above;
+// nxt holds the wave's first set (deal_load).  si, ht, wh: the wave's own LDS scratch.
+template <int MAS, int AXES, bool WT, bool RW, bool UNI>
+__device__ __forceinline__ void deal_run(unsigned long long *acc, unsigned short *si, unsigned char *ht, unsigned *wh,
+                                         const float *recs, unsigned long long s0, unsigned long long s1, float4 *nxt,
+                                         int wv, int ln, const TileGeom &g, const TileBox &tb, float to_q,
+                                         float weight_factor) {
+    constexpr int KR = kDepKR, RS = RW ? 4 : 3;
+    constexpr unsigned G = 4 * KR;                     // layers of 16 lanes
+    constexpr int NW = kDepBlock / 64;
+    // wave wv takes the round sets starting at s0 + (wv + NW*j)*wb; the next
+    // set's records are loaded (clamped into the run) while this one runs
+    const unsigned wb = deal_set(s1 - s0);
+    const unsigned long long step = (unsigned long long)NW * wb;
+    for (unsigned long long b0 = s0 + (unsigned long long)wv * wb; b0 < s1; b0 += step) {
+        float4 rec[KR];
+#pragma unroll
+        for (int k = 0; k < KR; ++k) rec[k] = nxt[k];
+        const int nb = (int)min((unsigned long long)wb, s1 - b0);   // records in this set
+        // rank within class (LDS ops of one wave run in issue order)
+        if (ln < 16) wh[ln] = 0u;
+        __builtin_amdgcn_wave_barrier();
+        unsigned cls[KR], rank[KR];
+#pragma unroll
+        for (int k = 0; k < KR; ++k) {
+            cls[k] = bank_class<MAS, AXES>(rec[k]);
+            rank[k] = (ln + 64 * k < nb) ? atomicAdd(&wh[cls[k]], 1u) : 0u;
+        }
+        __builtin_amdgcn_wave_barrier();
+        // lanes 0..15 hold class j = ln: c_j records, G - c_j holes or c_j - G
+        // excess copies.  Exclusive prefixes of both (excess in the high half)
+        // by an inclusive DPP scan over row 0 (row_shr 1, 2, 4, 8).
+        const unsigned cj = (ln < 16) ? wh[ln] : 0u;
+        const unsigned v = (ln < 16) ? ((cj > G ? cj - G : 0u) << 16) | (cj < G ? G - cj : 0u) : 0u;
+        unsigned incl = v;
+        incl += (unsigned)__builtin_amdgcn_update_dpp(0, (int)incl, 0x111, 0xf, 0xf, false);
+        incl += (unsigned)__builtin_amdgcn_update_dpp(0, (int)incl, 0x112, 0xf, 0xf, false);
+        incl += (unsigned)__builtin_amdgcn_update_dpp(0, (int)incl, 0x114, 0xf, 0xf, false);
+        incl += (unsigned)__builtin_amdgcn_update_dpp(0, (int)incl, 0x118, 0xf, 0xf, false);
+        const unsigned excl = incl - v;
+        const unsigned E = (unsigned)__builtin_amdgcn_readlane((int)incl, 15) >> 16;
+        __builtin_amdgcn_wave_barrier();
+        // class j's count, first hole and first excess index (9 bits each)
+        if (ln < 16) wh[ln] = cj | (excl & 0xffffu) << 9 | (excl >> 16) << 18;
+        __builtin_amdgcn_wave_barrier();
+        {
+            // the G*16 (layer, lane) slots, KR per lane: lane ln takes class ln % 16
+            const unsigned cw = wh[ln & 15];
+#pragma unroll
+            for (int k = 0; k < KR; ++k)
+                deal_hole<KR>((unsigned)(ln >> 4) + 4u * k, (unsigned)(ln & 15), cw & 511u,
+                              (cw >> 9) & 511u, E, ht, si);
+        }
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (int k = 0; k < KR; ++k) {
+            if (ln + 64 * k < nb) {
+                const unsigned X = rank[k] < G ? 0u : wh[cls[k]] >> 18;
+                si[deal_record_slot<KR>(cls[k], rank[k], X, ht)] = (unsigned short)(ln + 64 * k);
+            }
+        }
+        __builtin_amdgcn_wave_barrier();
+        // the dealt records of all rounds are reloaded (from cache) before the
+        // first atomic, and the next set is loaded only after them: loads
+        // complete in issue order, so the atomics wait for the reloads alone
+        // and the next set's memory latency overlaps this set's atomics.  The
+        // next-set loads are issued unconditionally (past the tile's end they
+        // all read its last record) so that the number of loads in flight is
+        // the same on every path and the waits before the atomics stay exact.
+        unsigned short di[KR];
+        float4 dealt[KR];
+#pragma unroll
+        for (int r = 0; r < KR; ++r) di[r] = si[r * 64 + ln];
+        const float *set = recs + (unsigned long long)RS * b0;
+#pragma unroll
+        for (int r = 0; r < KR; ++r)
+            dealt[r] = load_set_record<RW>(set, di[r] != kNoRecord ? di[r] : 0u);
+        __builtin_amdgcn_sched_barrier(0);         // keep the reloads ahead of the next set
+        deal_load<RW>(recs, s1, b0 + step, ln, nxt);
+        __builtin_amdgcn_sched_barrier(0);
+        // every reloaded record is consumed here, on all lanes: the reloads
+        // are not sunk into the per-round branches below (where they would be
+        // issued after the next set's loads), and one wait covers them
+#pragma unroll
+        for (int r = 0; r < KR; ++r) {
+            if constexpr (RW)
+                asm volatile("" ::"v"(dealt[r].x), "v"(dealt[r].y), "v"(dealt[r].z), "v"(dealt[r].w));
+            else
+                asm volatile("" ::"v"(dealt[r].x), "v"(dealt[r].y), "v"(dealt[r].z));
+        }
+#pragma unroll
+        for (int r = 0; r < KR; ++r) {
+            if (di[r] != kNoRecord) {
+                int bb;
+                if constexpr (UNI && AXES == 3) bb = box_base_uni<MAS>(dealt[r]);
+                else bb = box_base<MAS, AXES>(dealt[r], g, tb);
+                deposit_record<MAS, AXES, WT, RW>(acc + bb, dealt[r], to_q, weight_factor);
+            }
+        }
+        __builtin_amdgcn_wave_barrier();
+    }
+}
+
 // Writes a tile's box of integer sums (LDS or global): the nodes no other tile
 // touches go to the grid (grid already offset to the realisation), the band and
 // halo to the tile's partial slots (halo_index order).
@@ -1898,7 +2022,7 @@ __device__ __forceinline__ void flush_box(const unsigned long long *acc, int key
 // Records each thread takes per round in the swizzled boxes' deposit (the next round's
 // records are loaded while this one's are deposited).
 template <int MAS>
-constexpr int rot_kr() { return MAS == PYL_PCS ? 2 : 4; }
+constexpr int rot_kr() { return 2; }
 
 // This thread's records of a round: rot_kr blocks of up to kDepBlock records at set,
 // `left` of them in all; bit k of the result: dst[k] was loaded.  A block of fewer than
@@ -2027,17 +2151,8 @@ tile_deposit_kernel(const float *__restrict__ records, unsigned long long rcap,
     // the first round set of every wave is loaded before the box is cleared
     const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), ln = threadIdx.x & 63;
     constexpr int RS = RW ? 4 : 3;                     // floats per record
-    // records b .. b+WB-1 of a set, clamped to the tile's last record, through a
-    // wave-uniform pointer and 32-bit lane offsets
-    auto load_set = [&](unsigned long long b, float4 *dst) {
-        const unsigned long long sb = min(b, s1 - 1);
-        const float *set = recs + (unsigned long long)RS * sb;
-        const unsigned lim = (unsigned)min(s1 - 1 - sb, (unsigned long long)WB);
-#pragma unroll
-        for (int k = 0; k < KR; ++k) dst[k] = load_set_record<RW>(set, min((unsigned)(ln + 64 * k), lim));
-    };
     float4 nxt[KR];
-    if constexpr (BAL) load_set(s0 + (unsigned long long)wv * WB, nxt);
+    if constexpr (BAL) deal_load<RW>(recs, s1, s0 + (unsigned long long)wv * deal_set(s1 - s0), ln, nxt);
     for (int c = threadIdx.x; c < NB; c += blockDim.x) acc[c] = 0ull;
 
     float to_q;
@@ -2080,104 +2195,14 @@ tile_deposit_kernel(const float *__restrict__ records, unsigned long long rcap,
         unsigned *wh = whist + wv * 16;
         unsigned short *si = sidx + wv * WB;
         unsigned char *ht = htab + wv * WB;
-        constexpr unsigned G = 4 * KR;                 // layers of 16 lanes
-        // wave wv takes the round sets starting at s0 + (wv + NW*j)*WB; the next
-        // set's records are loaded (clamped into the segment) while this one runs
         for (int seg = 0;; ++seg) {
-            unsigned long long b0 = s0 + (unsigned long long)wv * WB;
-            for (; b0 < s1; b0 += (unsigned long long)NW * WB) {
-                float4 rec[KR];
-#pragma unroll
-                for (int k = 0; k < KR; ++k) rec[k] = nxt[k];
-                const int nb = (int)min((unsigned long long)WB, s1 - b0);   // records in this set
-                // rank within class (LDS ops of one wave run in issue order)
-                if (ln < 16) wh[ln] = 0u;
-                __builtin_amdgcn_wave_barrier();
-                unsigned cls[KR], rank[KR];
-#pragma unroll
-                for (int k = 0; k < KR; ++k) {
-                    cls[k] = bank_class<MAS, AXES>(rec[k]);
-                    rank[k] = (ln + 64 * k < nb) ? atomicAdd(&wh[cls[k]], 1u) : 0u;
-                }
-                __builtin_amdgcn_wave_barrier();
-                // lanes 0..15 hold class j = ln: c_j records, G - c_j holes or c_j - G
-                // excess copies.  Exclusive prefixes of both (excess in the high half)
-                // by an inclusive DPP scan over row 0 (row_shr 1, 2, 4, 8).
-                const unsigned cj = (ln < 16) ? wh[ln] : 0u;
-                const unsigned v = (ln < 16) ? ((cj > G ? cj - G : 0u) << 16) | (cj < G ? G - cj : 0u) : 0u;
-                unsigned incl = v;
-                incl += (unsigned)__builtin_amdgcn_update_dpp(0, (int)incl, 0x111, 0xf, 0xf, false);
-                incl += (unsigned)__builtin_amdgcn_update_dpp(0, (int)incl, 0x112, 0xf, 0xf, false);
-                incl += (unsigned)__builtin_amdgcn_update_dpp(0, (int)incl, 0x114, 0xf, 0xf, false);
-                incl += (unsigned)__builtin_amdgcn_update_dpp(0, (int)incl, 0x118, 0xf, 0xf, false);
-                const unsigned excl = incl - v;
-                const unsigned E = (unsigned)__builtin_amdgcn_readlane((int)incl, 15) >> 16;
-                __builtin_amdgcn_wave_barrier();
-                // class j's count, first hole and first excess index (9 bits each)
-                if (ln < 16) wh[ln] = cj | (excl & 0xffffu) << 9 | (excl >> 16) << 18;
-                __builtin_amdgcn_wave_barrier();
-                {
-                    // the G*16 (layer, lane) slots, KR per lane: lane ln takes class ln % 16
-                    const unsigned cw = wh[ln & 15];
-#pragma unroll
-                    for (int k = 0; k < KR; ++k)
-                        deal_hole<KR>((unsigned)(ln >> 4) + 4u * k, (unsigned)(ln & 15), cw & 511u,
-                                      (cw >> 9) & 511u, E, ht, si);
-                }
-                __builtin_amdgcn_wave_barrier();
-#pragma unroll
-                for (int k = 0; k < KR; ++k) {
-                    if (ln + 64 * k < nb) {
-                        const unsigned X = rank[k] < G ? 0u : wh[cls[k]] >> 18;
-                        si[deal_record_slot<KR>(cls[k], rank[k], X, ht)] = (unsigned short)(ln + 64 * k);
-                    }
-                }
-                __builtin_amdgcn_wave_barrier();
-                // the dealt records of all rounds are reloaded (from cache) before the
-                // first atomic, and the next set is loaded only after them: loads
-                // complete in issue order, so the atomics wait for the reloads alone
-                // and the next set's memory latency overlaps this set's atomics.  The
-                // next-set loads are issued unconditionally (past the tile's end they
-                // all read its last record) so that the number of loads in flight is
-                // the same on every path and the waits before the atomics stay exact.
-                unsigned short di[KR];
-                float4 dealt[KR];
-#pragma unroll
-                for (int r = 0; r < KR; ++r) di[r] = si[r * 64 + ln];
-                const float *set = recs + (unsigned long long)RS * b0;
-#pragma unroll
-                for (int r = 0; r < KR; ++r)
-                    dealt[r] = load_set_record<RW>(set, di[r] != kNoRecord ? di[r] : 0u);
-                __builtin_amdgcn_sched_barrier(0);         // keep the reloads ahead of the next set
-                load_set(b0 + (unsigned long long)NW * WB, nxt);
-                __builtin_amdgcn_sched_barrier(0);
-                // every reloaded record is consumed here, on all lanes: the reloads
-                // are not sunk into the per-round branches below (where they would be
-                // issued after the next set's loads), and one wait covers them
-#pragma unroll
-                for (int r = 0; r < KR; ++r) {
-                    if constexpr (RW)
-                        asm volatile("" ::"v"(dealt[r].x), "v"(dealt[r].y), "v"(dealt[r].z), "v"(dealt[r].w));
-                    else
-                        asm volatile("" ::"v"(dealt[r].x), "v"(dealt[r].y), "v"(dealt[r].z));
-                }
-#pragma unroll
-                for (int r = 0; r < KR; ++r) {
-                    if (di[r] != kNoRecord) {
-                        int bb;
-                        if constexpr (UNI && AXES == 3) bb = box_base_uni<MAS>(dealt[r]);
-                        else bb = box_base<MAS, AXES>(dealt[r], g, tb);
-                        deposit_record<MAS, AXES, WT, RW>(acc + bb, dealt[r], to_q, weight_factor);
-                    }
-                }
-                __builtin_amdgcn_wave_barrier();
-            }
+            deal_run<MAS, AXES, WT, RW, UNI>(acc, si, ht, wh, recs, s0, s1, nxt, wv, ln, g, tb, to_q, weight_factor);
             if (seg > 0 || !two_seg) break;
             // the tile's sorted records: the first set is loaded before the loop, as above
             recs = records;
             s0 = r0;
             s1 = r1;
-            load_set(s0 + (unsigned long long)wv * WB, nxt);
+            deal_load<RW>(recs, s1, s0 + (unsigned long long)wv * deal_set(s1 - s0), ln, nxt);
         }
     }
     __syncthreads();
@@ -2222,7 +2247,13 @@ tile_box_flush_kernel(const unsigned long long *__restrict__ gbox, TileGeom g, f
 // it (every tile's sums are its own integers).
 constexpr int kOrderBlock = 1024;
 constexpr int kOrderBuckets = 512;
-constexpr long long kOrderMinKeys = 4096;
+// Column deposit: tiles per segment, as many as leave kColMinSegs segments.
+// (134 M particles, TSC on 512^3, deposit + finalize: 1.39 ms with one tile per segment,
+// 1.31, 1.29 and 1.28 ms with 4, 8 and 16.)
+constexpr int kColMaxLen = 16;
+constexpr long long kColMinSegs = 2048;
+constexpr long long kColPcsDense = 2048;         // mean records per tile
+constexpr long long kOrderMinKeys = 2048;
 constexpr long long kOrderMinRecords = 512;      // mean records per key
 // Split deposit: below kSplitMaxKeys tiles, a tile holding more than
 // kSplitRecords records per workgroup on average is shared by up to kSplitMax
@@ -2249,10 +2280,21 @@ __host__ __device__ __forceinline__ int count_bucket(unsigned long long n) {
     return min(kOrderBuckets - 1, 1 + 16 * lg + q);
 }
 
-// Records of key k: its run of the sorted records plus its capacity slots.
+// What the deposit's workgroups take: runs of up to len consecutive keys of columns of
+// per keys, segs runs per column (one key each: {1, 1, 1}).
+struct OrderSeg {
+    int len, per, segs;
+};
+
+// Records of run k: the runs of the sorted records plus the capacity slots.
 __device__ __forceinline__ unsigned long long key_records(const unsigned long long *__restrict__ offsets,
-                                                          long long k, const CapRecs &cr) {
-    return offsets[k + 1] - offsets[k] + cap_count(cr, k);
+                                                          long long k, const OrderSeg &os, const CapRecs &cr) {
+    const long long c = k / os.segs;
+    const long long k0 = c * os.per + (k - c * os.segs) * os.len, k1 = min(k0 + os.len, (c + 1) * os.per);
+    unsigned long long n = offsets[k1] - offsets[k0];
+#pragma unroll 8
+    for (long long j = k0; j < k1; ++j) n += cap_count(cr, j);
+    return n;
 }
 
 // The order is built in two launches of order_wgs(nt) workgroups, each thread
@@ -2268,7 +2310,7 @@ inline int order_wgs(long long nt) {
 }
 
 __global__ void __launch_bounds__(kOrderBlock)
-order_hist_kernel(const unsigned long long *__restrict__ offsets, long long nt, CapRecs cr,
+order_hist_kernel(const unsigned long long *__restrict__ offsets, long long nt, OrderSeg os, CapRecs cr,
                   unsigned *__restrict__ ghist) {
     __shared__ unsigned hist[kOrderBuckets];
     for (int b = threadIdx.x; b < kOrderBuckets; b += blockDim.x) hist[b] = 0u;
@@ -2279,7 +2321,7 @@ order_hist_kernel(const unsigned long long *__restrict__ offsets, long long nt, 
 #pragma unroll
     for (int j = 0; j < kOrderPer; ++j) {        // all loads before the first atomic
         const long long k = k0 + j * step;
-        c[j] = k < nt ? key_records(offsets, k, cr) : 0ull;
+        c[j] = k < nt ? key_records(offsets, k, os, cr) : 0ull;
     }
 #pragma unroll
     for (int j = 0; j < kOrderPer; ++j)
@@ -2290,7 +2332,7 @@ order_hist_kernel(const unsigned long long *__restrict__ offsets, long long nt, 
 }
 
 __global__ void __launch_bounds__(kOrderBlock)
-order_place_kernel(const unsigned long long *__restrict__ offsets, long long nt, CapRecs cr,
+order_place_kernel(const unsigned long long *__restrict__ offsets, long long nt, OrderSeg os, CapRecs cr,
                    const unsigned *__restrict__ ghist, unsigned *__restrict__ gcur,
                    unsigned *__restrict__ order) {
     __shared__ unsigned start[kOrderBuckets];   // first slot of each bucket, largest first
@@ -2319,7 +2361,7 @@ order_place_kernel(const unsigned long long *__restrict__ offsets, long long nt,
 #pragma unroll
     for (int j = 0; j < kOrderPer; ++j) {
         const long long k = k0 + j * step;
-        bk[j] = k < nt ? count_bucket(key_records(offsets, k, cr)) : 0;
+        bk[j] = k < nt ? count_bucket(key_records(offsets, k, os, cr)) : 0;
     }
 #pragma unroll
     for (int j = 0; j < kOrderPer; ++j)
@@ -2550,6 +2592,410 @@ tile_finalize_uniform_kernel(const unsigned long long *__restrict__ offsets, Til
             if (on) v += (double)x[i];
         }
         store_node(grid, (long long)(node0 + (unsigned)lx * dd + (unsigned)(ly * g.dims + lz)), (float)v, om);
+    }
+}
+
+// ---- column deposit: 3D grids of two tiles or more per axis (CIC, TSC, PCS) ------
+// A workgroup takes a segment of ColSeg::len tiles that follow one another along z and
+// keeps the LDS box from tile to tile: the upper halo planes of a tile become, as
+// floats in registers (the carry), a second contribution to the first F-1 planes of the
+// next.  Compared with one workgroup per tile
+//  * the nodes a tile shares only with its z neighbours are final when their tile is
+//    flushed and are written once, in whole 64-byte rows of the grid; only the ring
+//    (nodes that x or y neighbours share) goes through partial values, in rows of a
+//    tile's z extent, and the finalize reads and writes such rows too;
+//  * a tile's first records are loaded while the previous tile is flushed, and the nodes
+//    of an accumulated grid while its last atomics run.
+// The value of a node is the float64 sum of the same float32 tile values in the same
+// order as in the tile form (own, then the lower z neighbour, per x and y image), rounded
+// once: the bits do not depend on the form or on the segment length.
+// Deposit and finalize together, tile form and column form: 134 M particles, TSC on 512^3
+// 1.34 and 1.26 ms, on 500^3 1.80 and 1.43; 2 M weighted, PCS on 512^3 1.23 and 0.94;
+// 67 M in 32 CIC grids of 128^3 0.47 and 0.40.
+//
+// Partial values of a tile (F-1 = L, extents e, zs = the largest extent; ring columns
+// by ring_col, interior columns by (x - L) * (ey - L) + y - L):
+//   ring  [rc * zs + z]       own sums, z < ez
+//   carry [rc * L + z]        the lower z neighbour's, z < L
+//   low   [ic * L + z]        own interior sums of a segment's first tile, z < L
+//   clow  [ic * L + z]        and what the segment before it carries over
+struct ColSeg {
+    int len;     // tiles per segment
+    int nz;      // segments per column of tiles
+    int zs;      // largest tile extent
+};
+
+template <int F>
+__host__ __device__ __forceinline__ int col_carry_at(int zs) { return 4 * (F - 1) * zs * zs; }
+template <int F>
+__host__ __device__ __forceinline__ int col_low_at(int zs) { return 4 * (F - 1) * zs * (zs + F - 1); }
+template <int F>
+__host__ __device__ __forceinline__ int col_clow_at(int zs) {
+    return col_low_at<F>(zs) + (zs - F + 1) * (zs - F + 1) * (F - 1);
+}
+
+// v / d and v % d for 0 <= v < 2048 and 1 <= d <= 19 (a tile's box).
+__host__ __device__ __forceinline__ void small_div(int v, int d, int &q, int &r) {
+    q = (int)(((unsigned)v * (65536u / (unsigned)d + 1u)) >> 16);
+    r = v - q * d;
+}
+
+// Ring columns of a tile: box columns outside its interior [L, ex) x [L, ey).
+template <int F>
+__host__ __device__ __forceinline__ int ring_count(int ex, int ey) { return 2 * (F - 1) * (ex + ey); }
+template <int F>
+__host__ __device__ __forceinline__ bool in_ring(int x, int y, int ex, int ey) {
+    return x < F - 1 || x >= ex || y < F - 1 || y >= ey;
+}
+template <int F>
+__host__ __device__ __forceinline__ int ring_col(int x, int y, int ex, int ey) {
+    constexpr int L = F - 1;
+    const int by = ey + L;
+    if (x < L || x >= ex) return (x < L ? x : x - ex + L) * by + y;
+    return 2 * L * by + (x - L) * (2 * L) + (y < L ? y : y - ey + L);
+}
+template <int F>
+__host__ __device__ __forceinline__ void ring_xy(int rc, int ex, int ey, int &x, int &y) {
+    constexpr int L = F - 1, L2 = L > 0 ? 2 * L : 1;
+    const int by = ey + L;
+    if (rc < 2 * L * by) {
+        small_div(rc, by, x, y);
+        x = x < L ? x : x - L + ex;
+    } else {
+        const int q = rc - 2 * L * by;
+        x = L + q / L2;
+        y = q % L2;
+        y = y < L ? y : y - L + ey;
+    }
+}
+
+// Output transform, the grid's old value given.
+__device__ __forceinline__ float out_value(float v, float old, const OutMode &om) {
+    if (!om.overwrite) return old + v;
+    return (om.scale == 1.0f ? v : v / om.scale) - om.shift;
+}
+
+// Waves per SIMD that the LDS boxes allow (two or three workgroups per CU).
+template <int MAS>
+constexpr int col_waves() { return MAS == PYL_PCS ? 4 : 6; }
+
+template <int MAS, bool WT, bool RW, bool UNI>
+__global__ void __launch_bounds__(kDepBlock, col_waves<MAS>())
+column_deposit_kernel(const float *__restrict__ records, unsigned long long rcap,
+                      const unsigned long long *__restrict__ offsets, TileGeom g, float weight_factor,
+                      const unsigned *__restrict__ wmax_bits, float *__restrict__ grid,
+                      float *__restrict__ partials, OutMode om, const unsigned *__restrict__ order, ColSeg cs,
+                      CapRecs cr) {
+    constexpr int F = MAS, L = F - 1, T = kT3, B = T + L, NT = kDepBlock;
+    constexpr bool ROT = box_rot<MAS>();
+    constexpr int NB = BoxDim<MAS, 3>::words;
+    constexpr int KR = ROT ? rot_kr<MAS>() : kDepKR;
+    constexpr int NW = NT / 64, WB = KR * 64, RS = RW ? 4 : 3;
+    constexpr int KC = (B * B * L + NT - 1) / NT;      // low (and carry) plane cells per thread
+    constexpr int ZW = UNI ? T - L : 16;               // lanes per row of the middle planes
+    constexpr int KI = ((T - L) * (T - L) * ZW + NT - 1) / NT;   // interior middle cells per thread
+    __shared__ unsigned long long acc[NB];
+    __shared__ unsigned short sidx[ROT ? 1 : NW * WB];
+    __shared__ unsigned char htab[ROT ? 1 : NW * WB];
+    __shared__ unsigned whist[ROT ? 1 : NW * 16];
+    const int t = threadIdx.x;
+    const int wv = __builtin_amdgcn_readfirstlane(t >> 6), ln = t & 63;
+    const int sid = __builtin_amdgcn_readfirstlane(order ? (int)order[blockIdx.x] : (int)blockIdx.x);
+    const int col = sid / cs.nz, tz0 = (sid - col * cs.nz) * cs.len, tz1 = min(g.nt, tz0 + cs.len);
+    const int real = col / (g.nt * g.nt);
+    TileBox tb;
+    tb.tx = col / g.nt - real * g.nt;
+    tb.ty = col % g.nt;
+    tb.ox = UNI ? tb.tx * T : g.orig[tb.tx];
+    tb.oy = UNI ? tb.ty * T : g.orig[tb.ty];
+    tb.ex = UNI ? T : g.orig[tb.tx + 1] - tb.ox;
+    tb.ey = UNI ? T : g.orig[tb.ty + 1] - tb.oy;
+    const int ex = UNI ? T : tb.ex, ey = UNI ? T : tb.ey, zs = UNI ? T : cs.zs;
+    const int Ix = ex - L, Iy = ey - L;
+    const unsigned dd = (unsigned)g.dims;
+    grid += real * g.ncell + ((long long)tb.ox * g.dims + tb.oy) * g.dims;
+
+    // record runs of a tile: its capacity slots, then its sorted records
+    struct Runs { unsigned long long c0, c1, r0, r1; };
+    auto runs_of = [&](int tz) {
+        const long long key = (long long)col * g.nt + tz;
+        Runs r;
+        r.r1 = min(offsets[key + 1], rcap);
+        r.r0 = min(offsets[key], r.r1);
+        r.c0 = r.c1 = 0;
+        if (cr.rec) {
+            r.c0 = (unsigned long long)key * cr.cap;
+            r.c1 = r.c0 + min(cr.count[key], cr.cap);
+        }
+        return r;
+    };
+    float4 nxt[KR];
+    unsigned on = 0;
+    auto load_run = [&](const float *recs, unsigned long long s0, unsigned long long s1) {
+        if constexpr (ROT) on = rot_load<MAS, RW>(recs + (unsigned long long)RS * s0, s1 - s0, wv, ln, nxt);
+        else deal_load<RW>(recs, s1, s0 + (unsigned long long)wv * deal_set(s1 - s0), ln, nxt);
+    };
+    auto load_first = [&](const Runs &r) {
+        if (r.c1 > r.c0) load_run(cr.rec, r.c0, r.c1);
+        else if (r.r1 > r.r0) load_run(records, r.r0, r.r1);
+    };
+    float to_q;
+    double from_q;
+    auto deposit = [&](const float *recs, unsigned long long s0, unsigned long long s1) {
+        if constexpr (ROT)
+            rot_run<MAS, 3, WT, RW, UNI>((char *)acc, recs + (unsigned long long)RS * s0, s1 - s0, nxt, on, wv, ln, g,
+                                         tb, to_q, weight_factor);
+        else
+            deal_run<MAS, 3, WT, RW, UNI>(acc, sidx + wv * WB, htab + wv * WB, whist + wv * 16, recs, s0, s1, nxt, wv,
+                                          ln, g, tb, to_q, weight_factor);
+    };
+
+    Runs run = runs_of(tz0);
+    load_first(run);
+    for (int c = t; c < NB; c += NT) acc[c] = 0ull;
+    // the realisation's record count, so that a batch and single calls agree bitwise
+    const unsigned long long nrec = cr.nrec >= 0 ? (unsigned long long)cr.nrec
+        : offsets[(long long)(real + 1) * g.ntiles] - offsets[(long long)real * g.ntiles];
+    box_quantum<WT>(wmax_bits, real, weight_factor, nrec, to_q, from_q);
+    __syncthreads();
+
+    float carry[KC];
+#pragma unroll
+    for (int k = 0; k < KC; ++k) carry[k] = 0.0f;
+    bool prev = false;                                  // the tile below in this segment had records
+    auto value = [&](int at) {                          // a box sum, cleared for the next tile
+        const long long v = (long long)acc[at];
+        acc[at] = 0ull;
+        return (float)((double)v * from_q);
+    };
+    for (int tz = tz0; tz < tz1; ++tz) {
+        const bool first = tz == tz0;
+        tb.tz = tz;
+        tb.oz = UNI ? tz * T : g.orig[tz];
+        tb.ez = UNI ? T : g.orig[tz + 1] - tb.oz;
+        const int ez = UNI ? T : tb.ez;
+        float *part = partials + ((long long)col * g.nt + tz) * g.pslot;
+        const bool some = run.c1 > run.c0 || run.r1 > run.r0;
+        if (run.c1 > run.c0) {
+            deposit(cr.rec, run.c0, run.c1);
+            if (run.r1 > run.r0) load_run(records, run.r0, run.r1);
+        }
+        if (run.r1 > run.r0) deposit(records, run.r0, run.r1);
+        if (tz + 1 < tz1) {
+            run = runs_of(tz + 1);
+            load_first(run);
+        }
+        if (!some && !prev && !om.overwrite) continue;  // nothing to write, nothing carried
+        // the flush's cell numbers are the same for every tile of the segment; worked out
+        // anew for each (from a thread number the compiler cannot see through), since
+        // kept over the deposit their 50 registers cost the third workgroup per CU
+        int tf = t;
+        asm volatile("" : "+v"(tf));
+        // this thread's interior nodes: the middle planes [L, ez), in rows; an accumulated
+        // grid is read while the last atomics of the tile run
+        auto middle = [&](int k, int &x, int &y, int &z) {
+            const int i = tf + k * NT, row = i / ZW;
+            z = L + i - row * ZW;
+            if constexpr (UNI) {
+                x = row / (T - L);
+                y = row - x * (T - L);
+            } else {
+                small_div(row, Iy, x, y);
+            }
+            const bool in = x < Ix && z < ez;
+            x += L;
+            y += L;
+            return in;
+        };
+        auto node = [&](int x, int y, int z) {
+            return grid + ((long long)((unsigned)x * dd + (unsigned)y) * dd + (unsigned)(tb.oz + z));
+        };
+        float old[KI];
+        if (!om.overwrite && some) {
+#pragma unroll
+            for (int k = 0; k < KI; ++k) {
+                int x, y, z;
+                if (middle(k, x, y, z)) old[k] = *node(x, y, z);
+            }
+        }
+        __syncthreads();
+        // low planes [0, L) with what the tile below carries up, and the new carry from
+        // the planes above the tile
+#pragma unroll
+        for (int k = 0; k < KC; ++k) {
+            const int i = tf + k * NT, xy = i / L, z = i - xy * L, x = xy / B, y = xy - x * B;
+            if (x < ex + L && y < ey + L) {
+                const float own = some ? value(box_off<MAS, 3>(x, y, z)) : 0.0f;
+                const float up = some ? value(box_off<MAS, 3>(x, y, ez + z)) : 0.0f;
+                if (in_ring<F>(x, y, ex, ey)) {
+                    const int rc = ring_col<F>(x, y, ex, ey);
+                    if (some) part[rc * zs + z] = own;
+                    if (!first && prev) part[col_carry_at<F>(zs) + rc * L + z] = carry[k];
+                } else if (first) {
+                    if (some) part[col_low_at<F>(zs) + ((x - L) * Iy + (y - L)) * L + z] = own;
+                } else if (some || prev || om.overwrite) {
+                    const float v = (float)((double)own + (double)carry[k]);
+                    float *q = node(x, y, z);
+                    *q = out_value(v, om.overwrite ? 0.0f : *q, om);
+                }
+                carry[k] = up;
+            }
+        }
+        // middle planes of the interior
+        if (some || om.overwrite) {
+#pragma unroll
+            for (int k = 0; k < KI; ++k) {
+                int x, y, z;
+                if (middle(k, x, y, z)) {
+                    const float v = some ? value(box_off<MAS, 3>(x, y, z)) : 0.0f;
+                    *node(x, y, z) = out_value(v, om.overwrite || !some ? 0.0f : old[k], om);
+                }
+            }
+        }
+        // middle planes of the ring
+        if (some) {
+            const int nr = ring_count<F>(ex, ey);
+            for (int i = tf; i < nr * ZW; i += NT) {
+                const int rc = i / ZW, zz = i - rc * ZW;
+                int x, y;
+                ring_xy<F>(rc, ex, ey, x, y);
+                if (UNI || zz < ez - L) part[rc * zs + L + zz] = value(box_off<MAS, 3>(x, y, L + zz));
+            }
+        }
+        prev = some;
+        __syncthreads();
+    }
+    // what the last tile carries over, for the tile above it (the next segment's first)
+    if (prev) {
+        float *part = partials + ((long long)col * g.nt + (tz1 == g.nt ? 0 : tz1)) * g.pslot;
+#pragma unroll
+        for (int k = 0; k < KC; ++k) {
+            const int i = t + k * NT, xy = i / L, z = i - xy * L, x = xy / B, y = xy - x * B;
+            if (x < ex + L && y < ey + L) {
+                if (in_ring<F>(x, y, ex, ey)) part[col_carry_at<F>(zs) + ring_col<F>(x, y, ex, ey) * L + z] = carry[k];
+                else part[col_clow_at<F>(zs) + ((x - L) * Iy + (y - L)) * L + z] = carry[k];
+            }
+        }
+    }
+}
+
+// Band columns (x < L or y < L) of a tile, and the low planes of a segment's first tile:
+// per x and y image the own ring value, then for z < L the carried one, summed in double
+// and written once.  One workgroup per tile; 16 lanes take a column.  Bound by HBM
+// latency: a column has two to five loads to wait for, so a thread issues those of
+// several columns (col_fin_unroll) before the first sum.  134 M particles, TSC on 512^3:
+// 0.29 ms in the tile form (partial values in runs of 2 to 18 floats, 8-byte pieces of
+// grid rows), 0.14 ms; 500^3 (uneven tiles): 0.57 -> 0.18 ms; 2 M weighted particles,
+// PCS on 512^3: 0.42 -> 0.20 ms.
+constexpr int kColFinBlock = 256;
+template <int MAS>
+constexpr int col_fin_unroll() { return MAS == PYL_CIC ? 2 : MAS == PYL_TSC ? 4 : 3; }
+
+template <int MAS, bool UNI>
+__global__ void __launch_bounds__(kColFinBlock)
+column_finalize_kernel(const unsigned long long *__restrict__ offsets, TileGeom g,
+                       const float *__restrict__ partials, float *__restrict__ grid, OutMode om, ColSeg cs,
+                       CapRecs cr) {
+    constexpr int F = MAS, L = F - 1, T = kT3;
+    __shared__ unsigned s_has;                          // bit (a*2 + b)*2 + c: image (a, b, c) has records
+    const int key = xcd_contiguous_block();
+    const int col = key / g.nt, tz = key - col * g.nt;
+    const int real = col / (g.nt * g.nt);
+    const int tx = col / g.nt - real * g.nt, ty = col % g.nt;
+    const int px = tx == 0 ? g.nt - 1 : tx - 1, py = ty == 0 ? g.nt - 1 : ty - 1, pz = tz == 0 ? g.nt - 1 : tz - 1;
+    const long long cbase = (long long)real * g.nt * g.nt;
+    if (threadIdx.x < 64) {
+        bool any = false;
+        if (threadIdx.x < 8) {
+            const int a = threadIdx.x >> 2, b = (threadIdx.x >> 1) & 1, c = threadIdx.x & 1;
+            const long long k = (cbase + (long long)(a ? px : tx) * g.nt + (b ? py : ty)) * g.nt + (c ? pz : tz);
+            any = offsets[k] != offsets[k + 1] || cap_count(cr, k) != 0;
+        }
+        const unsigned long long m = __ballot(any);
+        if (threadIdx.x == 0) s_has = (unsigned)m;
+    }
+    __syncthreads();
+    const unsigned has = s_has;
+    const bool first = tz % cs.len == 0;
+    // an accumulated grid is left alone where no tile contributes
+    if (!om.overwrite && has == 0) return;
+    auto extent = [&](int i) { return UNI ? T : g.orig[i + 1] - g.orig[i]; };
+    const int ex = extent(tx), ey = extent(ty), ez = extent(tz), pex = extent(px), pey = extent(py);
+    const int ox = UNI ? tx * T : g.orig[tx], oy = UNI ? ty * T : g.orig[ty], oz = UNI ? tz * T : g.orig[tz];
+    const int zs = UNI ? T : cs.zs;
+    const unsigned dd = (unsigned)g.dims;
+    grid += real * g.ncell + ((long long)ox * g.dims + oy) * g.dims + oz;
+    const float *img[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+        img[i] = partials + ((cbase + (long long)((i & 2) ? px : tx) * g.nt + ((i & 1) ? py : ty)) * g.nt + tz) * g.pslot;
+    const int Iy = ey - L, nband = ex * ey - (ex - L) * Iy;
+    const int lane = threadIdx.x & 15;
+    constexpr int U = col_fin_unroll<MAS>(), NC = kColFinBlock / 16;
+    for (int cb = threadIdx.x >> 4; cb < nband; cb += U * NC) {
+        float v[U][8], old[U];
+        float *q[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int c = cb + u * NC;
+            int x, y;
+            if (c < L * ey) {
+                if constexpr (UNI) {
+                    x = c / T;
+                    y = c - x * T;
+                } else {
+                    small_div(c, ey, x, y);
+                }
+            } else {
+                const int r = c - L * ey;
+                x = L + r / L;
+                y = r % L;
+            }
+            const bool on = c < nband && lane < ez;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const bool a = (i & 2) != 0, b = (i & 1) != 0;
+                const bool in = on && (!a || x < L) && (!b || y < L);
+                const int eax = a ? pex : ex, eby = b ? pey : ey;
+                const int rc = ring_col<F>(a ? eax + x : x, b ? eby + y : y, eax, eby);
+                v[u][2 * i] = v[u][2 * i + 1] = 0.0f;
+                if (in && ((has >> (2 * i)) & 1u)) v[u][2 * i] = img[i][rc * zs + lane];
+                if (in && lane < L && ((has >> (2 * i + 1)) & 1u))
+                    v[u][2 * i + 1] = img[i][col_carry_at<F>(zs) + rc * L + lane];
+            }
+            old[u] = 0.0f;
+            q[u] = on ? grid + (long long)((unsigned)x * dd + (unsigned)y) * dd + (unsigned)lane : nullptr;
+            if (on && !om.overwrite) old[u] = *q[u];
+        }
+        // every load is issued before the first sum
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+            asm volatile("" ::"v"(v[u][0]), "v"(v[u][1]), "v"(v[u][2]), "v"(v[u][3]), "v"(v[u][4]), "v"(v[u][5]),
+                         "v"(v[u][6]), "v"(v[u][7]), "v"(old[u]));
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            if (!q[u]) continue;
+            double sum = 0.0;
+#pragma unroll
+            for (int i = 0; i < 8; ++i) sum += (double)v[u][i];
+            *q[u] = out_value((float)sum, old[u], om);
+        }
+    }
+    if (!first) return;
+    for (int i = threadIdx.x; i < (ex - L) * Iy * L; i += kColFinBlock) {
+        const int ic = i / L, z = i - ic * L;
+        int x, y;
+        if constexpr (UNI) {
+            x = ic / (T - L);
+            y = ic - x * (T - L);
+        } else {
+            small_div(ic, Iy, x, y);
+        }
+        float own = 0.0f, up = 0.0f;
+        if (has & 1u) own = img[0][col_low_at<F>(zs) + i];
+        if (has & 2u) up = img[0][col_clow_at<F>(zs) + i];
+        float *q = grid + (long long)((unsigned)(x + L) * dd + (unsigned)(y + L)) * dd + (unsigned)z;
+        *q = out_value((float)((double)own + (double)up), om.overwrite ? 0.0f : *q, om);
     }
 }
 
@@ -2937,9 +3383,24 @@ int run_tiled(Ctx *c, const float *pos, const RSD &rsd, long long n, const long 
     //              (ordered) order bucket sizes[512] | bucket cursors[512]
     // Largest tiles first, when there are enough tiles, and records per tile, for the
     // dispatch tail to outweigh the ordering passes.
+    // 3D grids of two tiles or more per axis: the column deposit (segments along z), but
+    // for PCS in dense even tiles, whose deposit is bound by its LDS atomics throughout:
+    // there the flush between tiles costs what the finalize gains (1024^3 particles on
+    // 1024^3: tile form 14.4 + 2.9 ms, column form 15.9 + 1.7; 2 M on 512^3: 0.78 + 0.40
+    // and 0.73 + 0.23).
+    const bool uni = g.nt >= 2 && dims % (axes == 3 ? kT3 : kT2) == 0;
+    const bool column = axes == 3 && g.nt >= 2 && MAS > 1 && nsplit == 1 &&
+                        !(MAS == PYL_PCS && uni && n >= kColPcsDense * nt);
+    ColSeg cs{1, g.nt, (dims + g.nt - 1) / g.nt};
+    if (column) {
+        while (cs.len < kColMaxLen && nt >= 2 * cs.len * kColMinSegs) cs.len *= 2;
+        cs.nz = (g.nt + cs.len - 1) / cs.len;
+    }
+    const long long nseg = column ? (long long)nreal * g.nt * g.nt * cs.nz : nt;
+    const OrderSeg oseg = column ? OrderSeg{cs.len, g.nt, cs.nz} : OrderSeg{1, 1, 1};
     const bool ordered = c->tune_order >= 0
         ? (nsplit == 1 && c->tune_order == 1)
-        : (nsplit == 1 && nt >= kOrderMinKeys && n >= kOrderMinRecords * nt);
+        : (nsplit == 1 && nseg >= kOrderMinKeys && n >= kOrderMinRecords * nt);
     size_t nwords = (size_t)nt * 3 + (size_t)nreal + 1 + (two ? (size_t)nbk : 0);
     const size_t cur_at = nwords;
     if (capm) nwords += (size_t)nt;
@@ -3163,9 +3624,9 @@ int run_tiled(Ctx *c, const float *pos, const RSD &rsd, long long n, const long 
         PYL_TRY(stage_begin(c, PYL_STAGE_MA_SCAN));
         if (ordered) {
             const CapRecs ocr{crec, cursor, cap, (long long)n};
-            order_hist_kernel<<<order_wgs(nt), kOrderBlock, 0, c->stream>>>(offsets, nt, ocr, ohist);
-            order_place_kernel<<<order_wgs(nt), kOrderBlock, 0, c->stream>>>(offsets, nt, ocr, ohist,
-                                                                              ohist + kOrderBuckets, order);
+            order_hist_kernel<<<order_wgs(nseg), kOrderBlock, 0, c->stream>>>(offsets, nseg, oseg, ocr, ohist);
+            order_place_kernel<<<order_wgs(nseg), kOrderBlock, 0, c->stream>>>(offsets, nseg, oseg, ocr, ohist,
+                                                                                ohist + kOrderBuckets, order);
         }
         PYL_HIP(hipGetLastError());
         PYL_TRY(stage_end(c, PYL_STAGE_MA_SCAN));
@@ -3193,9 +3654,9 @@ int run_tiled(Ctx *c, const float *pos, const RSD &rsd, long long n, const long 
                                                                        offsets);
         if (ordered) {
             const CapRecs ocr{nullptr, nullptr, 0, -1};
-            order_hist_kernel<<<order_wgs(nt), kOrderBlock, 0, c->stream>>>(offsets, nt, ocr, ohist);
-            order_place_kernel<<<order_wgs(nt), kOrderBlock, 0, c->stream>>>(offsets, nt, ocr, ohist,
-                                                                              ohist + kOrderBuckets, order);
+            order_hist_kernel<<<order_wgs(nseg), kOrderBlock, 0, c->stream>>>(offsets, nseg, oseg, ocr, ohist);
+            order_place_kernel<<<order_wgs(nseg), kOrderBlock, 0, c->stream>>>(offsets, nseg, oseg, ocr, ohist,
+                                                                                ohist + kOrderBuckets, order);
         }
         PYL_HIP(hipGetLastError());
         PYL_TRY(stage_end(c, PYL_STAGE_MA_SCAN));
@@ -3283,7 +3744,27 @@ int run_tiled(Ctx *c, const float *pos, const RSD &rsd, long long n, const long 
     }
     const bool unit = W == nullptr && weight_factor == 1.0f;
     PYL_TRY(stage_begin(c, PYL_STAGE_MA_DEPOSIT));
-    const bool uni = g.nt >= 2 && dims % (axes == 3 ? kT3 : kT2) == 0;
+    const CapRecs cr = capm ? CapRecs{crec, cursor, cap, (long long)n} : CapRecs{nullptr, nullptr, 0, -1};
+    if constexpr (MAS > 1) {
+        if (column) {
+            auto kcol = uni ? (unit ? column_deposit_kernel<MAS, false, false, true>
+                                    : (W ? column_deposit_kernel<MAS, true, true, true>
+                                         : column_deposit_kernel<MAS, true, false, true>))
+                            : (unit ? column_deposit_kernel<MAS, false, false, false>
+                                    : (W ? column_deposit_kernel<MAS, true, true, false>
+                                         : column_deposit_kernel<MAS, true, false, false>));
+            kcol<<<(unsigned)nseg, kDepBlock, 0, c->stream>>>(records, rcap, offsets, g, weight_factor,
+                                                              W ? wmax : nullptr, grid, partials, om,
+                                                              ordered ? order : nullptr, cs, cr);
+            PYL_HIP(hipGetLastError());
+            PYL_TRY(stage_end(c, PYL_STAGE_MA_DEPOSIT));
+            PYL_TRY(stage_begin(c, PYL_STAGE_MA_FINAL));
+            (uni ? column_finalize_kernel<MAS, true> : column_finalize_kernel<MAS, false>)
+                <<<(unsigned)nt, kColFinBlock, 0, c->stream>>>(offsets, g, partials, grid, om, cs, cr);
+            PYL_HIP(hipGetLastError());
+            return stage_end(c, PYL_STAGE_MA_FINAL);
+        }
+    }
     auto kd = (axes == 3)
         ? (uni ? (unit ? tile_deposit_kernel<MAS, 3, false, false, true>
                        : (W ? tile_deposit_kernel<MAS, 3, true, true, true>
@@ -3298,7 +3779,6 @@ int run_tiled(Ctx *c, const float *pos, const RSD &rsd, long long n, const long 
                        : (W ? tile_deposit_kernel<MAS, 2, true, true, false>
                             : tile_deposit_kernel<MAS, 2, true, false, false>)));
     if (nsplit > 1) PYL_TRY(zero_bytes(c, gbox, (size_t)nt * nbox * sizeof(unsigned long long)));
-    const CapRecs cr = capm ? CapRecs{crec, cursor, cap, (long long)n} : CapRecs{nullptr, nullptr, 0, -1};
     kd<<<(unsigned)(nt * nsplit), kDepBlock, 0, c->stream>>>(records, rcap, offsets, g, weight_factor,
                                                             W ? wmax : nullptr, grid, partials, om,
                                                             ordered ? order : nullptr, nsplit, gbox, cr);

@@ -5,6 +5,7 @@
 //   - the 16 lanes of a pass are in 16 different bank pairs at every step (PCS), or in
 //     the 8 (2D: 4) residues of the coordinates' parities two (four) lanes each (CIC),
 //     whatever the lanes' first nodes;
+//   - the partial layout of the column deposit numbers every value once, inside the slot;
 //   - the tile of a node, taken by a multiplication, is the exact quotient;
 //   - the PCS weights match the cubic B-spline in long double to float rounding.
 // Built and run by tests/test_ma_box_emul.py (host compile only, no GPU calls).
@@ -136,10 +137,47 @@ static int check_node_tile() {
     return bad;
 }
 
+// Partial layout of the column deposit: for every pair of tile extents the ring columns
+// are numbered once each (ring_col and ring_xy inverse), the four parts of a tile's slot
+// do not overlap and fill at most the slot (halo_count of the largest tile).
+template <int F>
+static int check_ring() {
+    constexpr int L = F - 1;
+    int bad = 0;
+    for (int zs = 8; zs <= kT3; ++zs)
+        for (int ex = zs - 1; ex <= zs; ++ex)
+            for (int ey = zs - 1; ey <= zs; ++ey) {
+                std::vector<int> seen(ring_count<F>(ex, ey), 0);
+                for (int x = 0; x < ex + L; ++x)
+                    for (int y = 0; y < ey + L; ++y) {
+                        if (!in_ring<F>(x, y, ex, ey)) continue;
+                        const int rc = ring_col<F>(x, y, ex, ey);
+                        int a, b;
+                        if (rc < 0 || rc >= (int)seen.size() || seen[rc]++) { ++bad; continue; }
+                        ring_xy<F>(rc, ex, ey, a, b);
+                        if (a != x || b != y) ++bad;
+                    }
+                for (int v : seen) if (v != 1) ++bad;
+                const int nr = ring_count<F>(ex, ey), ni = (ex - L) * (ey - L) * L;
+                if (nr * zs > col_carry_at<F>(zs)) ++bad;
+                if (col_carry_at<F>(zs) + nr * L > col_low_at<F>(zs)) ++bad;
+                if (col_low_at<F>(zs) + ni > col_clow_at<F>(zs)) ++bad;
+                if (col_clow_at<F>(zs) + ni > halo_count<F, 3>(zs, zs, zs)) ++bad;
+            }
+    for (int d = 1; d <= 19; ++d)
+        for (int v = 0; v < 2048; ++v) {
+            int q, r;
+            small_div(v, d, q, r);
+            if (q != v / d || r != v % d) ++bad;
+        }
+    printf("ring F %d: %s\n", F, bad ? "FAIL" : "ok");
+    return bad;
+}
+
 int main() {
     int bad = check_steps<PYL_CIC, 3>() + check_steps<PYL_CIC, 2>() + check_steps<PYL_PCS, 3>() + check_steps<PYL_PCS, 2>();
     bad += check_box<PYL_NGP, 3>() + check_box<PYL_NGP, 2>() + check_box<PYL_TSC, 3>() + check_box<PYL_TSC, 2>();
-    bad += check_pcs_weights() + check_node_tile();
+    bad += check_pcs_weights() + check_node_tile() + check_ring<2>() + check_ring<3>() + check_ring<4>();
     printf(bad ? "FAILURES: %d\n" : "all ok\n", bad);
     return bad != 0;
 }
