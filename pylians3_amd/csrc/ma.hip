@@ -386,11 +386,24 @@ __host__ __device__ __forceinline__ long long win_key(int s, const Win &w, const
     return rbase + k;
 }
 
+// Particles per tile and chunk of the tile sort, at least, on grids of under 512 tiles
+// (100 k particles on 64^3, 64 tiles: 98 workgroups instead of 13, count 8 -> 6.7 us,
+// scatter 11.5 -> 6.8).  At 512 tiles chunks of 4096 lose more to the tiles' counter
+// atomics than the second workgroup per CU gains (2 M on 128^3, whole call: 106 us, with
+// 8192 100).
+constexpr long long kChunkPerTile = 16;
+
 // Particles per thread and loop trip: the loads of kUnroll particles are issued
 // (unconditionally, at clamped indices) before any of them is used, so their
 // latencies overlap.
 constexpr int kUnroll = 4;       // count pass (measured best of 2, 4, 8 at 512^3)
 constexpr int kUnrollS = 8;      // scatter pass (8: 0.80 -> 0.71 ms at 512^3)
+
+// Words of a chunk's row in the count pass's dump.
+template <int WS>
+__host__ __device__ __forceinline__ long long dump_stride(const TileGeom &g) {
+    return g.wmode == kWinDirect ? g.ntiles : (long long)WS;
+}
 
 template <int MAS, int AXES, bool POW2, int WS>
 __global__ void __launch_bounds__(kSortBlock)
@@ -445,7 +458,7 @@ tile_count_kernel(const float *__restrict__ pos, RSD rsd, float inv, TileGeom g,
         }
     }
     __syncthreads();
-    unsigned *dmp = dump + (long long)blockIdx.x * WS;
+    unsigned *dmp = dump + (long long)blockIdx.x * dump_stride<WS>(g);
     int smin = WS, smax = -1;
     for (int s = threadIdx.x; s < w.slots; s += blockDim.x) {
         const unsigned v = hist[s];
@@ -512,7 +525,7 @@ tile_scatter_kernel(const float *__restrict__ pos, RSD rsd, const float *__restr
         win.a = ch.wbase;
         win.slots = kWin;
     }
-    const unsigned *dmp = dump + (long long)blockIdx.x * WS;
+    const unsigned *dmp = dump + (long long)blockIdx.x * dump_stride<WS>(g);
     // only slots in [smin, smax] were counted; no other slot is looked up
     for (int s = ch.smin + threadIdx.x; s <= ch.smax; s += blockDim.x) cur[s] = dmp[s];
     __syncthreads();
@@ -783,6 +796,28 @@ spill_count_kernel(const float *__restrict__ sxyz, const unsigned long long *__r
     }
 }
 
+// What a sort tells the host, written by its last counting kernel straight into
+// pinned host words (with the single-launch scan and the smaller chunks: 100 k particles
+// on 64^3 88 -> 67 us a call; an 8-byte copy on the stream costs more than the scan).  A
+// null destination is not wanted.
+struct SortReport {
+    unsigned long long *total;               // records sorted
+    unsigned long long *miss;                // box misses of the count pass
+    unsigned long long *ndev;                // total of the device particle ranges
+    unsigned long long *spill;               // particles of the spill list
+    const unsigned *miss_src;
+    const long long *ndev_src;
+    const unsigned long long *spill_src;
+};
+
+__device__ __forceinline__ void report(const SortReport &r, unsigned long long total) {
+    if (r.miss) *r.miss = *r.miss_src;
+    if (r.ndev) *r.ndev = (unsigned long long)*r.ndev_src;
+    if (r.spill) *r.spill = *r.spill_src;
+    *r.total = total;
+    __threadfence_system();
+}
+
 // One record per spilled particle at offsets[key] + its rank (ocursors zeroed).  Also
 // the capacity sort's record total: total = sorted spill (offsets[ntiles]) + placed.
 template <int MAS, bool POW2, bool WT>
@@ -791,8 +826,8 @@ spill_scatter_kernel(const float *__restrict__ sxyz, const float *__restrict__ s
                      const unsigned long long *__restrict__ nspill, TileGeom g,
                      const unsigned long long *__restrict__ offsets, unsigned *__restrict__ ocursors,
                      float *__restrict__ records, unsigned long long rcap,
-                     const unsigned long long *__restrict__ placed, unsigned long long *__restrict__ total) {
-    if (blockIdx.x == 0 && threadIdx.x == 0) total[0] = offsets[g.ntiles] + placed[0];
+                     const unsigned long long *__restrict__ placed, SortReport rep) {
+    if (blockIdx.x == 0 && threadIdx.x == 0) report(rep, offsets[g.ntiles] + placed[0]);
     const unsigned long long ns = *nspill;
     if (ns > kSpillAtomic) return;
     const RSD off{sxyz, 0.0f, 0.0f, 0, 3, 0};
@@ -828,31 +863,39 @@ spill_scatter_kernel(const float *__restrict__ sxyz, const float *__restrict__ s
 constexpr int kScanBlock = 1024;
 constexpr int kScanItems = 4;
 constexpr int kScanTile = kScanBlock * kScanItems;
+constexpr int kScanOne = 16;                   // workgroups of the single-launch scan
 
+// Exclusive scan over the kScanBlock threads (sh: one word per wavefront): shuffles
+// inside a wavefront, then every thread adds the sums of the wavefronts before its own.
 __device__ __forceinline__ unsigned long long block_exclusive_scan(unsigned long long v,
                                                                    unsigned long long *sh,
                                                                    unsigned long long &total) {
-    // Hillis-Steele over the block in LDS (1024 entries).
-    int t = threadIdx.x;
-    sh[t] = v;
-    __syncthreads();
-    for (int off = 1; off < kScanBlock; off <<= 1) {
-        unsigned long long a = (t >= off) ? sh[t - off] : 0ull;
-        __syncthreads();
-        sh[t] += a;
-        __syncthreads();
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    unsigned long long s = v;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+        const unsigned long long a = __shfl_up(s, off);
+        if (lane >= off) s += a;
     }
-    total = sh[kScanBlock - 1];
-    unsigned long long incl = sh[t];
+    if (lane == 63) sh[wave] = s;
     __syncthreads();
-    return incl - v;
+    unsigned long long before = 0, all = 0;
+#pragma unroll
+    for (int w = 0; w < kScanBlock / 64; ++w) {
+        const unsigned long long x = sh[w];
+        if (w < wave) before += x;
+        all += x;
+    }
+    __syncthreads();                           // sh may be used again
+    total = all;
+    return before + s - v;
 }
 
 // The scanned value of element i is in[i] + in2[i].
 __global__ void __launch_bounds__(kScanBlock)
 scan_partial_kernel(const unsigned *__restrict__ in, const unsigned *__restrict__ in2,
                     long long n, unsigned long long *__restrict__ block_sums) {
-    __shared__ unsigned long long sh[kScanBlock];
+    __shared__ unsigned long long sh[kScanBlock / 64];
     long long base = (long long)blockIdx.x * kScanTile + (long long)threadIdx.x * kScanItems;
     unsigned long long s = 0;
     for (int k = 0; k < kScanItems; ++k)
@@ -865,7 +908,7 @@ scan_partial_kernel(const unsigned *__restrict__ in, const unsigned *__restrict_
 __global__ void __launch_bounds__(kScanBlock)
 scan_blocksums_kernel(unsigned long long *__restrict__ block_sums, int nblocks) {
     // Single block: nblocks <= kScanTile.
-    __shared__ unsigned long long sh[kScanBlock];
+    __shared__ unsigned long long sh[kScanBlock / 64];
     int t = threadIdx.x;
     unsigned long long v[kScanItems];
     unsigned long long s = 0;
@@ -883,12 +926,28 @@ scan_blocksums_kernel(unsigned long long *__restrict__ block_sums, int nblocks) 
     }
 }
 
+// ONE: the sums of the elements before the workgroup's are formed here (up to
+// kScanOne workgroups, which read at most 8 * kScanOne * kScanTile bytes each from
+// cache) instead of by the two kernels above: one launch, whose time is latency (4096
+// keys: 3 launches of 9.3 us and their gaps -> 3.7 us; 16384 keys 10 us).
+template <bool ONE>
 __global__ void __launch_bounds__(kScanBlock)
 scan_final_kernel(const unsigned *__restrict__ in, const unsigned *__restrict__ in2, long long n,
                   const unsigned long long *__restrict__ block_prefix,
-                  unsigned long long *__restrict__ out) {
-    __shared__ unsigned long long sh[kScanBlock];
-    long long base = (long long)blockIdx.x * kScanTile + (long long)threadIdx.x * kScanItems;
+                  unsigned long long *__restrict__ out, SortReport rep) {
+    __shared__ unsigned long long sh[kScanBlock / 64];
+    const long long first = (long long)blockIdx.x * kScanTile;
+    unsigned long long prefix = 0;
+    if (ONE) {
+        unsigned long long p = 0;
+#pragma unroll 4
+        for (long long i = threadIdx.x; i < first; i += kScanBlock)
+            p += (unsigned long long)in[i] + in2[i];
+        block_exclusive_scan(p, sh, prefix);
+    } else {
+        prefix = block_prefix[blockIdx.x];
+    }
+    const long long base = first + (long long)threadIdx.x * kScanItems;
     unsigned long long v[kScanItems];
     unsigned long long s = 0;
     for (int k = 0; k < kScanItems; ++k) {
@@ -896,12 +955,15 @@ scan_final_kernel(const unsigned *__restrict__ in, const unsigned *__restrict__ 
         s += v[k];
     }
     unsigned long long total;
-    unsigned long long ex = block_exclusive_scan(s, sh, total) + block_prefix[blockIdx.x];
+    unsigned long long ex = block_exclusive_scan(s, sh, total) + prefix;
     for (int k = 0; k < kScanItems; ++k) {
         if (base + k < n) out[base + k] = ex;
         ex += v[k];
     }
-    if (blockIdx.x == gridDim.x - 1 && threadIdx.x == kScanBlock - 1) out[n] = ex;
+    if (blockIdx.x == gridDim.x - 1 && threadIdx.x == kScanBlock - 1) {
+        out[n] = ex;
+        if (rep.total) report(rep, ex);
+    }
 }
 
 // ---- two-level sort (3D, particles in any order) -------------------------------
@@ -996,7 +1058,7 @@ bucket_count_kernel(const float *__restrict__ pos, RSD rsd, float inv, TileGeom 
 __global__ void __launch_bounds__(kScanBlock)
 bucket_scan_kernel(const unsigned *__restrict__ bmat, int nchunk, int nb,
                    unsigned *__restrict__ bdump, unsigned *__restrict__ bcounts) {
-    __shared__ unsigned long long sh[kScanBlock];
+    __shared__ unsigned long long sh[kScanBlock / 64];
     const int b = blockIdx.x;
     const unsigned *col = bmat + (long long)b * nchunk;
     unsigned long long carry = 0;
@@ -1028,7 +1090,7 @@ bucket_scan_kernel(const unsigned *__restrict__ bmat, int nchunk, int nb,
 __global__ void __launch_bounds__(kScanBlock)
 bucket_plan_kernel(const unsigned *__restrict__ bcounts, int nb, long long target,
                    unsigned long long *__restrict__ boffsets, Chunk *__restrict__ ch, int nchunk) {
-    __shared__ unsigned long long sh[kScanBlock];
+    __shared__ unsigned long long sh[kScanBlock / 64];
     const int b0 = threadIdx.x * kScanItems;
     unsigned long long len[kScanItems], s = 0, nc = 0;
     for (int k = 0; k < kScanItems; ++k) {
@@ -3205,6 +3267,19 @@ TileGeom make_geom(int dims, int axes, int mas) {
     return g;
 }
 
+// offsets[0..nt] of the tile counts; `rep` as in scan_final_kernel (rep.total null: none).
+void launch_scan(Ctx *c, const unsigned *counts, const unsigned *ocounts, long long nt, int nblocks,
+                 unsigned long long *bsums, unsigned long long *offsets, const SortReport &rep) {
+    if (nblocks <= kScanOne) {
+        scan_final_kernel<true><<<nblocks, kScanBlock, 0, c->stream>>>(counts, ocounts, nt, nullptr, offsets,
+                                                                       rep);
+        return;
+    }
+    scan_partial_kernel<<<nblocks, kScanBlock, 0, c->stream>>>(counts, ocounts, nt, bsums);
+    scan_blocksums_kernel<<<1, kScanBlock, 0, c->stream>>>(bsums, nblocks);
+    scan_final_kernel<false><<<nblocks, kScanBlock, 0, c->stream>>>(counts, ocounts, nt, bsums, offsets, rep);
+}
+
 // The latest order finding per (device, dims, MAS) over every context of the
 // process: a context that has not sorted such a grid yet starts from it (requests
 // from one source -- a server's slots, a pipeline's threads -- tend to share their
@@ -3354,10 +3429,16 @@ int run_tiled(Ctx *c, const float *pos, const RSD &rsd, long long n, const long 
     // kWinDirect/Box/Linear == PYL_WINDOW_DIRECT/BOX/LINEAR
     c->last_window = (capm && two) ? PYL_WINDOW_TWOLEVEL_CAPACITY
                    : capm ? PYL_WINDOW_CAPACITY : two ? PYL_WINDOW_TWOLEVEL : wide ? PYL_WINDOW_WIDE : g.wmode;
-    const int ws = capm ? sws : two ? kBktSlots : wide ? kWinWide : kWin;
+    const int ws = capm ? (gs.wmode == kWinDirect ? (int)g.ntiles : sws)
+                 : two ? kBktSlots
+                 : g.wmode == kWinDirect ? (int)g.ntiles : kWin;
     // Chunks of consecutive particles, never straddling two realisations.
+    // A few small tiles take small chunks down to kChunkPerTile particles per tile: more
+    // workgroups for a call that would not fill the chip.  (Fixed scratch keeps to 8192.)
+    const long long floor = c->arena ? 8192LL
+                                     : std::max(1024LL, std::min(8192LL, kChunkPerTile * g.ntiles));
     const long long target = wide ? std::max(2 * g.ntiles, std::min(16 * g.ntiles, (n + 2047) / 2048))
-                                  : std::max(8192LL, std::min(65536LL, (n + 4095) / 4096));
+                                  : std::max(floor, std::min(65536LL, (n + 4095) / 4096));
     long long nchunk_ll = 0;
     if (devt) nchunk_ll = (long long)nreal * c->chunks_per_real;
     else
@@ -3379,7 +3460,7 @@ int run_tiled(Ctx *c, const float *pos, const RSD &rsd, long long n, const long 
     //              (two-level) bucket counts[nbk] | pad | offsets[nt+1] | block sums |
     //              chunk table | tile origins | tile order | per-chunk window bases |
     //              (two-level) bucket offsets[nbk+1] | pass-2 chunk table | bucket bases
-    //              (capacity) tile cursors[nt] | pad | spill range {0, count}, placed, total (u64)
+    //              (capacity) tile cursors[nt] | pad | spill range {0, count}, placed (u64)
     //              (ordered) order bucket sizes[512] | bucket cursors[512]
     // Largest tiles first, when there are enough tiles, and records per tile, for the
     // dispatch tail to outweigh the ordering passes.
@@ -3559,6 +3640,41 @@ int run_tiled(Ctx *c, const float *pos, const RSD &rsd, long long n, const long 
         schunks = dchunks2;
         g.wmode = kWinBlock;
     }
+    // The record total (offsets[nt]; capacity form: the sorted spill plus the placed
+    // records) must equal n; the sort's last counting kernel writes it to the host,
+    // which checks it at the next synchronising call on this context.  Until then the
+    // scatter and the deposit keep every record index below n (capacity slots: below
+    // the tile's capacity), so a bad count cannot write or read outside the record
+    // buffers.
+    SortReport rep{};
+    const auto make_report = [&]() {
+        PYL_TRY(check_total(c));                // the previous call's words, if still unread
+        rep.miss_src = box_miss;
+        rep.ndev_src = devt ? c->dev_offs + nreal : nullptr;
+        rep.spill_src = capm ? capw + 1 : nullptr;
+        if (c->capturing) {
+            // each captured call writes its totals to pinned words of its own, compared
+            // after every replay
+            unsigned long long *ht = nullptr;
+            PYL_HIP(hipHostMalloc((void **)&ht, 2 * sizeof(unsigned long long), hipHostMallocDefault));
+            c->cap_host.push_back(ht);
+            ht[1] = (unsigned long long)n;
+            rep.total = ht;
+            if (devt) rep.ndev = ht + 1;
+            c->deferred.push_back([ht]() {
+                PYL_CHECK(ht[0] == ht[1], PYL_EHIP, "tile sort lost particles (%llu of %llu)", ht[0], ht[1]);
+                return PYL_OK;
+            });
+            return PYL_OK;
+        }
+        c->box_miss_n = -1;
+        c->cap_spill_n = -1;
+        rep.total = c->h_total;
+        if (devt) rep.ndev = c->h_total + 2;
+        if (tally && nchunk > 0) rep.miss = c->h_total + 1;
+        if (capm) rep.spill = c->h_total + 3;
+        return PYL_OK;
+    };
     if (capm) {
         // one read of the particles (or, after the two-level sort's first pass, of the
         // bucketed records) into the tile slots; the rest into the spill list
@@ -3601,9 +3717,7 @@ int run_tiled(Ctx *c, const float *pos, const RSD &rsd, long long n, const long 
                                           : tile_count_kernel<MAS, 3, false, kWin>);
         kc<<<kSpillChunks, kSortBlock, 0, c->stream>>>(pxyz, off, 1.0f, gs, dchunksS, counts, ocounts, dump,
                                                        nullptr);
-        scan_partial_kernel<<<nscan_blocks, kScanBlock, 0, c->stream>>>(counts, ocounts, nt, bsums);
-        scan_blocksums_kernel<<<1, kScanBlock, 0, c->stream>>>(bsums, nscan_blocks);
-        scan_final_kernel<<<nscan_blocks, kScanBlock, 0, c->stream>>>(counts, ocounts, nt, bsums, offsets);
+        launch_scan(c, counts, ocounts, nt, nscan_blocks, bsums, offsets, SortReport{});
         auto ks = sws == kWinWide
             ? (W ? (pow2 ? tile_scatter_kernel<MAS, 3, true, true, kWinWide>
                          : tile_scatter_kernel<MAS, 3, false, true, kWinWide>)
@@ -3617,8 +3731,9 @@ int run_tiled(Ctx *c, const float *pos, const RSD &rsd, long long n, const long 
                                                        ocursors, wmax, records, (unsigned long long)n);
         auto kss2 = W ? (pow2 ? spill_scatter_kernel<MAS, true, true> : spill_scatter_kernel<MAS, false, true>)
                       : (pow2 ? spill_scatter_kernel<MAS, true, false> : spill_scatter_kernel<MAS, false, false>);
+        PYL_TRY(make_report());
         kss2<<<kSpillBlocks, kBlock, 0, c->stream>>>(pxyz, pw, capw + 1, gs, offsets, ocursors, records,
-                                                     (unsigned long long)n, capw + 2, capw + 3);
+                                                     (unsigned long long)n, capw + 2, rep);
         PYL_HIP(hipGetLastError());
         PYL_TRY(stage_end(c, PYL_STAGE_MA_SPILL));
         PYL_TRY(stage_begin(c, PYL_STAGE_MA_SCAN));
@@ -3648,10 +3763,8 @@ int run_tiled(Ctx *c, const float *pos, const RSD &rsd, long long n, const long 
     }
     if (!capm) {
         PYL_TRY(stage_begin(c, PYL_STAGE_MA_SCAN));
-        scan_partial_kernel<<<nscan_blocks, kScanBlock, 0, c->stream>>>(counts, ocounts, nt, bsums);
-        scan_blocksums_kernel<<<1, kScanBlock, 0, c->stream>>>(bsums, nscan_blocks);
-        scan_final_kernel<<<nscan_blocks, kScanBlock, 0, c->stream>>>(counts, ocounts, nt, bsums,
-                                                                       offsets);
+        PYL_TRY(make_report());
+        launch_scan(c, counts, ocounts, nt, nscan_blocks, bsums, offsets, rep);
         if (ordered) {
             const CapRecs ocr{nullptr, nullptr, 0, -1};
             order_hist_kernel<<<order_wgs(nseg), kOrderBlock, 0, c->stream>>>(offsets, nseg, oseg, ocr, ohist);
@@ -3661,47 +3774,12 @@ int run_tiled(Ctx *c, const float *pos, const RSD &rsd, long long n, const long 
         PYL_HIP(hipGetLastError());
         PYL_TRY(stage_end(c, PYL_STAGE_MA_SCAN));
     }
-    // offsets[nt] (capacity form: the sorted spill plus the placed records) must
-    // equal n; it is read back asynchronously and checked at the next synchronising
-    // call on this context.  Until then the scatter and the deposit keep every
-    // record index below n (capacity slots: below the tile's capacity), so a bad
-    // count cannot write or read outside the record buffers.
-    const unsigned long long *total_word = capm ? capw + 3 : offsets + nt;
-    PYL_TRY(check_total(c));                    // the previous call's check, if still pending
-    if (c->capturing) {
-        // each captured call reads its totals into pinned words of its own, compared
-        // after every replay
-        unsigned long long *ht = nullptr;
-        PYL_HIP(hipHostMalloc((void **)&ht, 2 * sizeof(unsigned long long), hipHostMallocDefault));
-        c->cap_host.push_back(ht);
-        ht[1] = (unsigned long long)n;
-        PYL_HIP(hipMemcpyAsync(ht, total_word, sizeof(unsigned long long), hipMemcpyDeviceToHost,
-                               c->stream));
-        if (devt)
-            PYL_HIP(hipMemcpyAsync(ht + 1, c->dev_offs + nreal, sizeof(unsigned long long),
-                                   hipMemcpyDeviceToHost, c->stream));
-        c->deferred.push_back([ht]() {
-            PYL_CHECK(ht[0] == ht[1], PYL_EHIP, "tile sort lost particles (%llu of %llu)", ht[0], ht[1]);
-            return PYL_OK;
-        });
-    } else {
-        PYL_HIP(hipMemcpyAsync(c->h_total, total_word, sizeof(unsigned long long),
-                               hipMemcpyDeviceToHost, c->stream));
-        if (devt)
-            PYL_HIP(hipMemcpyAsync(c->h_total + 2, c->dev_offs + nreal, sizeof(unsigned long long),
-                                   hipMemcpyDeviceToHost, c->stream));
-        c->box_miss_n = -1;
-        if (tally && nchunk > 0) {
-            c->h_total[1] = 0;                 // the copy fills the low word
-            PYL_HIP(hipMemcpyAsync(c->h_total + 1, box_miss, sizeof(unsigned), hipMemcpyDeviceToHost,
-                                   c->stream));
+    if (!c->capturing) {
+        if (rep.miss) {
             c->box_miss_n = n;
             c->box_miss_key = hkey;
         }
-        c->cap_spill_n = -1;
-        if (capm) {
-            PYL_HIP(hipMemcpyAsync(c->h_total + 3, capw + 1, sizeof(unsigned long long),
-                                   hipMemcpyDeviceToHost, c->stream));
+        if (rep.spill) {
             c->cap_spill_n = n;
             c->cap_two = two;
             c->cap_key = hkey;
