@@ -166,16 +166,16 @@ class Pk:
         if verbose:
             print('Time to complete loop = %.2f' % (time.time() - start2))
         self.k1D = r['k1D']
-        self.Pk1D = r['Pk1D'][:, 0].copy()
+        self.Pk1D = r['Pk1D'][:, 0]           # one spectrum: the column is the whole array
         self.Nmodes1D = r['Nmodes1D']
         self.kpar = r['kpar']
         self.kper = r['kper']
-        self.Pk2D = r['Pk2D'][:, 0].copy()
+        self.Pk2D = r['Pk2D'][:, 0]
         self.Nmodes2D = r['Nmodes2D']
         check_number_modes(np.concatenate([[1.0], r['Nmodes3D']]), dims)
         self.k3D = r['k3D']
         self.Nmodes3D = r['Nmodes3D']
-        self.Pk = r['Pk3D'][:, :, 0].copy()
+        self.Pk = r['Pk3D'][:, :, 0]
         self.Pkphase = r['Pkphase']
         if verbose:
             print('Time taken = %.2f seconds' % (time.time() - start))

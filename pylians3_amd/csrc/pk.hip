@@ -1158,8 +1158,10 @@ int pk_bin_device(Ctx *c, const float2 *const *dk, long long fstride, long long 
         acc.S_total = S;
         acc.P3.resize((size_t)(p.kmax + 1) * 3 * S);
         acc.phase.assign(p.kmax + 1, 0.0);
-        acc.P2.resize((size_t)p.nb2 * S);
-        acc.P1.resize((size_t)(p.m + 1) * S);
+        if (F > 2) {              // one launch: the spectra are finalized where it put them
+            acc.P2.resize((size_t)p.nb2 * S);
+            acc.P1.resize((size_t)(p.m + 1) * S);
+        }
     }
     const bool phase = (F == 1) && !(flags & PYL_PK_NO_PHASE);
     if (F == 1) {
