@@ -1,11 +1,11 @@
 // Forward 3D real-to-complex FFT of power-of-two cubes (16..1024 per side).
 //
 // Same transform as FFT3Dr_f (library/Pk_library/Pk_library.pyx:117-130, FFTW
-// forward, unnormalised, e^{-i}): out[x][y][kz], kz in [0, N/2].  Three passes
-// over HBM:
+// forward, unnormalised, e^{-i}): out[x][y][kz], kz in [0, N/2].  Passes over HBM:
 //   z: r2c of the contiguous rows (N/2-point complex FFTs of the even/odd
 //      pairs, then the split into the N/2+1 output modes);
-//   y: complex FFTs along y, in place;
+//   y: complex FFTs along y, in place (N = 64 and 128: both in one pass, a plane
+//      per workgroup);
 //   x: complex FFTs along x, in place.
 // The y and x passes use the same column kernel: a workgroup loads C
 // consecutive kz columns (C*8 bytes contiguous per point) of one (x or y) line
@@ -75,10 +75,10 @@ __device__ __forceinline__ void dft(float2 *v) {
 }
 
 // One Stockham stage of radix R over C interleaved columns held in LDS
-// (element (n, c) at buf[n*CP + c], CP >= C a padded stride).  Span Ns:
-// sub-transforms of length Ns are complete; this stage makes them Ns*R long.
-// BLK threads; every thread reads its inputs before any thread writes.
-template <int N, int C, int CP, int R, int BLK>
+// (element (n, c) at buf[n*CP + c*CS]; CP, CS padded).  Span Ns: sub-transforms
+// of length Ns are complete; this stage makes them Ns*R long.  FIRST: span 1, without
+// its unit twiddles.  BLK threads; every thread reads its inputs before any thread writes.
+template <int N, int C, int CP, int R, int BLK, int CS = 1, bool FIRST = false>
 __device__ __forceinline__ void stage(float2 *buf, const float2 *__restrict__ tw, int Ns) {
     constexpr int NB = (N / R) * C;                          // butterflies
     constexpr int PER = (NB + BLK - 1) / BLK;                // per thread
@@ -94,12 +94,12 @@ __device__ __forceinline__ void stage(float2 *buf, const float2 *__restrict__ tw
             const int tstep = (N / (Ns * R)) * k;
 #pragma unroll
             for (int m = 0; m < R; ++m) {
-                float2 x = buf[(j + m * (N / R)) * CP + c];
-                if (m > 0) x = cmul(x, tw[(m * tstep) & (N - 1)]);
+                float2 x = buf[(j + m * (N / R)) * CP + c * CS];
+                if (!FIRST && m > 0) x = cmul(x, tw[(m * tstep) & (N - 1)]);
                 v[p][m] = x;
             }
             dft<R>(v[p]);
-            dst[p] = ((j / Ns) * Ns * R + k) * CP + c;
+            dst[p] = ((j / Ns) * Ns * R + k) * CP + c * CS;
         }
     }
     __syncthreads();
@@ -115,13 +115,14 @@ __device__ __forceinline__ void stage(float2 *buf, const float2 *__restrict__ tw
 
 // First and last stage of a column FFT straight from and to global memory: the
 // first stage (span 1, radix R, no twiddles) reads its R inputs of butterfly b from
-// base[n*nstride + c] (c clamped to the cw columns present; the copies of the last
+// base[n*nstride + c*cstride] (c clamped to the cw columns present; the copies of the last
 // column in the others are never stored) and writes the LDS block; the last stage
 // reads the LDS block and stores its outputs of the columns c < cw, returning the
 // largest |Re|, |Im| it stored.  Same butterflies and twiddles as stage<>, so the
 // same bits as staging the whole block through LDS.
 template <int N, int C, int CP, int R, int BLK>
-__device__ __forceinline__ void stage_first(const float2 *base, long long nstride, int cw, float2 *buf) {
+__device__ __forceinline__ void stage_first(const float2 *base, long long nstride, long long cstride, int cw,
+                                            float2 *buf) {
     constexpr int NB = (N / R) * C;
     constexpr int PER = (NB + BLK - 1) / BLK;
     float2 v[PER][R];
@@ -130,7 +131,7 @@ __device__ __forceinline__ void stage_first(const float2 *base, long long nstrid
         const int b = min((int)threadIdx.x + p * BLK, NB - 1);
         const int c = b % C, j = b / C;
 #pragma unroll
-        for (int m = 0; m < R; ++m) v[p][m] = base[(long long)(j + m * (N / R)) * nstride + min(c, cw - 1)];
+        for (int m = 0; m < R; ++m) v[p][m] = base[(long long)(j + m * (N / R)) * nstride + min(c, cw - 1) * cstride];
     }
 #pragma unroll
     for (int p = 0; p < PER; ++p) {
@@ -145,9 +146,9 @@ __device__ __forceinline__ void stage_first(const float2 *base, long long nstrid
     __syncthreads();
 }
 
-template <int N, int C, int CP, int R, int BLK>
+template <int N, int C, int CP, int R, int BLK, int CS = 1>
 __device__ __forceinline__ float stage_last(const float2 *buf, const float2 *__restrict__ tw, int Ns,
-                                            float2 *base, long long nstride, int cw) {
+                                            float2 *base, long long nstride, long long cstride, int cw) {
     constexpr int NB = (N / R) * C;
     constexpr int PER = (NB + BLK - 1) / BLK;
     float mx = 0.0f;
@@ -161,7 +162,7 @@ __device__ __forceinline__ float stage_last(const float2 *buf, const float2 *__r
             float2 v[R];
 #pragma unroll
             for (int m = 0; m < R; ++m) {
-                float2 x = buf[(j + m * (N / R)) * CP + c];
+                float2 x = buf[(j + m * (N / R)) * CP + c * CS];
                 if (m > 0) x = cmul(x, tw[(m * tstep) & (N - 1)]);
                 v[m] = x;
             }
@@ -170,7 +171,7 @@ __device__ __forceinline__ float stage_last(const float2 *buf, const float2 *__r
                 const int d = (j / Ns) * Ns * R + k;
 #pragma unroll
                 for (int m = 0; m < R; ++m) {
-                    base[(long long)(d + m * Ns) * nstride + c] = v[m];
+                    base[(long long)(d + m * Ns) * nstride + c * cstride] = v[m];
                     mx = fmaxf(mx, fmaxf(fabsf(v[m].x), fabsf(v[m].y)));
                 }
             }
@@ -183,10 +184,10 @@ __device__ __forceinline__ float stage_last(const float2 *buf, const float2 *__r
 // memory (stage_first, stage_last); radix-8 stages in between, the last stage of
 // radix 8, 4 or 2.
 template <int N, int C, int BLK>
-__device__ __forceinline__ float fft_columns_global(float2 *base, long long nstride, int cw, float2 *buf,
-                                                    const float2 *__restrict__ tw) {
+__device__ __forceinline__ float fft_columns_global(float2 *base, long long nstride, long long cstride, int cw,
+                                                    float2 *buf, const float2 *__restrict__ tw) {
     constexpr int RL = (N == 16 || N == 128 || N == 1024) ? 2 : (N == 32 || N == 256) ? 4 : 8;
-    stage_first<N, C, C, 8, BLK>(base, nstride, cw, buf);
+    stage_first<N, C, C, 8, BLK>(base, nstride, cstride, cw, buf);
     int Ns = 8;
 #pragma unroll
     for (int s = 0; s < 3; ++s) {
@@ -195,7 +196,7 @@ __device__ __forceinline__ float fft_columns_global(float2 *base, long long nstr
             Ns *= 8;
         }
     }
-    return stage_last<N, C, C, RL, BLK>(buf, tw, Ns, base, nstride, cw);
+    return stage_last<N, C, C, RL, BLK>(buf, tw, Ns, base, nstride, cstride, cw);
 }
 
 template <int N, int C, int CP, int BLK>
@@ -216,7 +217,10 @@ __device__ __forceinline__ void fft_columns(float2 *buf, const float2 *__restric
 
 // In-place FFT of length N along one axis of a batch of complex arrays:
 // element n of column (o, z) of batch b at data[b*bstride + o*ostride + n*nstride + z],
-// z in [0, zlen).  Grid: (ceil(zlen/C), nother, nbatch).
+// z in [0, zlen).  One workgroup per C columns of one o, but for a last column that
+// would be alone in its group (zlen = N/2+1): the first nlast workgroups take that column
+// of C neighbouring o each (nlast = ceil(nother/C) * nbatch, 0: no such column), instead
+// of a fifth (N = 128) to a seventeenth (512) of the workgroups working on one column.
 // amax (optional, the last pass): the largest |Re| or |Im| of the transform of cube
 // b, as float bits, atomically maxed into one of 64 words amax[b*64 + (group & 63)]
 // (an integer max, so the words do not depend on the order of the atomics).
@@ -235,25 +239,40 @@ __device__ __forceinline__ void block_absmax(float m, unsigned *__restrict__ ama
 template <int N, int C, int BLK>
 __global__ void __launch_bounds__(BLK)
 fft_col_kernel(float2 *__restrict__ data, long long nstride, long long ostride, long long bstride,
-               int zlen, int nother, const float2 *__restrict__ tw, unsigned *__restrict__ amax) {
+               int zlen, int nother, int nlast, const float2 *__restrict__ tw, unsigned *__restrict__ amax) {
     static_assert((N * C) % BLK == 0, "block shape");
     __shared__ float2 buf[N * C];
-    // Workgroups are dealt to the 8 XCDs round-robin by launch index, and each
-    // XCD has its own L2.  Rows are 8*zlen bytes long, so a group's 128-byte
-    // column segment straddles two cache lines shared with the neighbouring
-    // column groups: logical index w puts all column groups of one line set on
-    // the same XCD, next to each other in time, and the shared lines are
-    // fetched from HBM once.
-    const unsigned ngz = (unsigned)((zlen + C - 1) / C);
-    const unsigned total = gridDim.x, per = total / 8u;
     const unsigned L = blockIdx.x;
-    const unsigned w = (L < per * 8u) ? (L % 8u) * per + L / 8u : L;
-    const unsigned zg = w % ngz, t = w / ngz;
-    const unsigned line = t % (unsigned)nother, b = t / (unsigned)nother;
-    const int z0 = (int)zg * C;
-    const int cw = min(C, zlen - z0);
-    float2 *base = data + (long long)b * bstride + (long long)line * ostride + z0;
-    const float m = fft_columns_global<N, C, BLK>(base, nstride, cw, buf, tw);
+    float2 *base;
+    long long cstride;
+    int cw;
+    unsigned b;
+    if (L < (unsigned)nlast) {
+        const unsigned per = ((unsigned)nother + C - 1) / C;
+        b = L / per;
+        const unsigned o0 = (L - b * per) * C;
+        base = data + (long long)b * bstride + (long long)o0 * ostride + (zlen - 1);
+        cstride = ostride;
+        cw = min(C, nother - (int)o0);
+    } else {
+        // Workgroups are dealt to the 8 XCDs round-robin by launch index, and each
+        // XCD has its own L2.  With dense rows (8*zlen bytes) a group's 128-byte
+        // column segment straddles two cache lines shared with the neighbouring
+        // column groups: logical index w puts all column groups of one line set on
+        // the same XCD, next to each other in time, and the shared lines are
+        // fetched from HBM once.
+        const unsigned ngz = (unsigned)(nlast ? (zlen - 1) / C : (zlen + C - 1) / C);
+        const unsigned total = gridDim.x - (unsigned)nlast, per = total / 8u, l = L - (unsigned)nlast;
+        const unsigned w = (l < per * 8u) ? (l % 8u) * per + l / 8u : l;
+        const unsigned zg = w % ngz, t = w / ngz;
+        const unsigned line = t % (unsigned)nother;
+        b = t / (unsigned)nother;
+        const int z0 = (int)zg * C;
+        base = data + (long long)b * bstride + (long long)line * ostride + z0;
+        cstride = 1;
+        cw = min(C, zlen - z0);
+    }
+    const float m = fft_columns_global<N, C, BLK>(base, nstride, cstride, cw, buf, tw);
     if (amax) block_absmax(m, amax, b * 64u + (L & 63u));
 }
 
@@ -287,6 +306,26 @@ absmax_kernel(const float2 *__restrict__ dk, long long nrows, int zlen, long lon
 // 0.21 ms beside this kernel's 0.25) and, for a batch with scales, the prologue's own
 // pass over it (32 x 2 x 128^3: 0.34 + 0.25 ms) were pure extra traffic.  Pk of a 512^3
 // field on the GPU: 1.41 -> 1.18 ms, the batch of 32: 5.66 -> 5.20 ms.
+__device__ __forceinline__ void row_prologue(const RowSrc &rs, int field, int real, float2 *v, int n) {
+    if (!rs.apply) return;                                // uniform: (x / scale) - shift in float32
+    const int si = field * rs.sfield + real * rs.sreal;
+    const float scale = rs.scales ? rs.scales[si] : rs.scale;
+    const float shift = rs.shifts ? rs.shifts[si] : rs.shift;
+#pragma unroll
+    for (int p = 0; p < n; ++p) {
+        v[p].x = v[p].x / scale - shift;
+        v[p].y = v[p].y / scale - shift;
+    }
+}
+
+// X[k] of a = Z[k], b = Z[N/2 - k], w = e^{-2 pi i k/N}.
+__device__ __forceinline__ float2 split_mode(float2 a, float2 b, float2 w) {
+    const float2 e = make_float2(0.5f * (a.x + b.x), 0.5f * (a.y - b.y));
+    // O = -i/2 (a - conj(b)) = ((a.y + b.y)/2, -(a.x - b.x)/2)
+    const float2 o = make_float2(0.5f * (a.y + b.y), -0.5f * (a.x - b.x));
+    return cadd(e, cmul(w, o));
+}
+
 template <int N, int R>
 __global__ void __launch_bounds__(kFftBlock)
 fft_r2c_rows_kernel(RowSrc rs, float2 *__restrict__ out, long long nrows,
@@ -312,16 +351,7 @@ fft_r2c_rows_kernel(RowSrc rs, float2 *__restrict__ out, long long nrows,
         const int r = min(t / H, rw - 1);
         v[p] = src[(long long)r * H + t % H];
     }
-    if (rs.apply) {                                       // uniform: (x / scale) - shift in float32
-        const int si = field * rs.sfield + real * rs.sreal;
-        const float scale = rs.scales ? rs.scales[si] : rs.scale;
-        const float shift = rs.shifts ? rs.shifts[si] : rs.shift;
-#pragma unroll
-        for (int p = 0; p < PER; ++p) {
-            v[p].x = v[p].x / scale - shift;
-            v[p].y = v[p].y / scale - shift;
-        }
-    }
+    row_prologue(rs, field, real, v, PER);
 #pragma unroll
     for (int p = 0; p < PER; ++p) {
         const int t = threadIdx.x + p * kFftBlock;
@@ -336,12 +366,59 @@ fft_r2c_rows_kernel(RowSrc rs, float2 *__restrict__ out, long long nrows,
         if (r >= rw) continue;
         const float2 a = buf[(k % H) * RP + r];
         const float2 b = buf[((H - k) % H) * RP + r];     // Z[N/2 - k]
-        const float2 e = make_float2(0.5f * (a.x + b.x), 0.5f * (a.y - b.y));
-        // O = -i/2 (a - conj(b)) = ((a.y + b.y)/2, -(a.x - b.x)/2)
-        const float2 o = make_float2(0.5f * (a.y + b.y), -0.5f * (a.x - b.x));
-        const float2 w = tw_full[k];                      // k <= N/2 < N
-        dst[(long long)r * zs + k] = cadd(e, cmul(w, o));
+        dst[(long long)r * zs + k] = split_mode(a, b, tw_full[k]);   // k <= N/2 < N
     }
+}
+
+// The z and y passes of one x plane in LDS (N = 64, 128): the N rows are transformed as
+// in fft_r2c_rows_kernel (rows along the second index of buf), split into their N/2+1
+// modes in place (mode k and N/2 - k by one thread; mode N/2 gets a row of its own), and
+// the N/2+1 columns along y as in fft_col_kernel, with the same butterflies, twiddles and
+// order of stages, so the same bits.  One pass over HBM in place of two.  The odd row
+// stride keeps both directions free of bank conflicts.  32 x 2 cubes of 128^3: the three
+// passes 820 us, this one and the x pass 572 (a workgroup of 512: 650); one 64^3 field:
+// 15.9 -> 12.4 us and a launch less (256 threads: 13.5).  A larger plane does not fit
+// in LDS, a smaller one would leave a workgroup little to do.  Launching both passes on
+// 64 to 160 MB of cubes at a time, so that the second finds the first one's output in
+// the memory-side cache, gained less than the extra launches' tails cost (610 to 670 us).
+template <int N>
+constexpr int kPlaneBlock = N == 128 ? 1024 : 512;
+
+template <int N>
+__global__ void __launch_bounds__(kPlaneBlock<N>)
+fft_r2c_planes_kernel(RowSrc rs, float2 *__restrict__ out, const float2 *__restrict__ tw_half,
+                      const float2 *__restrict__ tw_full, long long zs) {
+    constexpr int H = N / 2, RP = N + 1, BLK = kPlaneBlock<N>;
+    constexpr int PER = N * H / BLK;
+    static_assert(PER * BLK == N * H, "block shape");
+    constexpr int RL = N == 128 ? 2 : 8;
+    __shared__ float2 buf[(H + 1) * RP];
+    const long long plane = blockIdx.x;
+    const int cube = (int)(plane / N);                    // field * nreal + realisation
+    const int field = cube / rs.nreal, real = cube - field * rs.nreal;
+    for (int i = blockIdx.x * BLK + threadIdx.x; i < rs.nzero; i += gridDim.x * BLK) rs.zero[i] = 0u;
+    const float2 *src = (const float2 *)(rs.in[field] + ((long long)real * N + plane % N) * (N * N));
+    float2 v[PER];
+#pragma unroll
+    for (int p = 0; p < PER; ++p) v[p] = src[threadIdx.x + p * BLK];
+    row_prologue(rs, field, real, v, PER);
+#pragma unroll
+    for (int p = 0; p < PER; ++p) {
+        const int t = threadIdx.x + p * BLK;
+        buf[(t % H) * RP + t / H] = v[p];
+    }
+    __syncthreads();
+    fft_columns<H, N, RP, BLK>(buf, tw_half);
+    for (int t = threadIdx.x; t < (H / 2 + 1) * N; t += BLK) {
+        const int k = t / N, r = t % N;
+        const float2 a = buf[k * RP + r], b = buf[((H - k) % H) * RP + r];
+        buf[k * RP + r] = split_mode(a, b, tw_full[k]);
+        if (k != H / 2) buf[(H - k) * RP + r] = split_mode(b, a, tw_full[H - k]);
+    }
+    __syncthreads();
+    stage<N, H + 1, 1, 8, BLK, RP, true>(buf, tw_full, 1);
+    if constexpr (N == 128) stage<N, H + 1, 1, 8, BLK, RP>(buf, tw_full, 8);
+    stage_last<N, H + 1, 1, RL, BLK, RP>(buf, tw_full, N / RL, out + plane * (N * zs), zs, 1, H + 1);
 }
 
 template <int N>
@@ -349,11 +426,13 @@ int launch_cols(Ctx *c, float2 *data, long long nstride, long long ostride, long
                 int zlen, int nother, int nbatch, const float2 *tw, unsigned *amax) {
     // 16 complex (128 B) contiguous per point; 64 KB of LDS at most
     constexpr int C = (N >= 1024) ? 8 : 16;
-    constexpr int BLK = (N >= 512) ? 512 : 256;
-    const long long nwg = (long long)ceil_div(zlen, C) * nother * nbatch;
+    constexpr int BLK = (N >= 1024) ? 1024 : (N >= 512) ? 512 : 256;
+    const bool alone = zlen > C && zlen % C == 1;
+    const long long nlast = alone ? (long long)ceil_div(nother, C) * nbatch : 0;
+    const long long nwg = (long long)(alone ? zlen / C : ceil_div(zlen, C)) * nother * nbatch + nlast;
     PYL_CHECK(nwg < (1ll << 31), PYL_EINVAL, "FFT column launch too large (%lld workgroups)", nwg);
     fft_col_kernel<N, C, BLK><<<(unsigned)nwg, BLK, 0, c->stream>>>(data, nstride, ostride, bstride,
-                                                                     zlen, nother, tw, amax);
+                                                                     zlen, nother, (int)nlast, tw, amax);
     PYL_HIP(hipGetLastError());
     return PYL_OK;
 }
@@ -383,19 +462,27 @@ int launch_rows(Ctx *c, const RowSrc &in, float2 *out, long long nrows, const fl
     return PYL_OK;
 }
 
+// (sides of 64 and 128 take launch_planes)
 int rows(Ctx *c, int n, const RowSrc &in, float2 *out, long long nrows, const float2 *twh,
          const float2 *twf, long long zs) {
     switch (n) {
         case 16: return launch_rows<16>(c, in, out, nrows, twh, twf, zs);
         case 32: return launch_rows<32>(c, in, out, nrows, twh, twf, zs);
-        case 64: return launch_rows<64>(c, in, out, nrows, twh, twf, zs);
-        case 128: return launch_rows<128>(c, in, out, nrows, twh, twf, zs);
         case 256: return launch_rows<256>(c, in, out, nrows, twh, twf, zs);
         case 512: return launch_rows<512>(c, in, out, nrows, twh, twf, zs);
         case 1024: return launch_rows<1024>(c, in, out, nrows, twh, twf, zs);
     }
     set_error("no row FFT of length %d", n);
     return PYL_EINVAL;
+}
+
+template <int N>
+int launch_planes(Ctx *c, const RowSrc &in, float2 *out, long long nplanes, const float2 *twh,
+                  const float2 *twf, long long zs) {
+    PYL_CHECK(nplanes < (1ll << 31), PYL_EINVAL, "FFT plane launch too large (%lld workgroups)", nplanes);
+    fft_r2c_planes_kernel<N><<<(unsigned)nplanes, kPlaneBlock<N>, 0, c->stream>>>(in, out, twh, twf, zs);
+    PYL_HIP(hipGetLastError());
+    return PYL_OK;
 }
 
 }  // namespace
@@ -463,8 +550,9 @@ int fft_r2c_fields(Ctx *c, const FieldSrc &fs, float2 *out, int dims, long long 
     const float2 *tw = nullptr, *twh = nullptr;
     PYL_TRY(get_twiddles(c, dims, &tw));
     PYL_TRY(get_twiddles(c, dims / 2, &twh));
-    // z: real rows -> half-complex rows (zs apart); kRowFields fields per launch
-    for (int f0 = 0; f0 < fs.nfields; f0 += kRowFields) {
+    const long long plane = N * zs, cube = N * plane;
+    const bool planes2d = N == 64 || N == 128;
+    for (int f0 = 0; f0 < fs.nfields; f0 += kRowFields) {     // kRowFields fields per launch
         RowSrc rs{};
         const int nf = std::min(kRowFields, fs.nfields - f0);
         for (int f = 0; f < nf; ++f) rs.in[f] = fs.in[f0 + f];
@@ -478,12 +566,21 @@ int fft_r2c_fields(Ctx *c, const FieldSrc &fs, float2 *out, int dims, long long 
         rs.sreal = fs.sreal;
         rs.zero = amax;
         rs.nzero = (amax && f0 == 0) ? (int)(64 * batch) : 0;
-        PYL_TRY(rows(c, dims, rs, out + (long long)f0 * fs.nreal * N * N * zs, N * N * fs.nreal * nf, twh, tw, zs));
+        const long long c0 = (long long)f0 * fs.nreal;
+        const int ncube = fs.nreal * nf;
+        float2 *o = out + c0 * cube;
+        // z: real rows -> half-complex rows (zs apart);
+        // y: n = y (stride zs), other = x planes; Z columns of each row
+        if (planes2d) {
+            PYL_TRY(N == 64 ? launch_planes<64>(c, rs, o, N * ncube, twh, tw, zs)
+                            : launch_planes<128>(c, rs, o, N * ncube, twh, tw, zs));
+        } else {
+            PYL_TRY(rows(c, dims, rs, o, N * N * ncube, twh, tw, zs));
+            PYL_TRY(cols(c, dims, o, zs, plane, cube, (int)Z, dims, ncube, tw));
+        }
+        // x: n = x (stride plane), other = y (stride zs)
+        PYL_TRY(cols(c, dims, o, plane, zs, cube, (int)Z, dims, ncube, tw, amax ? amax + 64 * c0 : nullptr));
     }
-    // y: n = y (stride zs), other = x (stride N*zs); Z columns of each row
-    PYL_TRY(cols(c, dims, out, zs, N * zs, N * N * zs, (int)Z, dims, (int)batch, tw));
-    // x: n = x (stride N*zs), other = y (stride zs)
-    PYL_TRY(cols(c, dims, out, N * zs, zs, N * N * zs, (int)Z, dims, (int)batch, tw, amax));
     return PYL_OK;
 }
 
