@@ -198,6 +198,7 @@ int get_bin_plan(Ctx *c, int dims, int axis, int nreal, BinPlan **out) {
     // an exact bin sum's low word takes at most kFixMaxAdds additions: one per run of
     // kRun modes of the item's groups
     G = std::max(1, std::min(G, kFixMaxAdds / runs_per_group));
+    const ModePlan *mp = get_mode_plan(c, dims, axis);
     SharedTables &st = shared_tables();
     std::lock_guard<std::mutex> lk(st.mu);
     const auto key = std::make_tuple(c->device, dims, axis, G);
@@ -239,6 +240,7 @@ int get_bin_plan(Ctx *c, int dims, int axis, int nreal, BinPlan **out) {
         (void)hipFree(bp.d_groups);
         (void)hipFree(bp.d_items);
         (void)hipFree(bp.d_key_items);
+        (void)hipFree(bp.d_n2);
         set_error("binning plan upload failed: %s", hipGetErrorString(e));
         return e == hipErrorOutOfMemory ? PYL_ENOMEM : PYL_EHIP;
     };
@@ -246,6 +248,10 @@ int get_bin_plan(Ctx *c, int dims, int axis, int nreal, BinPlan **out) {
     if ((e = hipMalloc(&bp.d_groups, groups.size() * sizeof(int))) != hipSuccess) return fail(e);
     if ((e = hipMalloc(&bp.d_items, items.size() * sizeof(int4))) != hipSuccess) return fail(e);
     if ((e = hipMalloc(&bp.d_key_items, key_items.size() * sizeof(int))) != hipSuccess) return fail(e);
+    if ((e = hipMalloc(&bp.d_n2, mp->N2D.size() * sizeof(double))) != hipSuccess) return fail(e);
+    if ((e = hipMemcpy(bp.d_n2, mp->N2D.data(), mp->N2D.size() * sizeof(double), hipMemcpyHostToDevice)) !=
+        hipSuccess)
+        return fail(e);
     if ((e = hipMemcpy(bp.d_groups, groups.data(), groups.size() * sizeof(int), hipMemcpyHostToDevice)) !=
         hipSuccess)
         return fail(e);
@@ -633,6 +639,8 @@ struct ReduceArgs {
     const int *phi;
     const int *key_items;
     const int *escale;
+    const double *n2;        // mode counts of the 2D bins
+    double fact;             // (BoxSize / dims^2)^3
     double *out3, *out2, *out1;
     int nitems, nkeys, n3, na3, L2, L1, S, P, off2, off1, axis, kmax_par, nreal;
     long long nb2, n1;       // out2 / out1 elements per realisation (nb2*S, (m+1)*S)
@@ -647,7 +655,9 @@ struct ReduceArgs {
 //    in the output);
 //  * g1 blocks: axes 0/1, the 1D bins (k_par = key).
 // The outputs go straight into the pinned host buffer the caller reads after the
-// stream, in runs of whole cache lines.  Latency-bound: the chunk sums, their sum, the
+// stream, in runs of whole cache lines; the 2D bins, the bulk of them, as the spectra
+// themselves (sum * fact / modes: on the host their divisions took the GPU's time of
+// 10 % of an XPk of two 256^3 fields), the others as sums.  Latency-bound: the chunk sums, their sum, the
 // 1D line's own pair of launches (axis 2) and the download used to take 36 us at 64^3
 // and 46 us at 512^3 for microseconds of data movement; now 4 and 28 us, and Pk of a 64^3
 // field went from 98 to 70 us, of a 512^3 field from 1084 to 1057 us.
@@ -719,7 +729,7 @@ pk_reduce_kernel(ReduceArgs a, int g3, int g2) {
             const long long i = (long long)x * kRedBlock + t;     // (key, line entry, spectrum)
             if (i >= (long long)a.nkeys * ncol) return;
             reduce_key_items(a, (int)(i / ncol), a.off2 + (int)(i % ncol), base, lo, hi);
-            out2[i] = fix_value(lo, hi, E);                       // (kmax_par+1) == L2
+            out2[i] = fix_value(lo, hi, E) * a.fact / a.n2[i / a.S];   // (kmax_par+1) == L2
             return;
         }
         const int tc = red_tile_cols(a.S), nct = (ncol + tc - 1) / tc;
@@ -734,8 +744,10 @@ pk_reduce_kernel(ReduceArgs a, int g3, int g2) {
         if (t >= 32 * tc) return;
         const int l = t / (32 * a.S), rest = t - l * 32 * a.S, kl = rest / a.S, sp = rest - kl * a.S;
         const int cl = l * a.S + sp;
-        if (k0 + kl < a.nkeys && c0 + cl < ncol)
-            out2[((long long)(a.kmax_par + 1) * (c0 / a.S + l) + k0 + kl) * a.S + sp] = tile[kl][cl];
+        if (k0 + kl < a.nkeys && c0 + cl < ncol) {
+            const long long bin = (long long)(a.kmax_par + 1) * (c0 / a.S + l) + k0 + kl;
+            out2[bin * a.S + sp] = tile[kl][cl] * a.fact / a.n2[bin];
+        }
     } else {
         const int bb = b - g3 - g2, xb = (a.nkeys * a.S + kRedBlock - 1) / kRedBlock, r = bb / xb;
         const int i = (bb - r * xb) * kRedBlock + t;
@@ -793,7 +805,7 @@ struct HostAcc {
     int S_total;
     std::vector<double> P3;     // [(kmax+1)*3*S_total] l-major per bin: (bin*3+l)*S_total+s
     std::vector<double> phase;  // [kmax+1]
-    std::vector<double> P2;     // [nb2*S_total]
+    std::vector<double> P2;     // [nb2*S_total], normalised (pk_reduce_kernel)
     std::vector<double> P1;     // [(m+1)*S_total]
     // the 2D and 1D sums to finalize: P2/P1, or the pinned download itself when one
     // launch produced every spectrum in output order (no copy of the 2D bins)
@@ -847,7 +859,7 @@ template <int AXIS, int NFL, bool PHASE>
 int launch_bin(Ctx *c, const BinPlan *bp, const PkDims &p, const float2 *const *dk,
                long long fstride, long long zs, int nreal, const double *const *corr,
                const float *cmax, const unsigned *const *amax, const AccsPtr &accs,
-               const int *spec_out) {
+               const int *spec_out, double fact, const std::function<int()> &meanwhile) {
     constexpr int S = Spec<NFL>::S;
     constexpr int NA3 = 3 * S + (PHASE ? 1 : 0);
     const int L2 = (AXIS == 2) ? p.zlen : p.kmax_per + 1;
@@ -912,6 +924,7 @@ int launch_bin(Ctx *c, const BinPlan *bp, const PkDims &p, const float2 *const *
     PYL_HIP(hipGetLastError());
     ReduceArgs r{};
     r.plo = plo; r.phi = phi; r.escale = escale;
+    r.n2 = bp->d_n2; r.fact = fact;
     r.key_items = bp->d_key_items; r.out3 = h3; r.out2 = h2; r.out1 = h1;
     r.nitems = bp->nitems; r.nkeys = bp->nkeys; r.n3 = n3; r.na3 = PHASE ? NA3 : 0;
     r.L2 = L2; r.L1 = L1; r.S = S; r.P = P; r.off2 = off2; r.off1 = off1; r.axis = AXIS;
@@ -926,7 +939,9 @@ int launch_bin(Ctx *c, const BinPlan *bp, const PkDims &p, const float2 *const *
     pk_reduce_kernel<<<(unsigned)(g3 + g2 + g1), kRedBlock, 0, c->stream>>>(r, (int)g3, (int)g2);
     PYL_HIP(hipGetLastError());
     PYL_TRY(stage_end(c, PYL_STAGE_PK_BIN));
+    const int rc = meanwhile();               // host work beside the transform and the binning
     if (c->capturing) {
+        PYL_TRY(rc);
         std::array<int, Spec<NFL>::S> so;
         for (int sp = 0; sp < Spec<NFL>::S; ++sp) so[sp] = spec_out[sp];
         const double *h = (const double *)hp;
@@ -938,6 +953,7 @@ int launch_bin(Ctx *c, const BinPlan *bp, const PkDims &p, const float2 *const *
         return PYL_OK;
     }
     PYL_HIP(hipStreamSynchronize(c->stream));
+    PYL_TRY(rc);
     bin_host_part<NFL, PHASE>(p, (const double *)hp, out3, out2, out1, nreal, spec_out, *accs);
     return PYL_OK;
 }
@@ -946,15 +962,22 @@ template <int NFL, bool PHASE>
 int launch_bin_axis(Ctx *c, int axis, const BinPlan *bp, const PkDims &p, const float2 *const *dk,
                     long long fstride, long long zs, int nreal, const double *const *corr,
                     const float *cmax, const unsigned *const *amax, const AccsPtr &accs,
-                    const int *spec_out) {
+                    const int *spec_out, double fact, const std::function<int()> &meanwhile) {
     if (axis == 0)
-        return launch_bin<0, NFL, PHASE>(c, bp, p, dk, fstride, zs, nreal, corr, cmax, amax, accs, spec_out);
+        return launch_bin<0, NFL, PHASE>(c, bp, p, dk, fstride, zs, nreal, corr, cmax, amax, accs, spec_out, fact,
+                                         meanwhile);
     if (axis == 1)
-        return launch_bin<1, NFL, PHASE>(c, bp, p, dk, fstride, zs, nreal, corr, cmax, amax, accs, spec_out);
-    return launch_bin<2, NFL, PHASE>(c, bp, p, dk, fstride, zs, nreal, corr, cmax, amax, accs, spec_out);
+        return launch_bin<1, NFL, PHASE>(c, bp, p, dk, fstride, zs, nreal, corr, cmax, amax, accs, spec_out, fact,
+                                         meanwhile);
+    return launch_bin<2, NFL, PHASE>(c, bp, p, dk, fstride, zs, nreal, corr, cmax, amax, accs, spec_out, fact,
+                                     meanwhile);
 }
 
 // Normalisation, Pk_library.pyx:384-418 (and :735-791 for XPk).
+double pk_fact(const PkDims &p, double BoxSize) {
+    return std::pow(BoxSize / ((double)p.dims * (double)p.dims), 3.0);
+}
+
 // The outputs that depend only on the mode plan (k, bin centres, mode counts):
 // filled while the GPU still transforms and bins.
 int finalize_modes(const ModePlan *mp, const PkDims &p, double BoxSize, pyl_pk_out *out) {
@@ -986,14 +1009,14 @@ int finalize_modes(const ModePlan *mp, const PkDims &p, double BoxSize, pyl_pk_o
     return PYL_OK;
 }
 
-// The spectra (Pk_library.pyx:384-418): 1D drops the DC bin, 2D keeps every bin,
-// 3D drops the DC bin with the multipoles times (2l+1).
+// The spectra (Pk_library.pyx:384-418): 1D drops the DC bin, 2D keeps every bin
+// (normalised where they were reduced), 3D drops the DC bin with the multipoles times (2l+1).
 void finalize_values(const ModePlan *mp, const PkDims &p, double BoxSize, const HostAcc &acc,
                      bool want_phase, pyl_pk_out *out) {
     const int S = acc.S_total;
     const double kF = 2.0 * M_PI / BoxSize;
     const double kN = p.m * kF;
-    const double fact = std::pow(BoxSize / ((double)p.dims * (double)p.dims), 3.0);
+    const double fact = pk_fact(p, BoxSize);
     if (out->Pk1D)
         for (int i = 1; i <= p.m; ++i) {
             const double N = mp->N1D[i];
@@ -1005,19 +1028,7 @@ void finalize_values(const ModePlan *mp, const PkDims &p, double BoxSize, const 
                 out->Pk1D[(size_t)(i - 1) * S + s] = v;
             }
         }
-    if (out->Pk2D) {
-        // (the 2D bins are the bulk of the host work: a restrict-qualified loop that
-        // the host compiler vectorizes for one spectrum)
-        double *__restrict__ o2 = out->Pk2D;
-        const double *__restrict__ s2 = acc.P2v;
-        const double *__restrict__ n2 = mp->N2D.data();
-        if (S == 1) {
-            for (long long i = 0; i < p.nb2; ++i) o2[i] = s2[i] * fact / n2[i];
-        } else {
-            for (long long i = 0; i < p.nb2; ++i)
-                for (int s = 0; s < S; ++s) o2[(size_t)i * S + s] = s2[(size_t)i * S + s] * fact / n2[i];
-        }
-    }
+    if (out->Pk2D) std::memcpy(out->Pk2D, acc.P2v, sizeof(double) * (size_t)p.nb2 * S);
     for (int b = 1; b <= p.kmax; ++b) {
         const double N = mp->N3D[b];
         if (out->Pk3D)
@@ -1093,8 +1104,8 @@ int fft_fields_device(Ctx *c, const float *const *deltas, FieldSrc fs, bool dev,
 // Binning of F device half-complex fields of nreal realisations -> finalized outputs.
 // Field f of realisation r is dk[f] + r*fstride.
 // Device-resident MAS correction table for (dims, p), built once per device with the
-// host's libm.
-int get_mas_tab(Ctx *c, int dims, int p, const double **out) {
+// host's libm; cmax: the largest product of three axis corrections, rounded up.
+int get_mas_tab(Ctx *c, int dims, int p, const double **out, float *cmax) {
     SharedTables &st = shared_tables();
     std::lock_guard<std::mutex> lk(st.mu);
     const auto key = std::make_tuple(c->device, dims, p);
@@ -1111,9 +1122,12 @@ int get_mas_tab(Ctx *c, int dims, int p, const double **out) {
             set_error("MAS table upload failed: %s", hipGetErrorString(e));
             return PYL_EHIP;
         }
-        it = st.mas.emplace(key, d).first;
+        double mx = 1.0;
+        for (double v : tab) mx = std::max(mx, v);
+        it = st.mas.emplace(key, std::make_pair(d, (float)(mx * mx * mx * 1.001))).first;
     }
-    *out = (const double *)it->second;
+    *out = (const double *)it->second.first;
+    *cmax = it->second.second;
     return PYL_OK;
 }
 
@@ -1131,16 +1145,16 @@ int pk_bin_device(Ctx *c, const float2 *const *dk, long long fstride, long long 
     std::vector<const double *> tab(F);
     std::vector<float> cmax(F);
     for (int f = 0; f < F; ++f) {
-        PYL_TRY(get_mas_tab(c, dims, mas[f], &tab[f]));
-        // the largest product of three axis corrections, rounded up
-        std::vector<double> h(dims);
-        mas_table(dims, mas[f], h.data());
-        double mx = 1.0;
-        for (double v : h) mx = std::max(mx, v);
-        cmax[f] = (float)(mx * mx * mx * 1.001);
+        PYL_TRY(get_mas_tab(c, dims, mas[f], &tab[f], &cmax[f]));
     }
-    // the mode-plan outputs are written while the FFT already queued runs
-    for (int r = 0; r < nreal; ++r) PYL_TRY(finalize_modes(mp, p, BoxSize, &outs[r]));
+    // the mode-plan outputs are written while the GPU works, after the first launch
+    bool modes_done = false;
+    const std::function<int()> meanwhile = [&]() {
+        for (int r = 0; r < nreal && !modes_done; ++r) PYL_TRY(finalize_modes(mp, p, BoxSize, &outs[r]));
+        modes_done = true;
+        return (int)PYL_OK;
+    };
+    const double fact = pk_fact(p, BoxSize);
     const int S = F + F * (F - 1) / 2;
     // host accumulators reused across calls on this thread (no fresh pages per call);
     // a captured call keeps its own, used by the host steps of every replay
@@ -1171,9 +1185,11 @@ int pk_bin_device(Ctx *c, const float2 *const *dk, long long fstride, long long 
         const unsigned *a0[1] = {amax[0]};
         int so[1] = {0};
         if (phase)
-            PYL_TRY((launch_bin_axis<1, true>(c, axis, bp, p, f0, fstride, zs, nreal, c0, m0, a0, accs_p, so)));
+            PYL_TRY((launch_bin_axis<1, true>(c, axis, bp, p, f0, fstride, zs, nreal, c0, m0, a0, accs_p, so,
+                                              fact, meanwhile)));
         else
-            PYL_TRY((launch_bin_axis<1, false>(c, axis, bp, p, f0, fstride, zs, nreal, c0, m0, a0, accs_p, so)));
+            PYL_TRY((launch_bin_axis<1, false>(c, axis, bp, p, f0, fstride, zs, nreal, c0, m0, a0, accs_p, so,
+                                               fact, meanwhile)));
     } else {
         // pairs i<j in lexicographic order; each launch yields auto i, auto j, cross ij
         std::vector<bool> have(F, false);
@@ -1187,7 +1203,7 @@ int pk_bin_device(Ctx *c, const float2 *const *dk, long long fstride, long long 
                 int so[3] = {have[i] ? -1 : i, have[j] ? -1 : j, F + xi};
                 have[i] = have[j] = true;
                 PYL_TRY((launch_bin_axis<2, false>(c, axis, bp, p, fp, fstride, zs, nreal, cp, mp2, ap,
-                                                   accs_p, so)));
+                                                   accs_p, so, fact, meanwhile)));
             }
     }
     if (c->capturing) {

@@ -99,6 +99,7 @@ struct BinPlan {
     int *d_groups = nullptr;     // |kx| << 16 | |ky|, ordered by key
     int4 *d_items = nullptr;     // (first group, ngroups, key, 0)
     int *d_key_items = nullptr;  // [nkeys+1] item range of each key
+    double *d_n2 = nullptr;      // mode counts of the 2D bins (ModePlan::N2D)
 };
 
 enum BufId {
@@ -211,7 +212,7 @@ struct SharedTables {
     std::mutex mu;
     std::map<std::pair<int, int>, ModePlan> mode;
     std::map<std::tuple<int, int, int, int>, BinPlan> bin;
-    std::map<std::tuple<int, int, int>, void *> mas;
+    std::map<std::tuple<int, int, int>, std::pair<void *, float>> mas;   // table, cmax (get_mas_tab)
     std::map<std::pair<int, int>, void *> twiddles;
 };
 SharedTables &shared_tables();
