@@ -229,8 +229,15 @@ struct Chunk {
     int r;              // realisation
     int wbase;          // window placement (count pass): w0 (linear) or wx * nt + wy (box, block)
     int smin, smax;     // first and last non-empty window slot (count pass; smin > smax: none)
-    int wz, pad1;       // block window: first tile along z
+    int wz;             // block window: first tile along z
+    int nfill;          // window slots filled (count pass)
 };
+
+// Particles in no order: few to each tile the chunk reaches, so that the records of a
+// tile are worth bringing together in LDS before they are written (staged_scatter_kernel
+// in place of tile_scatter_kernel, sorts of small grids).  8192 particles in random order
+// reach 512 tiles, 16 each; as many of a displaced lattice 64 to 128.
+__device__ __forceinline__ bool scattered(const Chunk &ch) { return ch.c1 - ch.c0 < 96ll * ch.nfill; }
 
 // Key windows of a sort chunk (TileGeom::wmode, chosen on the host):
 //  kWinDirect  ntiles <= kWin: slot = key - rbase, every key counted in LDS;
@@ -414,9 +421,10 @@ tile_count_kernel(const float *__restrict__ pos, RSD rsd, float inv, TileGeom g,
     __shared__ unsigned hist[WS];
     const Chunk ch = chunks[blockIdx.x];
     const long long rbase = (long long)ch.r * g.ntiles;
-    // every thread derives the window from the chunk's middle particle
+    // every thread derives the window from the chunk's middle particle (the window of
+    // every key needs none, and its chunks are spared the wait for it)
     int3 t0 = make_int3(0, 0, 0);
-    if (ch.c1 > ch.c0)
+    if (ch.c1 > ch.c0 && (g.wmode != kWinDirect || box_miss))
         t0 = dist_tiles<MAS, AXES, POW2>(load_dist<AXES>(pos, rsd, ch.c0 + (ch.c1 - ch.c0) / 2, inv), g);
     const Win w = make_win(g, t0, tiles_key(t0, g, rbase), rbase);
     if (threadIdx.x == 0) {
@@ -459,10 +467,11 @@ tile_count_kernel(const float *__restrict__ pos, RSD rsd, float inv, TileGeom g,
     }
     __syncthreads();
     unsigned *dmp = dump + (long long)blockIdx.x * dump_stride<WS>(g);
-    int smin = WS, smax = -1;
+    int smin = WS, smax = -1, nfill = 0;
     for (int s = threadIdx.x; s < w.slots; s += blockDim.x) {
         const unsigned v = hist[s];
         if (v) {
+            ++nfill;
             dmp[s] = atomicAdd(&counts[win_key(s, w, g, rbase)], v);
             smin = min(smin, s);
             smax = max(smax, s);
@@ -472,6 +481,7 @@ tile_count_kernel(const float *__restrict__ pos, RSD rsd, float inv, TileGeom g,
     for (int off = 32; off > 0; off >>= 1) {
         smin = min(smin, __shfl_xor(smin, off));
         smax = max(smax, __shfl_xor(smax, off));
+        nfill += __shfl_xor(nfill, off);
         if (box_miss) miss += (unsigned)__shfl_xor((int)miss, off);
     }
     __syncthreads();                           // hist is reused for the wave results
@@ -481,16 +491,19 @@ tile_count_kernel(const float *__restrict__ pos, RSD rsd, float inv, TileGeom g,
         red[2 * (threadIdx.x >> 6)] = smin;
         red[2 * (threadIdx.x >> 6) + 1] = smax;
         red[2 * nw + (threadIdx.x >> 6)] = (int)miss;
+        red[3 * nw + (threadIdx.x >> 6)] = nfill;
     }
     __syncthreads();
     if (threadIdx.x == 0) {
-        int a = WS, b = -1;
+        int a = WS, b = -1, f = 0;
         unsigned m = 0;
         for (int k = 0; k < nw; ++k) {
             a = min(a, red[2 * k]);
             b = max(b, red[2 * k + 1]);
             m += (unsigned)red[2 * nw + k];
+            f += red[3 * nw + k];
         }
+        chunks[blockIdx.x].nfill = f;
         chunks[blockIdx.x].smin = a;
         chunks[blockIdx.x].smax = b;
         // one atomic per workgroup on the single tally word
@@ -509,10 +522,11 @@ tile_scatter_kernel(const float *__restrict__ pos, RSD rsd, const float *__restr
                     const unsigned *__restrict__ dump, const unsigned long long *__restrict__ offsets,
                     const unsigned *__restrict__ counts, unsigned *__restrict__ ocursors,
                     unsigned *__restrict__ wmax_bits, float *__restrict__ records,
-                    unsigned long long rcap) {
+                    unsigned long long rcap, int split) {
     __shared__ unsigned cur[WS];
     const Chunk ch = chunks[blockIdx.x];
     if (ch.c1 <= ch.c0) return;                // empty chunk (uniform over the workgroup)
+    if (split && scattered(ch)) return;        // left to staged_scatter_kernel
     const long long rbase = (long long)ch.r * g.ntiles;
     // the count pass's window of this chunk
     Win win{g.wmode, 0, 0, 0, (int)g.ntiles};
@@ -1125,6 +1139,16 @@ bucket_plan_kernel(const unsigned *__restrict__ bcounts, int nb, long long targe
 // the one-pass scatter; the runs of a chunk's sub-chunks follow one another.
 constexpr int kStage1 = 4096;      // particles per sub-chunk, pass 1 (buckets)
 constexpr int kStage2 = 8192;      // and pass 2 (tiles)
+// MODE 2, the only pass over small grids (3D, every tile in the window): a launch beside
+// tile_scatter_kernel's, which takes the chunks that are not scattered().  33 M particles
+// in random order on 32 grids of 128^3, CIC: 302 -> 210 us, weighted 405 -> 260; of a
+// displaced lattice, which leave in runs as they come, 153 us one by one and 172 staged.
+constexpr int kStage3 = 8192;
+constexpr int kStageSlots = 512;
+// From kStageMin particles on, where the second launch (3 to 6 us) is within 2 % of a call
+// on coherent particles (8.4 M on 128^3: lattice 142 -> 146 us, random order 177 -> 164; 33.5 M
+// there: 474 -> 465 and 662 -> 558), with chunks up to twice as long, which make up for it.
+constexpr long long kStageMin = 10ll << 20;
 
 // Exclusive scan of cnt[0..ns) into ofs[0..ns) over the workgroup (kSortBlock
 // threads, ns <= NS); returns the total.  wsum: kSortBlock / 64 + 1 words of LDS.
@@ -1186,6 +1210,7 @@ staged_scatter_kernel(const float *__restrict__ pos, RSD rsd, const float *__res
     __shared__ unsigned long long gcur[NS];
     __shared__ unsigned wsum[kSortBlock / 64 + 1];
     const Chunk ch = chunks[blockIdx.x];
+    if (MODE == 2 && !scattered(ch)) return;   // written by tile_scatter_kernel (uniform)
     const long long rbase = (long long)ch.r * g.ntiles;
     const int t = threadIdx.x;
     const int nbtz = bucket_counts_z(g.ntz);
@@ -1197,13 +1222,16 @@ staged_scatter_kernel(const float *__restrict__ pos, RSD rsd, const float *__res
         win.c = ch.wz;
         ns = kBktSlots;
     }
+    if (MODE == 2) ns = (int)g.ntiles;
     // run bases: pass 1, bucket offset + the chunk's base in the bucket; pass 2, tile
     // offset + the chunk's base in the tile (only the slots the count found filled
     // have a base; in pass 2 they lie in [smin, smax], and a slot of the block past
     // the grid's last tile is never filled)
-    const unsigned *dmp = dump + (long long)blockIdx.x * (MODE == 0 ? ns : NS);
+    const unsigned *dmp = dump + (long long)blockIdx.x * (MODE == 1 ? NS : ns);
     if (MODE == 0) {
         for (int s = t; s < ns; s += blockDim.x) gcur[s] = base[s] + dmp[s];
+    } else if (MODE == 2) {
+        for (int s = ch.smin + t; s <= ch.smax; s += blockDim.x) gcur[s] = base[rbase + s] + dmp[s];
     } else {
         for (int s = ch.smin + t; s <= ch.smax; s += blockDim.x) {
             const int dz = s % kBktZ, dy = (s / kBktZ) % kBkt, dx = s / (kBkt * kBktZ);
@@ -1233,6 +1261,8 @@ staged_scatter_kernel(const float *__restrict__ pos, RSD rsd, const float *__res
                 const int3 tt = dist_tiles<MAS, 3, POW2>(d[k], g);
                 if (MODE == 0) {
                     sl[k] = tile_bucket(tt, nbt, nbtz);
+                } else if (MODE == 2) {
+                    sl[k] = (int)(tiles_key(tt, g, rbase) - rbase);
                 } else {
                     const unsigned key = tiles_key(tt, g, rbase);
                     const unsigned s = win_slot(tt, key, win, g, rbase);
@@ -1255,7 +1285,7 @@ staged_scatter_kernel(const float *__restrict__ pos, RSD rsd, const float *__res
                     }
                 }
                 if (sl[k] >= 0) rk[k] = atomicAdd(&hist[sl[k]], 1u);
-                if (MODE == 1 && WT) {
+                if (MODE != 0 && WT) {
                     const unsigned b = __float_as_uint(fabsf(w[k]));
                     if (b < 0x7f800000u) m = max(m, b);
                 }
@@ -1279,7 +1309,7 @@ staged_scatter_kernel(const float *__restrict__ pos, RSD rsd, const float *__res
             const int s = sslot[j];
             const unsigned long long at = gcur[s] + (unsigned long long)(j - (int)lofs[s]);
             if (at >= rcap) continue;                 // only after a miscount (reported)
-            if (MODE == 1 && WT) {
+            if (MODE != 0 && WT) {
                 reinterpret_cast<float4 *>(out)[at] = make_float4(sx[j], sy[j], sz[j], sw[j]);
             } else {
                 out[3 * at] = sx[j];
@@ -1292,7 +1322,7 @@ staged_scatter_kernel(const float *__restrict__ pos, RSD rsd, const float *__res
         for (int s = t; s < ns; s += blockDim.x) gcur[s] += hist[s];
         __syncthreads();
     }
-    if (MODE == 1 && WT) {
+    if (MODE != 0 && WT) {
         for (int off = 32; off > 0; off >>= 1) m = max(m, (unsigned)__shfl_xor((int)m, off));
         if ((t & 63) == 0) wsum[t >> 6] = m;
         __syncthreads();
@@ -3433,12 +3463,14 @@ int run_tiled(Ctx *c, const float *pos, const RSD &rsd, long long n, const long 
                  : two ? kBktSlots
                  : g.wmode == kWinDirect ? (int)g.ntiles : kWin;
     // Chunks of consecutive particles, never straddling two realisations.
+    const bool staged = !capm && !two && !wide && axes == 3 && g.wmode == kWinDirect && g.ntiles <= kStageSlots &&
+                        n >= kStageMin;
     // A few small tiles take small chunks down to kChunkPerTile particles per tile: more
     // workgroups for a call that would not fill the chip.  (Fixed scratch keeps to 8192.)
     const long long floor = c->arena ? 8192LL
                                      : std::max(1024LL, std::min(8192LL, kChunkPerTile * g.ntiles));
     const long long target = wide ? std::max(2 * g.ntiles, std::min(16 * g.ntiles, (n + 2047) / 2048))
-                                  : std::max(floor, std::min(65536LL, (n + 4095) / 4096));
+                                  : std::max(floor, std::min(65536LL, staged ? (n + 2047) / 2048 : (n + 4095) / 4096));
     long long nchunk_ll = 0;
     if (devt) nchunk_ll = (long long)nreal * c->chunks_per_real;
     else
@@ -3728,7 +3760,7 @@ int run_tiled(Ctx *c, const float *pos, const RSD &rsd, long long n, const long 
                  : (pow2 ? tile_scatter_kernel<MAS, 3, true, false, kWin>
                          : tile_scatter_kernel<MAS, 3, false, false, kWin>));
         ks<<<kSpillChunks, kSortBlock, 0, c->stream>>>(pxyz, off, pw, 1.0f, gs, dchunksS, dump, offsets, counts,
-                                                       ocursors, wmax, records, (unsigned long long)n);
+                                                       ocursors, wmax, records, (unsigned long long)n, 0);
         auto kss2 = W ? (pow2 ? spill_scatter_kernel<MAS, true, true> : spill_scatter_kernel<MAS, false, true>)
                       : (pow2 ? spill_scatter_kernel<MAS, true, false> : spill_scatter_kernel<MAS, false, false>);
         PYL_TRY(make_report());
@@ -3816,7 +3848,15 @@ int run_tiled(Ctx *c, const float *pos, const RSD &rsd, long long n, const long 
                                : (pow2 ? tile_scatter_kernel<MAS, 2, true, false, kWin>
                                        : tile_scatter_kernel<MAS, 2, false, false, kWin>));
         ks<<<nsort, kSortBlock, 0, c->stream>>>(spos, srsd, sW, sinv, g, schunks, dump, offsets, counts,
-                                                ocursors, wmax, records, rcap);
+                                                ocursors, wmax, records, rcap, staged);
+        if (staged) {                          // the chunks it left
+            auto kss = W ? (pow2 ? staged_scatter_kernel<MAS, true, true, 2, kStageSlots, kStage3>
+                                 : staged_scatter_kernel<MAS, false, true, 2, kStageSlots, kStage3>)
+                         : (pow2 ? staged_scatter_kernel<MAS, true, false, 2, kStageSlots, kStage3>
+                                 : staged_scatter_kernel<MAS, false, false, 2, kStageSlots, kStage3>);
+            kss<<<nsort, kSortBlock, 0, c->stream>>>(spos, srsd, sW, sinv, g, nbt, schunks, dump, offsets,
+                                                     counts, ocursors, records, nullptr, wmax, rcap);
+        }
         PYL_HIP(hipGetLastError());
         PYL_TRY(stage_end(c, PYL_STAGE_MA_SCATTER));
     }
