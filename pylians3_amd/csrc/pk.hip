@@ -333,6 +333,8 @@ __device__ __forceinline__ float phase_sq(float xr, float xi) {
     return ph * ph;
 }
 
+__device__ __forceinline__ float masked(float x, unsigned on) { return __uint_as_float(__float_as_uint(x) & on); }
+
 // VALU-bound: about 170 instructions per mode when every row was binned by itself
 // (0.305 ms at 512^3, axis 0, against 0.1 ms for its 0.54 GB).  The symmetric rows of a
 // group share everything but their values, so the geometry, the MAS factor, the
@@ -512,14 +514,16 @@ __global__ void __launch_bounds__(kBinBlock) pk_bin_kernel(BinArgs a) {
             for (int sp = 0; sp < S; ++sp) d2[sp] = 0.0;
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
-                // rows that are not there, or not independent, count with factor 0
-                const bool on = (mask >> q) & 1u;
+                // rows that are not there, or not independent, count as 0: their values are
+                // masked, not multiplied by 0, since a caller's field may hold NaN or
+                // infinities in them (the mask costs no more than the factor did)
+                const unsigned on = (unsigned)__builtin_amdgcn_sbfe((int)mask, q, 1);   // all ones or 0
                 double re[NFL], im[NFL];
                 float xr0 = 0.0f, xi0 = 0.0f;
 #pragma unroll
                 for (int f = 0; f < NFL; ++f) {
-                    const float mq = on ? mf[f] : 0.0f;
-                    const float xr = v[f][q][s].x * mq, xi = v[f][q][s].y * mq;   // complex64 * float
+                    const float xr = masked(v[f][q][s].x * mf[f], on);   // complex64 * float
+                    const float xi = masked(v[f][q][s].y * mf[f], on);
                     re[f] = (double)xr;
                     im[f] = (double)xi;
                     if (f == 0) {
