@@ -150,6 +150,13 @@ def _run_pk(fields, mas_ids, BoxSize, axis, ctx=None, fourier=False, flags=0):
     return arrs
 
 
+def _only(a):
+    """The result array of one spectrum without its spectra axis, in place: no copy, and
+    still an array that owns its memory."""
+    a.resize(a.shape[:-1], refcheck=False)     # the same elements: nothing moves
+    return a
+
+
 class Pk:
     """1D, 2D and 3D (l = 0, 2, 4) power spectrum of a density field (Pk_library.pyx:263-420)."""
 
@@ -166,16 +173,16 @@ class Pk:
         if verbose:
             print('Time to complete loop = %.2f' % (time.time() - start2))
         self.k1D = r['k1D']
-        self.Pk1D = r['Pk1D'][:, 0]           # one spectrum: the column is the whole array
+        self.Pk1D = _only(r['Pk1D'])
         self.Nmodes1D = r['Nmodes1D']
         self.kpar = r['kpar']
         self.kper = r['kper']
-        self.Pk2D = r['Pk2D'][:, 0]
+        self.Pk2D = _only(r['Pk2D'])
         self.Nmodes2D = r['Nmodes2D']
         check_number_modes(np.concatenate([[1.0], r['Nmodes3D']]), dims)
         self.k3D = r['k3D']
         self.Nmodes3D = r['Nmodes3D']
-        self.Pk = r['Pk3D'][:, :, 0]
+        self.Pk = _only(r['Pk3D'])
         self.Pkphase = r['Pkphase']
         if verbose:
             print('Time taken = %.2f seconds' % (time.time() - start))

@@ -6,8 +6,8 @@ call raises.
 """
 import ctypes
 import functools
-import math
 import os
+import struct
 import threading
 
 import numpy as np
@@ -261,34 +261,34 @@ def pk_sizes(dims, nfields):
     return s
 
 
+_PK_NAMES = [name for name, _ in PkOut._fields_]
+_pk_pack = struct.Struct('=%dQ' % len(_PK_NAMES)).pack
+_at = (ctypes.c_char * 0).from_buffer
+
+
 @functools.lru_cache(maxsize=64)
-def _pk_layout(dims, nfields):
-    """Where the arrays of a PkOut lie in one block of float64: (its length, byte offsets
-    in field order, [(name, slice, shape)], spectra)."""
+def _pk_shapes(dims, nfields):
+    """Shapes of the arrays of a PkOut in field order, and the number of spectra."""
     s = pk_sizes(dims, nfields)
     S = s.nspectra
     shape = dict(k1D=(s.n1d,), Nmodes1D=(s.n1d,), Pk1D=(s.n1d, S), kpar=(s.n2d,), kper=(s.n2d,),
                  Nmodes2D=(s.n2d,), Pk2D=(s.n2d, S), k3D=(s.n3d,), Nmodes3D=(s.n3d,),
                  Pk3D=(s.n3d, 3, S), Pkphase=(s.n3d,))
-    at, offs, views = 0, [], []
-    for name, _ in PkOut._fields_:
-        n = math.prod(shape[name])
-        offs.append(8 * at)
-        views.append((name, slice(at, at + n), shape[name]))
-        at += n
-    return at, np.array(offs, np.uint64), views, S
+    return [shape[name] for name in _PK_NAMES], S
 
 
 def alloc_pk_out(dims, nfields):
     """Allocate float64 result arrays and the PkOut struct pointing at them.
 
-    One block and 11 views of it: eleven allocations and ctypes casts took 22 us of a
-    70 us spectrum of 64^3, and 0.7 ms of the 4.7 ms of 32 realisations of 128^3."""
-    total, offs, views, S = _pk_layout(int(dims), int(nfields))
-    block = np.empty(total)       # the library writes every element but Pkphase's
-    arrs = {name: block[at].reshape(shape) if len(shape) > 1 else block[at] for name, at, shape in views}
-    arrs['Pkphase'].fill(0.0)
-    out = PkOut.from_buffer(offs + np.uint64(block.ctypes.data))
+    Every array has memory of its own: a caller that keeps one keeps only that (of a 512^3
+    spectrum 10 kB of multipoles, not the 3 MB of all).  Addresses by from_buffer: eleven
+    casts with ctypes.data_as took 22 us of a 70 us spectrum of 64^3, this whole function
+    takes 7.4, as did one block with eleven views of it."""
+    shapes, S = _pk_shapes(int(dims), int(nfields))
+    a = list(map(np.empty, shapes))       # the library writes every element but Pkphase's
+    a[-1].fill(0.0)
+    arrs = dict(zip(_PK_NAMES, a))
+    out = PkOut.from_buffer_copy(_pk_pack(*map(ctypes.addressof, map(_at, a))))
     out._keep = arrs          # the struct holds raw pointers into these arrays
     return out, arrs, S
 
