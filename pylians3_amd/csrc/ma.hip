@@ -948,7 +948,7 @@ template <bool ONE>
 __global__ void __launch_bounds__(kScanBlock)
 scan_final_kernel(const unsigned *__restrict__ in, const unsigned *__restrict__ in2, long long n,
                   const unsigned long long *__restrict__ block_prefix,
-                  unsigned long long *__restrict__ out, SortReport rep) {
+                  unsigned long long *__restrict__ out, SortReport rep, unsigned *clear) {
     __shared__ unsigned long long sh[kScanBlock / 64];
     const long long first = (long long)blockIdx.x * kScanTile;
     unsigned long long prefix = 0;
@@ -977,6 +977,7 @@ scan_final_kernel(const unsigned *__restrict__ in, const unsigned *__restrict__ 
     if (blockIdx.x == gridDim.x - 1 && threadIdx.x == kScanBlock - 1) {
         out[n] = ex;
         if (rep.total) report(rep, ex);
+        if (clear) *clear = 0u;                // (may be in2[n - 1], read by this workgroup only)
     }
 }
 
@@ -2341,9 +2342,17 @@ constexpr int kOrderBlock = 1024;
 constexpr int kOrderBuckets = 512;
 // Column deposit: tiles per segment, as many as leave kColMinSegs segments.
 // (134 M particles, TSC on 512^3, deposit + finalize: 1.39 ms with one tile per segment,
-// 1.31, 1.29 and 1.28 ms with 4, 8 and 16.)
+// 1.31, 1.29 and 1.28 ms with 4, 8 and 16; MA of 2 M, CIC on 512^3: 0.90 ms with one, 0.70
+// with 16.)  A segment of 2^kColMinCut records and more is cut so that the cuts of a call
+// are kColCuts at most: a workgroup that had a whole segment of a beam, a cluster or a
+// refined region to itself set the time of the call (MA of 16 M particles in a beam of 4 x 4
+// tiles along z, TSC on 512^3: one tile per workgroup 1.61 ms, whole segments 3.06, cut 1.46;
+// 134 M, half of them in 3000 clusters: 9.6, 12.7 and 9.6).  Twice as many cuts gained
+// nothing (1.44), and every workgroup that finds no unit costs 9 ns.
 constexpr int kColMaxLen = 16;
 constexpr long long kColMinSegs = 2048;
+constexpr int kColMinCut = 13;
+constexpr long long kColCuts = 512;
 constexpr long long kColPcsDense = 2048;         // mean records per tile
 constexpr long long kOrderMinKeys = 2048;
 constexpr long long kOrderMinRecords = 512;      // mean records per key
@@ -2372,28 +2381,64 @@ __host__ __device__ __forceinline__ int count_bucket(unsigned long long n) {
     return min(kOrderBuckets - 1, 1 + 16 * lg + q);
 }
 
-// What the deposit's workgroups take: runs of up to len consecutive keys of columns of
-// per keys, segs runs per column (one key each: {1, 1, 1}).
+// What the deposit's workgroups take (units): segments of up to len (a power of two, at most
+// 16) consecutive keys of columns of per keys, segs segments per column (one key each: {1, 1,
+// 1}).  A segment is cut before every key at which the records in front of it, counted from
+// the segment's first key, pass a multiple of 2^shift: a unit holds less than 2^shift records
+// besides those of its last key, and n records make at most n >> shift more units than there
+// are segments.  starts[segment] (if wanted): bit j set where key j starts a unit.
 struct OrderSeg {
-    int len, per, segs;
+    int len, per, segs, shift;
+    unsigned nseg;
+    unsigned *starts;
 };
 
-// Records of run k: the runs of the sorted records plus the capacity slots.
-__device__ __forceinline__ unsigned long long key_records(const unsigned long long *__restrict__ offsets,
-                                                          long long k, const OrderSeg &os, const CapRecs &cr) {
-    const long long c = k / os.segs;
-    const long long k0 = c * os.per + (k - c * os.segs) * os.len, k1 = min(k0 + os.len, (c + 1) * os.per);
-    unsigned long long n = offsets[k1] - offsets[k0];
-#pragma unroll 8
-    for (long long j = k0; j < k1; ++j) n += cap_count(cr, j);
-    return n;
+// A listed unit: its first key (below 2^24) and number of keys (those past the column's end
+// are not there).
+__host__ __device__ __forceinline__ unsigned make_unit(unsigned key, unsigned len) { return key | (len - 1) << 28; }
+__host__ __device__ __forceinline__ unsigned unit_key(unsigned unit) { return unit & 0xfffffffu; }
+__host__ __device__ __forceinline__ int unit_len(unsigned unit) { return (int)(unit >> 28) + 1; }
+
+// Keys of the unit that starts at key j of a segment of len keys.
+__host__ __device__ __forceinline__ int unit_keys(unsigned starts, int j, int len) {
+    const unsigned next = starts >> j >> 1;
+    return next ? __builtin_ctz(next) + 1 : len - j;
+}
+
+// Key slot i (slot j of segment q is i = q * len + j: a segment's keys are read by
+// neighbouring lanes): its unit and the unit's records; false: no unit starts there.  Called
+// by whole wavefronts, for consecutive slots from a multiple of 64 on.
+__device__ __forceinline__ bool order_unit(const unsigned long long *__restrict__ offsets, unsigned i,
+                                           const OrderSeg &os, const CapRecs &cr, unsigned &unit,
+                                           unsigned long long &n) {
+    const unsigned q = i / (unsigned)os.len, j = i - q * os.len;
+    const unsigned c = q / (unsigned)os.segs, z = (q - c * os.segs) * os.len + j;
+    const unsigned k = c * os.per + z;
+    const bool in = q < os.nseg && z < (unsigned)os.per;
+    const unsigned long long own = in ? offsets[k + 1] - offsets[k] + cap_count(cr, k) : 0ull;
+    unsigned long long upto = own;                     // records of keys 0..j of the segment
+    for (int o = 1; o < os.len; o <<= 1) {
+        const unsigned long long v = __shfl_up(upto, o);
+        if ((int)j >= o) upto += v;
+    }
+    const unsigned piece = (unsigned)((upto - own) >> os.shift);
+    const unsigned below = (unsigned)__shfl_up((int)piece, 1);
+    const bool start = in && (j == 0 || piece != below);
+    const int first = (int)(threadIdx.x & 63) - (int)j;            // the segment's first lane
+    const unsigned starts = (unsigned)(__ballot(start) >> first) & ((1u << os.len) - 1u);
+    if (os.starts && in && j == 0) os.starts[q] = starts;
+    const int len = unit_keys(starts, (int)j, os.len);
+    n = __shfl(upto, first + (int)j + len - 1) - (upto - own);
+    unit = make_unit(k, (unsigned)len);
+    return start;
 }
 
 // The order is built in two launches of order_wgs(nt) workgroups, each thread
-// taking up to kOrderPer keys (k = its global index + j * threads): bucket sizes
-// (order_hist_kernel), then the keys placed at their bucket's start plus a run
-// claimed per workgroup (order_place_kernel).  Counters sit in LDS per workgroup
-// and only their totals go to the global ones (ghist, gcur: zeroed by the call).
+// taking up to kOrderPer of the nt key slots (k = its global index + j * threads): bucket
+// sizes (order_hist_kernel), then the units placed at their bucket's start plus a run
+// claimed per workgroup (order_place_kernel, which also writes their number to nunits
+// unless that is null).  Counters sit in LDS per workgroup and only their totals go to the
+// global ones (ghist, gcur: zeroed by the call).
 constexpr int kOrderPer = 8;
 constexpr int kOrderMinWGs = 32;
 inline int order_wgs(long long nt) {
@@ -2402,31 +2447,33 @@ inline int order_wgs(long long nt) {
 }
 
 __global__ void __launch_bounds__(kOrderBlock)
-order_hist_kernel(const unsigned long long *__restrict__ offsets, long long nt, OrderSeg os, CapRecs cr,
+order_hist_kernel(const unsigned long long *__restrict__ offsets, OrderSeg os, CapRecs cr,
                   unsigned *__restrict__ ghist) {
     __shared__ unsigned hist[kOrderBuckets];
     for (int b = threadIdx.x; b < kOrderBuckets; b += blockDim.x) hist[b] = 0u;
     __syncthreads();
-    const long long k0 = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    const long long step = (long long)gridDim.x * blockDim.x;
-    unsigned long long c[kOrderPer];
+    const unsigned k0 = blockIdx.x * blockDim.x + threadIdx.x, step = gridDim.x * blockDim.x;
+    int bk[kOrderPer];
 #pragma unroll
     for (int j = 0; j < kOrderPer; ++j) {        // all loads before the first atomic
-        const long long k = k0 + j * step;
-        c[j] = k < nt ? key_records(offsets, k, os, cr) : 0ull;
+        unsigned unit;
+        unsigned long long n;
+        bk[j] = -1;
+        if ((k0 & ~63u) + j * step >= os.nseg * os.len) continue;     // (whole wavefronts)
+        if (order_unit(offsets, k0 + j * step, os, cr, unit, n)) bk[j] = count_bucket(n);
     }
 #pragma unroll
     for (int j = 0; j < kOrderPer; ++j)
-        if (k0 + j * step < nt) atomicAdd(&hist[count_bucket(c[j])], 1u);
+        if (bk[j] >= 0) atomicAdd(&hist[bk[j]], 1u);
     __syncthreads();
     for (int b = threadIdx.x; b < kOrderBuckets; b += blockDim.x)
         if (hist[b]) atomicAdd(&ghist[b], hist[b]);
 }
 
 __global__ void __launch_bounds__(kOrderBlock)
-order_place_kernel(const unsigned long long *__restrict__ offsets, long long nt, OrderSeg os, CapRecs cr,
+order_place_kernel(const unsigned long long *__restrict__ offsets, OrderSeg os, CapRecs cr,
                    const unsigned *__restrict__ ghist, unsigned *__restrict__ gcur,
-                   unsigned *__restrict__ order) {
+                   unsigned *__restrict__ order, unsigned *__restrict__ nunits) {
     __shared__ unsigned start[kOrderBuckets];   // first slot of each bucket, largest first
     __shared__ unsigned lrun[kOrderBuckets];    // this workgroup's keys per bucket, then its cursor
     if (threadIdx.x < 64) {                      // exclusive scan of ghist from the top bucket down
@@ -2444,30 +2491,45 @@ order_place_kernel(const unsigned long long *__restrict__ offsets, long long nt,
         unsigned run = incl - sum;
 #pragma unroll
         for (int j = 0; j < PB; ++j) { start[top - j] = run; run += h[j]; }
+        if (nunits && blockIdx.x == 0 && threadIdx.x == 63) *nunits = run;
     }
     for (int b = threadIdx.x; b < kOrderBuckets; b += blockDim.x) lrun[b] = 0u;
     __syncthreads();
-    const long long k0 = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    const long long step = (long long)gridDim.x * blockDim.x;
+    const unsigned k0 = blockIdx.x * blockDim.x + threadIdx.x, step = gridDim.x * blockDim.x;
     int bk[kOrderPer];
+    unsigned unit[kOrderPer];
 #pragma unroll
     for (int j = 0; j < kOrderPer; ++j) {
-        const long long k = k0 + j * step;
-        bk[j] = k < nt ? count_bucket(key_records(offsets, k, os, cr)) : 0;
+        unsigned long long n;
+        bk[j] = -1;
+        if ((k0 & ~63u) + j * step >= os.nseg * os.len) continue;     // (whole wavefronts)
+        if (order_unit(offsets, k0 + j * step, os, cr, unit[j], n)) bk[j] = count_bucket(n);
     }
 #pragma unroll
     for (int j = 0; j < kOrderPer; ++j)
-        if (k0 + j * step < nt) atomicAdd(&lrun[bk[j]], 1u);
+        if (bk[j] >= 0) atomicAdd(&lrun[bk[j]], 1u);
     __syncthreads();
     // one claim per bucket this workgroup holds keys of
     for (int b = threadIdx.x; b < kOrderBuckets; b += blockDim.x)
         if (lrun[b]) lrun[b] = start[b] + atomicAdd(&gcur[b], lrun[b]);
     __syncthreads();
 #pragma unroll
-    for (int j = 0; j < kOrderPer; ++j) {
-        const long long k = k0 + j * step;
-        if (k < nt) order[atomicAdd(&lrun[bk[j]], 1u)] = (unsigned)k;
-    }
+    for (int j = 0; j < kOrderPer; ++j)
+        if (bk[j] >= 0) order[atomicAdd(&lrun[bk[j]], 1u)] = unit[j];
+}
+
+// Without the order: the units that do not start a segment, in any order (count: zeroed
+// before).  One launch of 3 us; the order's two would take 20 us of a 0.70 ms call (2 M, CIC
+// on 512^3).
+constexpr int kPlanBlock = 256;
+__global__ void __launch_bounds__(kPlanBlock)
+segment_plan_kernel(const unsigned long long *__restrict__ offsets, OrderSeg os, CapRecs cr,
+                    unsigned *__restrict__ list, unsigned *__restrict__ count) {
+    const unsigned i = blockIdx.x * kPlanBlock + threadIdx.x;
+    unsigned unit;
+    unsigned long long n;
+    const bool is = order_unit(offsets, i, os, cr, unit, n);
+    if (is && i % (unsigned)os.len != 0) list[atomicAdd(count, 1u)] = unit;
 }
 
 // Images along one axis of a tile t: the tiles whose boxes cover its nodes and
@@ -2688,10 +2750,10 @@ tile_finalize_uniform_kernel(const unsigned long long *__restrict__ offsets, Til
 }
 
 // ---- column deposit: 3D grids of two tiles or more per axis (CIC, TSC, PCS) ------
-// A workgroup takes a segment of ColSeg::len tiles that follow one another along z and
-// keeps the LDS box from tile to tile: the upper halo planes of a tile become, as
-// floats in registers (the carry), a second contribution to the first F-1 planes of the
-// next.  Compared with one workgroup per tile
+// A workgroup takes a segment of ColSeg::len tiles that follow one another along z, or a
+// part of one (OrderSeg), and keeps the LDS box from tile to tile: the upper halo planes of
+// a tile become, as floats in registers (the carry), a second contribution to the first F-1
+// planes of the next.  Compared with one workgroup per tile
 //  * the nodes a tile shares only with its z neighbours are final when their tile is
 //    flushed and are written once, in whole 64-byte rows of the grid; only the ring
 //    (nodes that x or y neighbours share) goes through partial values, in rows of a
@@ -2700,7 +2762,7 @@ tile_finalize_uniform_kernel(const unsigned long long *__restrict__ offsets, Til
 //    of an accumulated grid while its last atomics run.
 // The value of a node is the float64 sum of the same float32 tile values in the same
 // order as in the tile form (own, then the lower z neighbour, per x and y image), rounded
-// once: the bits do not depend on the form or on the segment length.
+// once: the bits do not depend on the form, on the segment length or on the cuts.
 // Deposit and finalize together, tile form and column form: 134 M particles, TSC on 512^3
 // 1.34 and 1.26 ms, on 500^3 1.80 and 1.43; 2 M weighted, PCS on 512^3 1.23 and 0.94;
 // 67 M in 32 CIC grids of 128^3 0.47 and 0.40.
@@ -2709,12 +2771,15 @@ tile_finalize_uniform_kernel(const unsigned long long *__restrict__ offsets, Til
 // by ring_col, interior columns by (x - L) * (ey - L) + y - L):
 //   ring  [rc * zs + z]       own sums, z < ez
 //   carry [rc * L + z]        the lower z neighbour's, z < L
-//   low   [ic * L + z]        own interior sums of a segment's first tile, z < L
-//   clow  [ic * L + z]        and what the segment before it carries over
+//   low   [ic * L + z]        own interior sums of the first tile of a unit, z < L
+//   clow  [ic * L + z]        and what the unit before it carries over
 struct ColSeg {
-    int len;     // tiles per segment
-    int nz;      // segments per column of tiles
-    int zs;      // largest tile extent
+    int len;                   // tiles per segment
+    int nz;                    // segments per column of tiles
+    int zs;                    // largest tile extent
+    const unsigned *starts;    // where units start in each segment (OrderSeg), null: no segment is cut
+    const unsigned *nunits;    // units listed, null: one for each workgroup of the list
+    int nwhole;                // workgroups that take a segment's first unit each, before the list's
 };
 
 template <int F>
@@ -2792,8 +2857,21 @@ column_deposit_kernel(const float *__restrict__ records, unsigned long long rcap
     __shared__ unsigned whist[ROT ? 1 : NW * 16];
     const int t = threadIdx.x;
     const int wv = __builtin_amdgcn_readfirstlane(t >> 6), ln = t & 63;
-    const int sid = __builtin_amdgcn_readfirstlane(order ? (int)order[blockIdx.x] : (int)blockIdx.x);
-    const int col = sid / cs.nz, tz0 = (sid - col * cs.nz) * cs.len, tz1 = min(g.nt, tz0 + cs.len);
+    int col, tz0, len;
+    const int li = (int)blockIdx.x - cs.nwhole;
+    if (li < 0) {
+        const int q = (int)blockIdx.x;
+        col = q / cs.nz;
+        tz0 = (q - col * cs.nz) * cs.len;
+        len = cs.starts ? unit_keys(cs.starts[q], 0, cs.len) : cs.len;
+    } else {
+        if (cs.nunits && (unsigned)li >= *cs.nunits) return;   // the launch has room for the most there can be
+        const unsigned unit = (unsigned)__builtin_amdgcn_readfirstlane((int)order[li]);
+        col = (int)(unit_key(unit) / (unsigned)g.nt);
+        tz0 = (int)unit_key(unit) - col * g.nt;
+        len = unit_len(unit);
+    }
+    const int tz1 = min(g.nt, tz0 + len);
     const int real = col / (g.nt * g.nt);
     TileBox tb;
     tb.tx = col / g.nt - real * g.nt;
@@ -2854,7 +2932,7 @@ column_deposit_kernel(const float *__restrict__ records, unsigned long long rcap
     float carry[KC];
 #pragma unroll
     for (int k = 0; k < KC; ++k) carry[k] = 0.0f;
-    bool prev = false;                                  // the tile below in this segment had records
+    bool prev = false;                                  // the tile below in this unit had records
     auto value = [&](int at) {                          // a box sum, cleared for the next tile
         const long long v = (long long)acc[at];
         acc[at] = 0ull;
@@ -2957,7 +3035,7 @@ column_deposit_kernel(const float *__restrict__ records, unsigned long long rcap
         prev = some;
         __syncthreads();
     }
-    // what the last tile carries over, for the tile above it (the next segment's first)
+    // what the last tile carries over, for the tile above it (the next unit's first)
     if (prev) {
         float *part = partials + ((long long)col * g.nt + (tz1 == g.nt ? 0 : tz1)) * g.pslot;
 #pragma unroll
@@ -3008,7 +3086,9 @@ column_finalize_kernel(const unsigned long long *__restrict__ offsets, TileGeom 
     }
     __syncthreads();
     const unsigned has = s_has;
-    const bool first = tz % cs.len == 0;
+    // its own low planes were left to here: the first tile of a unit
+    const unsigned starts = cs.starts ? cs.starts[col * cs.nz + tz / cs.len] : 1u;
+    const bool first = (starts >> (tz % cs.len)) & 1u;
     // an accumulated grid is left alone where no tile contributes
     if (!om.overwrite && has == 0) return;
     auto extent = [&](int i) { return UNI ? T : g.orig[i + 1] - g.orig[i]; };
@@ -3297,17 +3377,18 @@ TileGeom make_geom(int dims, int axes, int mas) {
     return g;
 }
 
-// offsets[0..nt] of the tile counts; `rep` as in scan_final_kernel (rep.total null: none).
+// offsets[0..nt] of the tile counts; `rep` as in scan_final_kernel (rep.total null: none);
+// `clear` (or null): a word set to 0 once the counts are read.
 void launch_scan(Ctx *c, const unsigned *counts, const unsigned *ocounts, long long nt, int nblocks,
-                 unsigned long long *bsums, unsigned long long *offsets, const SortReport &rep) {
+                 unsigned long long *bsums, unsigned long long *offsets, const SortReport &rep, unsigned *clear) {
     if (nblocks <= kScanOne) {
         scan_final_kernel<true><<<nblocks, kScanBlock, 0, c->stream>>>(counts, ocounts, nt, nullptr, offsets,
-                                                                       rep);
+                                                                       rep, clear);
         return;
     }
     scan_partial_kernel<<<nblocks, kScanBlock, 0, c->stream>>>(counts, ocounts, nt, bsums);
     scan_blocksums_kernel<<<1, kScanBlock, 0, c->stream>>>(bsums, nblocks);
-    scan_final_kernel<false><<<nblocks, kScanBlock, 0, c->stream>>>(counts, ocounts, nt, bsums, offsets, rep);
+    scan_final_kernel<false><<<nblocks, kScanBlock, 0, c->stream>>>(counts, ocounts, nt, bsums, offsets, rep, clear);
 }
 
 // The latest order finding per (device, dims, MAS) over every context of the
@@ -3494,6 +3575,8 @@ int run_tiled(Ctx *c, const float *pos, const RSD &rsd, long long n, const long 
     //              (two-level) bucket offsets[nbk+1] | pass-2 chunk table | bucket bases
     //              (capacity) tile cursors[nt] | pad | spill range {0, count}, placed (u64)
     //              (ordered) order bucket sizes[512] | bucket cursors[512]
+    //              (cut segments: starts[nseg], nseg < nt, and the number of units listed take
+    //              the place of ocounts once the scan has read it)
     // Largest tiles first, when there are enough tiles, and records per tile, for the
     // dispatch tail to outweigh the ordering passes.
     // 3D grids of two tiles or more per axis: the column deposit (segments along z), but
@@ -3504,16 +3587,22 @@ int run_tiled(Ctx *c, const float *pos, const RSD &rsd, long long n, const long 
     const bool uni = g.nt >= 2 && dims % (axes == 3 ? kT3 : kT2) == 0;
     const bool column = axes == 3 && g.nt >= 2 && MAS > 1 && nsplit == 1 &&
                         !(MAS == PYL_PCS && uni && n >= kColPcsDense * nt);
-    ColSeg cs{1, g.nt, (dims + g.nt - 1) / g.nt};
-    if (column) {
+    ColSeg cs{1, g.nt, (dims + g.nt - 1) / g.nt, nullptr, nullptr, 0};
+    if (column)
         while (cs.len < kColMaxLen && nt >= 2 * cs.len * kColMinSegs) cs.len *= 2;
-        cs.nz = (g.nt + cs.len - 1) / cs.len;
-    }
+    if (column) cs.nz = (g.nt + cs.len - 1) / cs.len;
     const long long nseg = column ? (long long)nreal * g.nt * g.nt * cs.nz : nt;
-    const OrderSeg oseg = column ? OrderSeg{cs.len, g.nt, cs.nz} : OrderSeg{1, 1, 1};
+    const long long nslots = nseg * cs.len;      // key slots of the order (order_unit)
     const bool ordered = c->tune_order >= 0
         ? (nsplit == 1 && c->tune_order == 1)
         : (nsplit == 1 && nseg >= kOrderMinKeys && n >= kOrderMinRecords * nt);
+    // segments that hold much of the particles are cut (OrderSeg), into `more` units more at
+    // most; without the order these are listed by themselves
+    int shift = kColMinCut;
+    while ((n >> shift) > kColCuts) ++shift;
+    const long long more = cs.len > 1 ? std::min(n >> shift, nt - nseg) : 0;
+    const bool cut = more > 0;
+    cs.nwhole = (int)(ordered ? 0 : nseg);
     size_t nwords = (size_t)nt * 3 + (size_t)nreal + 1 + (two ? (size_t)nbk : 0);
     const size_t cur_at = nwords;
     if (capm) nwords += (size_t)nt;
@@ -3569,6 +3658,24 @@ int run_tiled(Ctx *c, const float *pos, const RSD &rsd, long long n, const long 
     float *bw = ((two || capm) && W) ? (float *)((char *)kv + bxyz_bytes) : nullptr;
     unsigned *cursor = counts + cur_at;
     unsigned *ohist = counts + ohist_at;
+    unsigned *nunits = cut ? ocounts + (nt - 1) : nullptr;
+    unsigned *plan_count = ordered ? nullptr : nunits;
+    cs.nunits = nunits;
+    if (cut) cs.starts = ocounts;
+    const OrderSeg oseg = column ? OrderSeg{cs.len, g.nt, cs.nz, cut ? shift : 63, (unsigned)nseg,
+                                            cut ? ocounts : nullptr}
+                                 : OrderSeg{1, 1, 1, 63, (unsigned)nt, nullptr};
+    const auto launch_order = [&](const CapRecs &ocr) {
+        if (ordered) {
+            const int wgs = order_wgs(nslots);
+            order_hist_kernel<<<wgs, kOrderBlock, 0, c->stream>>>(offsets, oseg, ocr, ohist);
+            order_place_kernel<<<wgs, kOrderBlock, 0, c->stream>>>(offsets, oseg, ocr, ohist, ohist + kOrderBuckets,
+                                                                   order, nunits);
+        } else if (cut) {
+            segment_plan_kernel<<<(unsigned)((nslots + kPlanBlock - 1) / kPlanBlock), kPlanBlock, 0, c->stream>>>(
+                offsets, oseg, ocr, order, nunits);
+        }
+    };
     unsigned long long *capw = (unsigned long long *)(counts + capw_at);
     float *crec = (float *)cv;
     float *pxyz = two ? (float *)sv : bxyz;
@@ -3749,7 +3856,7 @@ int run_tiled(Ctx *c, const float *pos, const RSD &rsd, long long n, const long 
                                           : tile_count_kernel<MAS, 3, false, kWin>);
         kc<<<kSpillChunks, kSortBlock, 0, c->stream>>>(pxyz, off, 1.0f, gs, dchunksS, counts, ocounts, dump,
                                                        nullptr);
-        launch_scan(c, counts, ocounts, nt, nscan_blocks, bsums, offsets, SortReport{});
+        launch_scan(c, counts, ocounts, nt, nscan_blocks, bsums, offsets, SortReport{}, plan_count);
         auto ks = sws == kWinWide
             ? (W ? (pow2 ? tile_scatter_kernel<MAS, 3, true, true, kWinWide>
                          : tile_scatter_kernel<MAS, 3, false, true, kWinWide>)
@@ -3769,12 +3876,7 @@ int run_tiled(Ctx *c, const float *pos, const RSD &rsd, long long n, const long 
         PYL_HIP(hipGetLastError());
         PYL_TRY(stage_end(c, PYL_STAGE_MA_SPILL));
         PYL_TRY(stage_begin(c, PYL_STAGE_MA_SCAN));
-        if (ordered) {
-            const CapRecs ocr{crec, cursor, cap, (long long)n};
-            order_hist_kernel<<<order_wgs(nseg), kOrderBlock, 0, c->stream>>>(offsets, nseg, oseg, ocr, ohist);
-            order_place_kernel<<<order_wgs(nseg), kOrderBlock, 0, c->stream>>>(offsets, nseg, oseg, ocr, ohist,
-                                                                                ohist + kOrderBuckets, order);
-        }
+        launch_order(CapRecs{crec, cursor, cap, (long long)n});
         PYL_HIP(hipGetLastError());
         PYL_TRY(stage_end(c, PYL_STAGE_MA_SCAN));
     }
@@ -3796,13 +3898,8 @@ int run_tiled(Ctx *c, const float *pos, const RSD &rsd, long long n, const long 
     if (!capm) {
         PYL_TRY(stage_begin(c, PYL_STAGE_MA_SCAN));
         PYL_TRY(make_report());
-        launch_scan(c, counts, ocounts, nt, nscan_blocks, bsums, offsets, rep);
-        if (ordered) {
-            const CapRecs ocr{nullptr, nullptr, 0, -1};
-            order_hist_kernel<<<order_wgs(nseg), kOrderBlock, 0, c->stream>>>(offsets, nseg, oseg, ocr, ohist);
-            order_place_kernel<<<order_wgs(nseg), kOrderBlock, 0, c->stream>>>(offsets, nseg, oseg, ocr, ohist,
-                                                                                ohist + kOrderBuckets, order);
-        }
+        launch_scan(c, counts, ocounts, nt, nscan_blocks, bsums, offsets, rep, plan_count);
+        launch_order(CapRecs{nullptr, nullptr, 0, -1});
         PYL_HIP(hipGetLastError());
         PYL_TRY(stage_end(c, PYL_STAGE_MA_SCAN));
     }
@@ -3871,9 +3968,9 @@ int run_tiled(Ctx *c, const float *pos, const RSD &rsd, long long n, const long 
                             : (unit ? column_deposit_kernel<MAS, false, false, false>
                                     : (W ? column_deposit_kernel<MAS, true, true, false>
                                          : column_deposit_kernel<MAS, true, false, false>));
-            kcol<<<(unsigned)nseg, kDepBlock, 0, c->stream>>>(records, rcap, offsets, g, weight_factor,
-                                                              W ? wmax : nullptr, grid, partials, om,
-                                                              ordered ? order : nullptr, cs, cr);
+            kcol<<<(unsigned)(nseg + more), kDepBlock, 0, c->stream>>>(records, rcap, offsets, g, weight_factor,
+                                                                   W ? wmax : nullptr, grid, partials, om, order, cs,
+                                                                   cr);
             PYL_HIP(hipGetLastError());
             PYL_TRY(stage_end(c, PYL_STAGE_MA_DEPOSIT));
             PYL_TRY(stage_begin(c, PYL_STAGE_MA_FINAL));
