@@ -399,6 +399,12 @@ __host__ __device__ __forceinline__ long long win_key(int s, const Win &w, const
 // atomics than the second workgroup per CU gains (2 M on 128^3, whole call: 106 us, with
 // 8192 100).
 constexpr long long kChunkPerTile = 16;
+// And no more chunks than this for being small: every chunk adds to the counters of every
+// tile, one after the other.  4 M particles, CIC, whole call, with chunks of 8192, down to
+// 1024 without this line, and with it (256, 512): 64^3 124, 187, 116 us (117, 117), a 256^2
+// map 120, 184, 103 us (109, 107); 64 x 64 k on 64^3 149, 225, 148 us; 400 k on 64^3 77, 64,
+// 59 us (60, 65).
+constexpr long long kChunkSmall = 128;
 
 // Particles per thread and loop trip: the loads of kUnroll particles are issued
 // (unconditionally, at clamped indices) before any of them is used, so their
@@ -3542,9 +3548,11 @@ int run_tiled(Ctx *c, const float *pos, const RSD &rsd, long long n, const long 
     const bool staged = !capm && !two && !wide && axes == 3 && g.wmode == kWinDirect && g.ntiles <= kStageSlots &&
                         n >= kStageMin;
     // A few small tiles take small chunks down to kChunkPerTile particles per tile: more
-    // workgroups for a call that would not fill the chip.  (Fixed scratch keeps to 8192.)
-    const long long floor = c->arena ? 8192LL
-                                     : std::max(1024LL, std::min(8192LL, kChunkPerTile * g.ntiles));
+    // workgroups, up to kChunkSmall, for a call that would not fill the chip.  (Fixed scratch
+    // keeps to 8192.)
+    const long long floor = c->arena
+        ? 8192LL
+        : std::max(1024LL, std::min(8192LL, std::max(n / kChunkSmall, kChunkPerTile * g.ntiles)));
     const long long target = wide ? std::max(2 * g.ntiles, std::min(16 * g.ntiles, (n + 2047) / 2048))
                                   : std::max(floor, std::min(65536LL, staged ? (n + 2047) / 2048 : (n + 4095) / 4096));
     long long nchunk_ll = 0;
