@@ -517,6 +517,102 @@ tile_count_kernel(const float *__restrict__ pos, RSD rsd, float inv, TileGeom g,
     }
 }
 
+// Records of the capacity sort (cap_scatter_kernel): tile `key` has min(count[key],
+// cap) records at rec + key*cap; rec == nullptr: none (the sorted records alone).
+// nrec >= 0: the realisation's record total (otherwise taken from the offsets).
+struct CapRecs {
+    const float *rec;
+    const unsigned *count;
+    unsigned cap;
+    long long nrec;
+};
+
+__device__ __forceinline__ unsigned long long cap_count(const CapRecs &cr, long long key) {
+    return cr.rec ? (unsigned long long)min(cr.count[key], cr.cap) : 0ull;
+}
+
+// ---- units of the deposit ----
+// What the deposit's workgroups take: segments of len (at most 16) consecutive keys of
+// columns of per keys, segs segments per column, the last one with what is left (one key
+// each: {1, 1, 1, 1}).  A segment is cut before every key at which the records in front of it, counted from
+// the segment's first key, pass a multiple of 2^shift: a unit holds less than 2^shift records
+// besides those of its last key, and n records make at most n >> shift more units than there
+// are segments.  starts[segment] (if wanted): bit j set where key j starts a unit.
+struct OrderSeg {
+    int len, per, segs;
+    int slots;                 // key slots per segment: the power of two that holds len
+    int shift;
+    unsigned nseg;
+    unsigned *starts;
+};
+
+// A listed unit: its first key (below 2^24) and number of keys (those past the column's end
+// are not there).
+__host__ __device__ __forceinline__ unsigned make_unit(unsigned key, unsigned len) { return key | (len - 1) << 28; }
+__host__ __device__ __forceinline__ unsigned unit_key(unsigned unit) { return unit & 0xfffffffu; }
+__host__ __device__ __forceinline__ int unit_len(unsigned unit) { return (int)(unit >> 28) + 1; }
+
+// Keys of the unit that starts at key j of a segment of len keys.
+__host__ __device__ __forceinline__ int unit_keys(unsigned starts, int j, int len) {
+    const unsigned next = starts >> j >> 1;
+    return next ? __builtin_ctz(next) + 1 : len - j;
+}
+
+// Key slot i (slot j of segment q is i = q * slots + j: a segment's keys are read by
+// neighbouring lanes): its unit and the unit's records; false: no unit starts there.  Called
+// by whole wavefronts, for consecutive slots from a multiple of 64 on.
+__device__ __forceinline__ bool order_unit(const unsigned long long *__restrict__ offsets, unsigned i,
+                                           const OrderSeg &os, const CapRecs &cr, unsigned &unit,
+                                           unsigned long long &n) {
+    const unsigned q = i / (unsigned)os.slots, j = i - q * os.slots;
+    const unsigned c = q / (unsigned)os.segs, z = (q - c * os.segs) * os.len + j;
+    const unsigned k = c * os.per + z;
+    const bool in = q < os.nseg && j < (unsigned)os.len && z < (unsigned)os.per;
+    const unsigned long long own = in ? offsets[k + 1] - offsets[k] + cap_count(cr, k) : 0ull;
+    unsigned long long upto = own;                     // records of keys 0..j of the segment
+    for (int o = 1; o < os.slots; o <<= 1) {
+        const unsigned long long v = __shfl_up(upto, o);
+        if ((int)j >= o) upto += v;
+    }
+    const unsigned piece = (unsigned)((upto - own) >> os.shift);
+    const unsigned below = (unsigned)__shfl_up((int)piece, 1);
+    const bool start = in && (j == 0 || piece != below);
+    const int first = (int)(threadIdx.x & 63) - (int)j;            // the segment's first lane
+    const unsigned starts = (unsigned)(__ballot(start) >> first) & ((1u << os.slots) - 1u);
+    if (os.starts && in && j == 0) os.starts[q] = starts;
+    const int len = in ? unit_keys(starts, (int)j, os.len) : 1;
+    n = __shfl(upto, first + (int)j + len - 1) - (upto - own);
+    unit = make_unit(k, (unsigned)len);
+    return start;
+}
+
+// The units that do not start a segment, in any order (count: zeroed before): what the column
+// deposit needs to know where its units are not ordered by records.  Taken by the scatter
+// kernel's threads on the way, or a launch of its own (nthreads in whole wavefronts); nseg 0:
+// nothing to do.  Beside 20 us for the order's two launches (2 M particles, CIC on 512^3, a
+// call of 0.70 ms) and 5 for one.
+struct UnitPlan {
+    OrderSeg os;
+    unsigned *list, *count;
+};
+
+__device__ __forceinline__ void plan_units(const unsigned long long *__restrict__ offsets, const UnitPlan &p,
+                                           const CapRecs &cr, unsigned thread, unsigned nthreads) {
+    const unsigned n = p.os.nseg * (unsigned)p.os.slots;
+    for (unsigned i = thread; (i & ~63u) < n; i += nthreads) {
+        unsigned unit;
+        unsigned long long records;
+        const bool is = order_unit(offsets, i, p.os, cr, unit, records);
+        if (is && i % (unsigned)p.os.slots != 0) p.list[atomicAdd(p.count, 1u)] = unit;
+    }
+}
+
+constexpr int kPlanBlock = 256;
+__global__ void __launch_bounds__(kPlanBlock)
+plan_units_kernel(const unsigned long long *__restrict__ offsets, UnitPlan p, CapRecs cr) {
+    plan_units(offsets, p, cr, blockIdx.x * kPlanBlock + threadIdx.x, gridDim.x * kPlanBlock);
+}
+
 // One record (dist_x, dist_y, dist_z, w) per particle at offsets[key] + slot:
 // window keys take slot = chunk base + LDS cursor, overflow keys slot =
 // counts[key] + global cursor.  Weighted input also records max|W| per
@@ -528,8 +624,11 @@ tile_scatter_kernel(const float *__restrict__ pos, RSD rsd, const float *__restr
                     const unsigned *__restrict__ dump, const unsigned long long *__restrict__ offsets,
                     const unsigned *__restrict__ counts, unsigned *__restrict__ ocursors,
                     unsigned *__restrict__ wmax_bits, float *__restrict__ records,
-                    unsigned long long rcap, int split) {
+                    unsigned long long rcap, int split, UnitPlan plan) {
     __shared__ unsigned cur[WS];
+    if (plan.os.nseg)
+        plan_units(offsets, plan, CapRecs{nullptr, nullptr, 0, -1}, blockIdx.x * kSortBlock + threadIdx.x,
+                   gridDim.x * kSortBlock);
     const Chunk ch = chunks[blockIdx.x];
     if (ch.c1 <= ch.c0) return;                // empty chunk (uniform over the workgroup)
     if (split && scattered(ch)) return;        // left to staged_scatter_kernel
@@ -1480,20 +1579,6 @@ staged_cap_scatter_kernel(const float *__restrict__ bxyz, const float *__restric
 }
 
 // ---- deposit -----------------------------------------------------------------
-// Records of the capacity sort (cap_scatter_kernel): tile `key` has min(count[key],
-// cap) records at rec + key*cap; rec == nullptr: none (the sorted records alone).
-// nrec >= 0: the realisation's record total (otherwise taken from the offsets).
-struct CapRecs {
-    const float *rec;
-    const unsigned *count;
-    unsigned cap;
-    long long nrec;
-};
-
-__device__ __forceinline__ unsigned long long cap_count(const CapRecs &cr, long long key) {
-    return cr.rec ? (unsigned long long)min(cr.count[key], cr.cap) : 0ull;
-}
-
 // Output transform of a final node value v: overwrite ? v/scale - shift : grid + v.
 struct OutMode {
     int overwrite;
@@ -2382,58 +2467,6 @@ __host__ __device__ __forceinline__ int count_bucket(unsigned long long n) {
     return min(kOrderBuckets - 1, 1 + 16 * lg + q);
 }
 
-// What the deposit's workgroups take (units): segments of up to len (a power of two, at most
-// 16) consecutive keys of columns of per keys, segs segments per column (one key each: {1, 1,
-// 1}).  A segment is cut before every key at which the records in front of it, counted from
-// the segment's first key, pass a multiple of 2^shift: a unit holds less than 2^shift records
-// besides those of its last key, and n records make at most n >> shift more units than there
-// are segments.  starts[segment] (if wanted): bit j set where key j starts a unit.
-struct OrderSeg {
-    int len, per, segs, shift;
-    unsigned nseg;
-    unsigned *starts;
-};
-
-// A listed unit: its first key (below 2^24) and number of keys (those past the column's end
-// are not there).
-__host__ __device__ __forceinline__ unsigned make_unit(unsigned key, unsigned len) { return key | (len - 1) << 28; }
-__host__ __device__ __forceinline__ unsigned unit_key(unsigned unit) { return unit & 0xfffffffu; }
-__host__ __device__ __forceinline__ int unit_len(unsigned unit) { return (int)(unit >> 28) + 1; }
-
-// Keys of the unit that starts at key j of a segment of len keys.
-__host__ __device__ __forceinline__ int unit_keys(unsigned starts, int j, int len) {
-    const unsigned next = starts >> j >> 1;
-    return next ? __builtin_ctz(next) + 1 : len - j;
-}
-
-// Key slot i (slot j of segment q is i = q * len + j: a segment's keys are read by
-// neighbouring lanes): its unit and the unit's records; false: no unit starts there.  Called
-// by whole wavefronts, for consecutive slots from a multiple of 64 on.
-__device__ __forceinline__ bool order_unit(const unsigned long long *__restrict__ offsets, unsigned i,
-                                           const OrderSeg &os, const CapRecs &cr, unsigned &unit,
-                                           unsigned long long &n) {
-    const unsigned q = i / (unsigned)os.len, j = i - q * os.len;
-    const unsigned c = q / (unsigned)os.segs, z = (q - c * os.segs) * os.len + j;
-    const unsigned k = c * os.per + z;
-    const bool in = q < os.nseg && z < (unsigned)os.per;
-    const unsigned long long own = in ? offsets[k + 1] - offsets[k] + cap_count(cr, k) : 0ull;
-    unsigned long long upto = own;                     // records of keys 0..j of the segment
-    for (int o = 1; o < os.len; o <<= 1) {
-        const unsigned long long v = __shfl_up(upto, o);
-        if ((int)j >= o) upto += v;
-    }
-    const unsigned piece = (unsigned)((upto - own) >> os.shift);
-    const unsigned below = (unsigned)__shfl_up((int)piece, 1);
-    const bool start = in && (j == 0 || piece != below);
-    const int first = (int)(threadIdx.x & 63) - (int)j;            // the segment's first lane
-    const unsigned starts = (unsigned)(__ballot(start) >> first) & ((1u << os.len) - 1u);
-    if (os.starts && in && j == 0) os.starts[q] = starts;
-    const int len = unit_keys(starts, (int)j, os.len);
-    n = __shfl(upto, first + (int)j + len - 1) - (upto - own);
-    unit = make_unit(k, (unsigned)len);
-    return start;
-}
-
 // The order is built in two launches of order_wgs(nt) workgroups, each thread
 // taking up to kOrderPer of the nt key slots (k = its global index + j * threads): bucket
 // sizes (order_hist_kernel), then the units placed at their bucket's start plus a run
@@ -2460,7 +2493,7 @@ order_hist_kernel(const unsigned long long *__restrict__ offsets, OrderSeg os, C
         unsigned unit;
         unsigned long long n;
         bk[j] = -1;
-        if ((k0 & ~63u) + j * step >= os.nseg * os.len) continue;     // (whole wavefronts)
+        if ((k0 & ~63u) + j * step >= os.nseg * os.slots) continue;     // (whole wavefronts)
         if (order_unit(offsets, k0 + j * step, os, cr, unit, n)) bk[j] = count_bucket(n);
     }
 #pragma unroll
@@ -2503,7 +2536,7 @@ order_place_kernel(const unsigned long long *__restrict__ offsets, OrderSeg os, 
     for (int j = 0; j < kOrderPer; ++j) {
         unsigned long long n;
         bk[j] = -1;
-        if ((k0 & ~63u) + j * step >= os.nseg * os.len) continue;     // (whole wavefronts)
+        if ((k0 & ~63u) + j * step >= os.nseg * os.slots) continue;     // (whole wavefronts)
         if (order_unit(offsets, k0 + j * step, os, cr, unit[j], n)) bk[j] = count_bucket(n);
     }
 #pragma unroll
@@ -2517,20 +2550,6 @@ order_place_kernel(const unsigned long long *__restrict__ offsets, OrderSeg os, 
 #pragma unroll
     for (int j = 0; j < kOrderPer; ++j)
         if (bk[j] >= 0) order[atomicAdd(&lrun[bk[j]], 1u)] = unit[j];
-}
-
-// Without the order: the units that do not start a segment, in any order (count: zeroed
-// before).  One launch of 3 us; the order's two would take 20 us of a 0.70 ms call (2 M, CIC
-// on 512^3).
-constexpr int kPlanBlock = 256;
-__global__ void __launch_bounds__(kPlanBlock)
-segment_plan_kernel(const unsigned long long *__restrict__ offsets, OrderSeg os, CapRecs cr,
-                    unsigned *__restrict__ list, unsigned *__restrict__ count) {
-    const unsigned i = blockIdx.x * kPlanBlock + threadIdx.x;
-    unsigned unit;
-    unsigned long long n;
-    const bool is = order_unit(offsets, i, os, cr, unit, n);
-    if (is && i % (unsigned)os.len != 0) list[atomicAdd(count, 1u)] = unit;
 }
 
 // Images along one axis of a tile t: the tiles whose boxes cover its nodes and
@@ -3593,9 +3612,17 @@ int run_tiled(Ctx *c, const float *pos, const RSD &rsd, long long n, const long 
     ColSeg cs{1, g.nt, (dims + g.nt - 1) / g.nt, nullptr, nullptr, 0};
     if (column)
         while (cs.len < kColMaxLen && nt >= 2 * cs.len * kColMinSegs) cs.len *= 2;
-    if (column) cs.nz = (g.nt + cs.len - 1) / cs.len;
+    int slots = cs.len;                          // key slots of a segment (OrderSeg)
+    if (column) {
+        // the same number of segments of more equal lengths (24 grids of 160^3, columns of ten
+        // tiles, 2.4 M particles, CIC: segments of 8 and 2 0.51 ms, of 5 and 5 0.39; one of
+        // 448^3, 2.4 M, TSC: of 8, 8, 8 and 4 0.77, of 7 0.69)
+        cs.nz = (g.nt + cs.len - 1) / cs.len;
+        cs.len = (g.nt + cs.nz - 1) / cs.nz;
+        while (slots / 2 >= cs.len) slots /= 2;
+    }
     const long long nseg = column ? (long long)nreal * g.nt * g.nt * cs.nz : nt;
-    const long long nslots = nseg * cs.len;      // key slots of the order (order_unit)
+    const long long nslots = nseg * slots;
     const bool ordered = c->tune_order >= 0
         ? (nsplit == 1 && c->tune_order == 1)
         : (nsplit == 1 && nseg >= kOrderMinKeys && n >= kOrderMinRecords * nt);
@@ -3665,18 +3692,22 @@ int run_tiled(Ctx *c, const float *pos, const RSD &rsd, long long n, const long 
     unsigned *plan_count = ordered ? nullptr : nunits;
     cs.nunits = nunits;
     if (cut) cs.starts = ocounts;
-    const OrderSeg oseg = column ? OrderSeg{cs.len, g.nt, cs.nz, cut ? shift : 63, (unsigned)nseg,
+    const OrderSeg oseg = column ? OrderSeg{cs.len, g.nt, cs.nz, slots, cut ? shift : 63, (unsigned)nseg,
                                             cut ? ocounts : nullptr}
-                                 : OrderSeg{1, 1, 1, 63, (unsigned)nt, nullptr};
+                                 : OrderSeg{1, 1, 1, 1, 63, (unsigned)nt, nullptr};
+    // (the one-pass tile scatter lists the units itself)
+    const UnitPlan no_plan{OrderSeg{1, 1, 1, 1, 63, 0, nullptr}, nullptr, nullptr};
+    const UnitPlan plan = cut && !ordered ? UnitPlan{oseg, order, nunits} : no_plan;
+    const bool scatter_plans = !capm && !two && nsort > 0;
     const auto launch_order = [&](const CapRecs &ocr) {
         if (ordered) {
             const int wgs = order_wgs(nslots);
             order_hist_kernel<<<wgs, kOrderBlock, 0, c->stream>>>(offsets, oseg, ocr, ohist);
             order_place_kernel<<<wgs, kOrderBlock, 0, c->stream>>>(offsets, oseg, ocr, ohist, ohist + kOrderBuckets,
                                                                    order, nunits);
-        } else if (cut) {
-            segment_plan_kernel<<<(unsigned)((nslots + kPlanBlock - 1) / kPlanBlock), kPlanBlock, 0, c->stream>>>(
-                offsets, oseg, ocr, order, nunits);
+        } else if (cut && !scatter_plans) {
+            plan_units_kernel<<<(unsigned)((nslots + kPlanBlock - 1) / kPlanBlock), kPlanBlock, 0, c->stream>>>(
+                offsets, plan, ocr);
         }
     };
     unsigned long long *capw = (unsigned long long *)(counts + capw_at);
@@ -3870,7 +3901,7 @@ int run_tiled(Ctx *c, const float *pos, const RSD &rsd, long long n, const long 
                  : (pow2 ? tile_scatter_kernel<MAS, 3, true, false, kWin>
                          : tile_scatter_kernel<MAS, 3, false, false, kWin>));
         ks<<<kSpillChunks, kSortBlock, 0, c->stream>>>(pxyz, off, pw, 1.0f, gs, dchunksS, dump, offsets, counts,
-                                                       ocursors, wmax, records, (unsigned long long)n, 0);
+                                                       ocursors, wmax, records, (unsigned long long)n, 0, no_plan);
         auto kss2 = W ? (pow2 ? spill_scatter_kernel<MAS, true, true> : spill_scatter_kernel<MAS, false, true>)
                       : (pow2 ? spill_scatter_kernel<MAS, true, false> : spill_scatter_kernel<MAS, false, false>);
         PYL_TRY(make_report());
@@ -3948,7 +3979,7 @@ int run_tiled(Ctx *c, const float *pos, const RSD &rsd, long long n, const long 
                                : (pow2 ? tile_scatter_kernel<MAS, 2, true, false, kWin>
                                        : tile_scatter_kernel<MAS, 2, false, false, kWin>));
         ks<<<nsort, kSortBlock, 0, c->stream>>>(spos, srsd, sW, sinv, g, schunks, dump, offsets, counts,
-                                                ocursors, wmax, records, rcap, staged);
+                                                ocursors, wmax, records, rcap, staged, plan);
         if (staged) {                          // the chunks it left
             auto kss = W ? (pow2 ? staged_scatter_kernel<MAS, true, true, 2, kStageSlots, kStage3>
                                  : staged_scatter_kernel<MAS, false, true, 2, kStageSlots, kStage3>)

@@ -49,21 +49,23 @@ def test_beam_exact(dims, nbeam, nbg, mas):
     assert torch.equal(over, ref)
 
 
+# segments of 2 tiles (64^3: 4 tiles a column), of 5 and 5 (160^3), of 4 and 3 uneven ones (100^3)
+@pytest.mark.parametrize('dims,R', [(64, 130), (160, 17), (100, 25)])
 @pytest.mark.parametrize('mas', ['CIC', 'TSC', 'PCS'])
 @pytest.mark.parametrize('weighted', [False, True])
-def test_cut_segments_do_not_change_bits(mas, weighted):
+def test_cut_segments_do_not_change_bits(dims, R, mas, weighted):
     import torch
     from pylians3_amd import MAS_library as MASL, batch
     g = torch.Generator(device='cuda').manual_seed(9)
-    dims, box, R = 64, 100.0, 130                     # 130 * 64 tiles: segments of two
+    box = 100.0
     counts = [int(x) for x in np.random.default_rng(2).integers(0, 3000, R)]
-    counts[0], counts[5], counts[77], counts[129] = 60000, 0, 90000, 30000
+    counts[0], counts[5], counts[R // 2], counts[R - 1] = 60000, 0, 90000, 30000
     pos = []
     for r, n in enumerate(counts):
         p = torch.rand((n, 3), generator=g, device='cuda') * box
-        if n >= 30000:                                # one column of tiles, or half of it
+        if n >= 30000:                                # a column of tiles or two, or half of it
             p[:, :2] = p[:, :2] * 0.2 + 26.0
-            if r == 129:
+            if r == R - 1:
                 p[:, 2] = p[:, 2] * 0.4 + 58.0
         pos.append(p)
     offs = np.concatenate([[0], np.cumsum(counts)]).astype(np.int64)
@@ -72,7 +74,7 @@ def test_cut_segments_do_not_change_bits(mas, weighted):
     for accumulate in (False, True):
         grids = torch.full((R,) + (dims,) * 3, 3.0, device='cuda')
         batch.MA_batch(allp, offs, grids, box, mas, W=W, accumulate=accumulate)
-        for r in (0, 1, 5, 6, 77, 78, 128, 129):
+        for r in (0, 1, 5, 6, R // 2, R // 2 + 1, R - 2, R - 1):
             a, b = int(offs[r]), int(offs[r + 1])
             one = torch.full((dims,) * 3, 3.0 if accumulate else 0.0, device='cuda')
             MASL.MA(allp[a:b].contiguous(), one, box, mas, W=None if W is None else W[a:b].contiguous())
