@@ -2440,6 +2440,12 @@ constexpr long long kColMinSegs = 2048;
 constexpr int kColMinCut = 13;
 constexpr long long kColCuts = 512;
 constexpr long long kColPcsDense = 2048;         // mean records per tile
+// TSC on even grids: tiles per segment from which on the column form is taken, for grids
+// written and for grids added to.  Tile form and column form, 1000 particles per tile, added:
+// 256^3 (2 tiles) 183 and 184 us, 320^3 (2) 346 and 370, 384^3 (4) 556 and 579, 300 grids of
+// 64^3 (4) 763 and 780, 448^3 (7) 817 and 817, 480^3 (8) 986 and 966; written: 320^3 333 and
+// 344, 384^3 540 and 525, 300 of 64^3 646 and 626, 448^3 805 and 728, 480^3 970 and 864.
+constexpr int kColTscOver = 4, kColTscAdd = 5;
 constexpr long long kOrderMinKeys = 2048;
 constexpr long long kOrderMinRecords = 512;      // mean records per key
 // Split deposit: below kSplitMaxKeys tiles, a tile holding more than
@@ -3607,8 +3613,8 @@ int run_tiled(Ctx *c, const float *pos, const RSD &rsd, long long n, const long 
     // 1024^3: tile form 14.4 + 2.9 ms, column form 15.9 + 1.7; 2 M on 512^3: 0.78 + 0.40
     // and 0.73 + 0.23).
     const bool uni = g.nt >= 2 && dims % (axes == 3 ? kT3 : kT2) == 0;
-    const bool column = axes == 3 && g.nt >= 2 && MAS > 1 && nsplit == 1 &&
-                        !(MAS == PYL_PCS && uni && n >= kColPcsDense * nt);
+    bool column = axes == 3 && g.nt >= 2 && MAS > 1 && nsplit == 1 &&
+                  !(MAS == PYL_PCS && uni && n >= kColPcsDense * nt);
     ColSeg cs{1, g.nt, (dims + g.nt - 1) / g.nt, nullptr, nullptr, 0};
     if (column)
         while (cs.len < kColMaxLen && nt >= 2 * cs.len * kColMinSegs) cs.len *= 2;
@@ -3620,6 +3626,12 @@ int run_tiled(Ctx *c, const float *pos, const RSD &rsd, long long n, const long 
         cs.nz = (g.nt + cs.len - 1) / cs.len;
         cs.len = (g.nt + cs.nz - 1) / cs.nz;
         while (slots / 2 >= cs.len) slots /= 2;
+        // TSC in even tiles, whose deposit is no faster in columns: where the segments are
+        // long enough for what the finalize gains
+        if (MAS == PYL_TSC && uni && cs.len < (om.overwrite ? kColTscOver : kColTscAdd)) {
+            column = false;
+            cs.len = slots = 1;
+        }
     }
     const long long nseg = column ? (long long)nreal * g.nt * g.nt * cs.nz : nt;
     const long long nslots = nseg * slots;
