@@ -1251,10 +1251,16 @@ constexpr int kStage2 = 8192;      // and pass 2 (tiles)
 // displaced lattice, which leave in runs as they come, 153 us one by one and 172 staged.
 constexpr int kStage3 = 8192;
 constexpr int kStageSlots = 512;
-// From kStageMin particles on, where the second launch (3 to 6 us) is within 2 % of a call
-// on coherent particles (8.4 M on 128^3: lattice 142 -> 146 us, random order 177 -> 164; 33.5 M
-// there: 474 -> 465 and 662 -> 558), with chunks up to twice as long, which make up for it.
+// From kStageMin particles on, where the second launch is within 2 to 4 % of a call on coherent
+// particles (8.4 M on 128^3: lattice 142 -> 146 us, random order 177 -> 164; 33.5 M there,
+// with longer chunks: 474 -> 465 and 662 -> 558).  (One workgroup per chunk: 512 with several
+// each take as long, and a list of the scattered chunks costs their appends 20 us.)
+// Grids of kStageLong tiles and more with kStageLongMin particles a realisation and more take
+// chunks up to twice as long besides (33.5 M on 128^3: lattice 472 -> 454 us, random order 561
+// -> 553); with fewer tiles or short realisations they lose more (67 M in random order on
+// 64^3: 956 -> 1035 us, 2000 grids of 10 k particles: 439 -> 548).
 constexpr long long kStageMin = 10ll << 20;
+constexpr long long kStageLong = 256, kStageLongMin = 1ll << 20;
 
 // Exclusive scan of cnt[0..ns) into ofs[0..ns) over the workgroup (kSortBlock
 // threads, ns <= NS); returns the total.  wsum: kSortBlock / 64 + 1 words of LDS.
@@ -3572,6 +3578,7 @@ int run_tiled(Ctx *c, const float *pos, const RSD &rsd, long long n, const long 
     // Chunks of consecutive particles, never straddling two realisations.
     const bool staged = !capm && !two && !wide && axes == 3 && g.wmode == kWinDirect && g.ntiles <= kStageSlots &&
                         n >= kStageMin;
+    const bool longer = staged && g.ntiles >= kStageLong && n >= kStageLongMin * nreal;
     // A few small tiles take small chunks down to kChunkPerTile particles per tile: more
     // workgroups, up to kChunkSmall, for a call that would not fill the chip.  (Fixed scratch
     // keeps to 8192.)
@@ -3579,7 +3586,7 @@ int run_tiled(Ctx *c, const float *pos, const RSD &rsd, long long n, const long 
         ? 8192LL
         : std::max(1024LL, std::min(8192LL, std::max(n / kChunkSmall, kChunkPerTile * g.ntiles)));
     const long long target = wide ? std::max(2 * g.ntiles, std::min(16 * g.ntiles, (n + 2047) / 2048))
-                                  : std::max(floor, std::min(65536LL, staged ? (n + 2047) / 2048 : (n + 4095) / 4096));
+                                  : std::max(floor, std::min(65536LL, longer ? (n + 2047) / 2048 : (n + 4095) / 4096));
     long long nchunk_ll = 0;
     if (devt) nchunk_ll = (long long)nreal * c->chunks_per_real;
     else
