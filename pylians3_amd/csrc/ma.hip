@@ -626,85 +626,86 @@ tile_scatter_kernel(const float *__restrict__ pos, RSD rsd, const float *__restr
                     unsigned *__restrict__ wmax_bits, float *__restrict__ records,
                     unsigned long long rcap, int split, UnitPlan plan) {
     __shared__ unsigned cur[WS];
+    const Chunk ch = chunks[blockIdx.x];
+    // not for an empty chunk, nor one left to staged_scatter_kernel (uniform over the workgroup)
+    if (ch.c1 > ch.c0 && !(split && scattered(ch))) {
+        const long long rbase = (long long)ch.r * g.ntiles;
+        // the count pass's window of this chunk
+        Win win{g.wmode, 0, 0, 0, (int)g.ntiles};
+        if (g.wmode == kWinBox || g.wmode == kWinBlock) {
+            win.a = ch.wbase / g.nt;
+            win.b = ch.wbase - win.a * g.nt;
+            win.c = ch.wz;
+            win.slots = g.wmode == kWinBox ? kBoxW * kBoxW * g.ntz : kBktSlots;
+        } else if (g.wmode == kWinLinear) {
+            win.a = ch.wbase;
+            win.slots = kWin;
+        }
+        const unsigned *dmp = dump + (long long)blockIdx.x * dump_stride<WS>(g);
+        // only slots in [smin, smax] were counted; no other slot is looked up
+        for (int s = ch.smin + threadIdx.x; s <= ch.smax; s += blockDim.x) cur[s] = dmp[s];
+        __syncthreads();
+        unsigned m = 0;
+        const long long step = (long long)blockDim.x * kUnrollS;
+        const long long last = ch.c1 - 1;
+        for (long long base = ch.c0 + threadIdx.x; base < ch.c1; base += step) {
+            float3 d[kUnrollS];
+            float w[kUnrollS];
+            unsigned key[kUnrollS];
+            unsigned long long slot[kUnrollS];
+#pragma unroll
+            for (int u = 0; u < kUnrollS; ++u) {
+                const long long i = min(base + (long long)u * blockDim.x, last);
+                d[u] = load_dist<AXES>(pos, rsd, i, inv);
+                w[u] = WT ? W[i] : 1.0f;
+            }
+#pragma unroll
+            for (int u = 0; u < kUnrollS; ++u) {
+                const int3 t = dist_tiles<MAS, AXES, POW2>(d[u], g);
+                key[u] = tiles_key(t, g, rbase);
+                slot[u] = 0;
+                if (base + (long long)u * blockDim.x < ch.c1) {
+                    const unsigned s = win_slot(t, key[u], win, g, rbase);
+                    if (s < (unsigned)win.slots) slot[u] = atomicAdd(&cur[s], 1u);
+                    else slot[u] = (unsigned long long)counts[key[u]] + atomicAdd(&ocursors[key[u]], 1u);
+                }
+            }
+#pragma unroll
+            for (int u = 0; u < kUnrollS; ++u) {
+                if (base + (long long)u * blockDim.x < ch.c1) {
+                    const unsigned long long at = offsets[key[u]] + slot[u];
+                    if (at >= rcap) continue;               // only after a miscount (reported)
+                    if (WT) {
+                        reinterpret_cast<float4 *>(records)[at] = make_float4(d[u].x, d[u].y, d[u].z, w[u]);
+                    } else {
+                        float *o = records + 3 * at;
+                        o[0] = d[u].x;
+                        o[1] = d[u].y;
+                        o[2] = d[u].z;
+                    }
+                    if (WT) {
+                        const unsigned b = __float_as_uint(fabsf(w[u]));
+                        if (b < 0x7f800000u) m = max(m, b);
+                    }
+                }
+            }
+        }
+        if (WT) {
+            // block max through the (no longer needed) cursor table
+            for (int off = 32; off > 0; off >>= 1) m = max(m, (unsigned)__shfl_xor((int)m, off));
+            __syncthreads();
+            if ((threadIdx.x & 63) == 0) cur[threadIdx.x >> 6] = m;
+            __syncthreads();
+            if (threadIdx.x == 0) {
+                unsigned mm = 0;
+                for (int k = 0; k < (int)(blockDim.x >> 6); ++k) mm = max(mm, cur[k]);
+                atomicMax(&wmax_bits[ch.r], mm);
+            }
+        }
+    }
     if (plan.os.nseg)
         plan_units(offsets, plan, CapRecs{nullptr, nullptr, 0, -1}, blockIdx.x * kSortBlock + threadIdx.x,
                    gridDim.x * kSortBlock);
-    const Chunk ch = chunks[blockIdx.x];
-    if (ch.c1 <= ch.c0) return;                // empty chunk (uniform over the workgroup)
-    if (split && scattered(ch)) return;        // left to staged_scatter_kernel
-    const long long rbase = (long long)ch.r * g.ntiles;
-    // the count pass's window of this chunk
-    Win win{g.wmode, 0, 0, 0, (int)g.ntiles};
-    if (g.wmode == kWinBox || g.wmode == kWinBlock) {
-        win.a = ch.wbase / g.nt;
-        win.b = ch.wbase - win.a * g.nt;
-        win.c = ch.wz;
-        win.slots = g.wmode == kWinBox ? kBoxW * kBoxW * g.ntz : kBktSlots;
-    } else if (g.wmode == kWinLinear) {
-        win.a = ch.wbase;
-        win.slots = kWin;
-    }
-    const unsigned *dmp = dump + (long long)blockIdx.x * dump_stride<WS>(g);
-    // only slots in [smin, smax] were counted; no other slot is looked up
-    for (int s = ch.smin + threadIdx.x; s <= ch.smax; s += blockDim.x) cur[s] = dmp[s];
-    __syncthreads();
-    unsigned m = 0;
-    const long long step = (long long)blockDim.x * kUnrollS;
-    const long long last = ch.c1 - 1;
-    for (long long base = ch.c0 + threadIdx.x; base < ch.c1; base += step) {
-        float3 d[kUnrollS];
-        float w[kUnrollS];
-        unsigned key[kUnrollS];
-        unsigned long long slot[kUnrollS];
-#pragma unroll
-        for (int u = 0; u < kUnrollS; ++u) {
-            const long long i = min(base + (long long)u * blockDim.x, last);
-            d[u] = load_dist<AXES>(pos, rsd, i, inv);
-            w[u] = WT ? W[i] : 1.0f;
-        }
-#pragma unroll
-        for (int u = 0; u < kUnrollS; ++u) {
-            const int3 t = dist_tiles<MAS, AXES, POW2>(d[u], g);
-            key[u] = tiles_key(t, g, rbase);
-            slot[u] = 0;
-            if (base + (long long)u * blockDim.x < ch.c1) {
-                const unsigned s = win_slot(t, key[u], win, g, rbase);
-                if (s < (unsigned)win.slots) slot[u] = atomicAdd(&cur[s], 1u);
-                else slot[u] = (unsigned long long)counts[key[u]] + atomicAdd(&ocursors[key[u]], 1u);
-            }
-        }
-#pragma unroll
-        for (int u = 0; u < kUnrollS; ++u) {
-            if (base + (long long)u * blockDim.x < ch.c1) {
-                const unsigned long long at = offsets[key[u]] + slot[u];
-                if (at >= rcap) continue;               // only after a miscount (reported)
-                if (WT) {
-                    reinterpret_cast<float4 *>(records)[at] = make_float4(d[u].x, d[u].y, d[u].z, w[u]);
-                } else {
-                    float *o = records + 3 * at;
-                    o[0] = d[u].x;
-                    o[1] = d[u].y;
-                    o[2] = d[u].z;
-                }
-                if (WT) {
-                    const unsigned b = __float_as_uint(fabsf(w[u]));
-                    if (b < 0x7f800000u) m = max(m, b);
-                }
-            }
-        }
-    }
-    if (WT) {
-        // block max through the (no longer needed) cursor table
-        for (int off = 32; off > 0; off >>= 1) m = max(m, (unsigned)__shfl_xor((int)m, off));
-        __syncthreads();
-        if ((threadIdx.x & 63) == 0) cur[threadIdx.x >> 6] = m;
-        __syncthreads();
-        if (threadIdx.x == 0) {
-            unsigned mm = 0;
-            for (int k = 0; k < (int)(blockDim.x >> 6); ++k) mm = max(mm, cur[k]);
-            atomicMax(&wmax_bits[ch.r], mm);
-        }
-    }
 }
 
 // ---- capacity sort: one read of the particles ----------------------------------
