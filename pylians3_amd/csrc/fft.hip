@@ -294,20 +294,9 @@ absmax_kernel(const float2 *__restrict__ dk, long long nrows, int zlen, long lon
     block_absmax(m, amax, (unsigned)cube * 64u + (blockIdx.x & 63u));
 }
 
-// Real-to-complex FFT of rows of N floats (contiguous), R rows per workgroup:
-// z[j] = x[2j] + i x[2j+1] is transformed with N/2-point Stockham FFTs, then
-// X[k] = E[k] + e^{-2 pi i k/N} O[k] with E[k] = (Z[k] + conj(Z[N/2-k]))/2 and
-// O[k] = -i (Z[k] - conj(Z[N/2-k]))/2, k = 0..N/2 (indices mod N/2).  Output
-// rows of N/2+1 complex.
-//
-// The rows are read where the caller keeps them (RowSrc: one array per field) and the
-// prologue x/scale - shift is applied to them as they are read, so no copy of the
-// field is made before the transform: the pass is HBM-bound, and the copy (512^3:
-// 0.21 ms beside this kernel's 0.25) and, for a batch with scales, the prologue's own
-// pass over it (32 x 2 x 128^3: 0.34 + 0.25 ms) were pure extra traffic.  Pk of a 512^3
-// field on the GPU: 1.41 -> 1.18 ms, the batch of 32: 5.66 -> 5.20 ms.
+// The prologue of the n pairs v of cube (field, real): x/scale - shift in float32.
 __device__ __forceinline__ void row_prologue(const RowSrc &rs, int field, int real, float2 *v, int n) {
-    if (!rs.apply) return;                                // uniform: (x / scale) - shift in float32
+    if (!rs.apply) return;                                // uniform
     const int si = field * rs.sfield + real * rs.sreal;
     const float scale = rs.scales ? rs.scales[si] : rs.scale;
     const float shift = rs.shifts ? rs.shifts[si] : rs.shift;
@@ -326,6 +315,18 @@ __device__ __forceinline__ float2 split_mode(float2 a, float2 b, float2 w) {
     return cadd(e, cmul(w, o));
 }
 
+// Real-to-complex FFT of rows of N floats (contiguous), R rows per workgroup:
+// z[j] = x[2j] + i x[2j+1] is transformed with N/2-point Stockham FFTs, then
+// X[k] = E[k] + e^{-2 pi i k/N} O[k] with E[k] = (Z[k] + conj(Z[N/2-k]))/2 and
+// O[k] = -i (Z[k] - conj(Z[N/2-k]))/2, k = 0..N/2 (indices mod N/2).  Output
+// rows of N/2+1 complex.
+//
+// The rows are read where the caller keeps them (RowSrc: one array per field) and the
+// prologue x/scale - shift is applied to them as they are read, so no copy of the
+// field is made before the transform: the pass is HBM-bound, and the copy (512^3:
+// 0.21 ms beside this kernel's 0.25) and, for a batch with scales, the prologue's own
+// pass over it (32 x 2 x 128^3: 0.34 + 0.25 ms) were pure extra traffic.  Pk of a 512^3
+// field on the GPU: 1.41 -> 1.18 ms, the batch of 32: 5.66 -> 5.20 ms.
 template <int N, int R>
 __global__ void __launch_bounds__(kFftBlock)
 fft_r2c_rows_kernel(RowSrc rs, float2 *__restrict__ out, long long nrows,
@@ -378,7 +379,7 @@ fft_r2c_rows_kernel(RowSrc rs, float2 *__restrict__ out, long long nrows,
 // stride keeps both directions free of bank conflicts.  32 x 2 cubes of 128^3: the three
 // passes 820 us, this one and the x pass 572 (a workgroup of 512: 650); one 64^3 field:
 // 15.9 -> 12.4 us and a launch less (256 threads: 13.5).  A larger plane does not fit
-// in LDS, a smaller one would leave a workgroup little to do.  Launching both passes on
+// in LDS; sides of 16 and 32 were not tried.  Launching both passes on
 // 64 to 160 MB of cubes at a time, so that the second finds the first one's output in
 // the memory-side cache, gained less than the extra launches' tails cost (610 to 670 us).
 template <int N>

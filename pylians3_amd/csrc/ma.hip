@@ -1049,7 +1049,10 @@ scan_blocksums_kernel(unsigned long long *__restrict__ block_sums, int nblocks) 
 // ONE: the sums of the elements before the workgroup's are formed here (up to
 // kScanOne workgroups, which read at most 8 * kScanOne * kScanTile bytes each from
 // cache) instead of by the two kernels above: one launch, whose time is latency (4096
-// keys: 3 launches of 9.3 us and their gaps -> 3.7 us; 16384 keys 10 us).
+// keys: 3 launches of 9.3 us and their gaps -> 3.7 us; 16384 keys 10 us; 32768 keys 17 us
+// against 16.4 and two gaps).  Whole calls of 1 M particles, CIC, in three launches and in
+// one: 400^3 (15625 keys) 409 and 400 us, 512^3 (32768) 661 and 655, 640^3 (64000) 1210
+// both: the limit lies where the gaps are made up for.
 template <bool ONE>
 __global__ void __launch_bounds__(kScanBlock)
 scan_final_kernel(const unsigned *__restrict__ in, const unsigned *__restrict__ in2, long long n,
@@ -2446,7 +2449,11 @@ constexpr int kColMaxLen = 16;
 constexpr long long kColMinSegs = 2048;
 constexpr int kColMinCut = 13;
 constexpr long long kColCuts = 512;
-constexpr long long kColPcsDense = 2048;         // mean records per tile
+// PCS on even grids: mean records per tile from which on the tile form is taken.  Column form
+// and tile form, grids added to: 512^3 1000 per tile 1395 and 1517 us, 2000 1862 and 1872, 4096
+// 2979 and 2905; 256^3 300 per tile 230 and 239, 1000 229 and 220, 2000 314 and 296, 4096 473
+// and 442: the line lies where the larger grid's forms meet.
+constexpr long long kColPcsDense = 2048;
 // TSC on even grids: tiles per segment from which on the column form is taken, for grids
 // written and for grids added to.  Tile form and column form, 1000 particles per tile, added:
 // 256^3 (2 tiles) 183 and 184 us, 320^3 (2) 346 and 370, 384^3 (4) 556 and 579, 300 grids of
