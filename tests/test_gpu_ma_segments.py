@@ -79,3 +79,27 @@ def test_cut_segments_do_not_change_bits(dims, R, mas, weighted):
             one = torch.full((dims,) * 3, 3.0 if accumulate else 0.0, device='cuda')
             MASL.MA(allp[a:b].contiguous(), one, box, mas, W=None if W is None else W[a:b].contiguous())
             assert torch.equal(grids[r], one), (r, accumulate)
+
+
+def test_cut_segments_in_a_graph():
+    """Replays with other particles in the same places: units are found anew by every replay."""
+    import torch
+    from pylians3_amd import batch
+    g = torch.Generator(device='cuda').manual_seed(4)
+    dims, box, R, n = 64, 100.0, 70, 300000            # 4480 tiles: segments of two
+    offs = torch.arange(R + 1, dtype=torch.int64, device='cuda') * (n // R)
+    offs[1:] += n - n // R * R
+    pos = torch.rand((n, 3), generator=g, device='cuda') * box
+    graph = batch.BatchGraph([dict(pos=pos, offs=offs, W=None, mas='CIC')], R, dims, box)
+    for rep in range(3):
+        p = torch.rand((n, 3), generator=g, device='cuda') * box
+        if rep:                                         # beams in all realisations, in the first ones
+            m = n if rep == 1 else n // 4
+            p[:m, :2] = p[:m, :2] * 0.1 + 10.0 * rep
+        pos.copy_(p)
+        torch.cuda.synchronize()
+        graph.run()
+        ref = torch.empty((R,) + (dims,) * 3, device='cuda')
+        batch.MA_batch(p, offs.cpu().numpy(), ref, box, 'CIC', accumulate=False)
+        assert torch.equal(graph.grids[0], ref), rep
+    graph.close()
